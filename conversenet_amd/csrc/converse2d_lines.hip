@@ -1,0 +1,432 @@
+// Row and column passes of the multi-pass routes for any transform length up to 1024, on the in-place
+// prime-factor engine of fft_lines.h.  Same spectra scratch and transfer table as the runtime-plan passes
+// of converse2d_generic.hip (half spectra S[plane][col][row], tables (psf plane, col, row), twiddles
+// exp(-2 pi i m / L)), which keep the longer lengths.
+//
+// Every block transforms 16 lines (row pairs or columns) of any planes: lines are numbered through all
+// planes, so small planes fill their blocks.
+//
+// What bounds them: each pass is one trip of the plane through HBM or the MALL (4.6 to 6 bytes moved per
+// byte of plane and pass), overlapped by the 2 to 16 blocks of a CU with two or three LDS passes.  Measured
+// (one layer, us, runtime-plan passes -> these): 128 planes 333 x 493: 679 -> 210 (rows 214 -> 58, columns
+// 282 -> 90, inverse rows 214 -> 58); 512 planes 136 x 136: 282 -> 90; 256 planes 499 x 509 (primes):
+// 1283 ms -> 1.7 ms; the backward's 1024 x 260 rows of 260, compile-time plan before: 172 -> 127.
+#include <algorithm>
+
+#include "cvn_common.h"
+#include "fft_lines.h"
+
+namespace cvn {
+namespace {
+
+constexpr int kLineThreads = 1024;
+constexpr size_t kLineLds = 160 * 1024;
+
+__device__ __forceinline__ int line_pad_src(int i, int n, int p, int mode) {
+  int j = i - p;
+  if (j >= 0 && j < n) return j;
+  switch (mode) {
+    case CVN_PAD_CIRCULAR: j %= n; return j < 0 ? j + n : j;
+    case CVN_PAD_REPLICATE: return j < 0 ? 0 : n - 1;
+    case CVN_PAD_REFLECT: return j < 0 ? -j : 2 * (n - 1) - j;
+    default: return -1;
+  }
+}
+
+// The dispatcher places block i on XCD i mod 8; items run contiguously per XCD, so that neighbouring
+// batches (which share 128-byte lines of the spectra) and the planes of one psf meet in one L2.
+__device__ __forceinline__ int line_item(int blk, int nblk) {
+  const int x = blk & 7, k = blk >> 3, per = nblk >> 3, rem = nblk & 7;
+  return x * per + min(x, rem) + k;
+}
+
+// ------------------------------------------------------------------------------------------------
+// Forward row pass: real row pairs (2 t, 2 t + 1) as one complex line, half spectra to S[plane][v][row].
+// ------------------------------------------------------------------------------------------------
+struct RowsFwdArgs {
+  const float* x;   // (P, Hin, Win)
+  float2* S;        // (P, NC, h)
+  const float2* tw;
+  int Hin, Win, h, pad, mode, NC, npair, total, nblk;  // total = P npair lines
+  int vec;          // S allows 16-byte stores of a row pair (h even, S 16-byte aligned)
+  LinePlan plan;
+};
+
+__global__ void __launch_bounds__(kLineThreads) k_lines_rows_fwd(RowsFwdArgs) {
+  const CVN_KARG RowsFwdArgs& a = *(const CVN_KARG RowsFwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int NB = kLines, LD = kLineLd;
+  const int tid = threadIdx.x, nth = blockDim.x, L = a.plan.L;
+  float2* buf = (float2*)smem;
+  char* tab = smem + ((size_t)L * LD * sizeof(float2) + 15) / 16 * 16;
+  int64_t* src = (int64_t*)tab;  // 2 NB: element offset of each line's source rows, -1: zeros
+  float2* tw = (float2*)(src + 2 * NB);
+  unsigned short* ipos = (unsigned short*)(tw + a.plan.T);
+  const int g0 = line_item(blockIdx.x, a.nblk) * NB;
+  if (tid < 2 * NB) {
+    const int gp = g0 + (tid >> 1);
+    const int plane = gp / a.npair, r = 2 * (gp - plane * a.npair) + (tid & 1);
+    const int sr = (gp < a.total && r < a.h) ? line_pad_src(r, a.Hin, a.pad, a.mode) : -1;
+    src[tid] = sr >= 0 ? ((int64_t)plane * a.Hin + sr) * a.Win : -1;
+  }
+  __syncthreads();
+  // items (8 lines, sample n), n fastest; the tables are filled while the first loads are on their way
+  const int nitem = L * (NB / 8);
+  for (int i0 = tid; i0 < nitem || i0 == tid; i0 += nth) {
+    const int idx = min(i0, nitem - 1);
+    const int q = mg_div(idx, a.plan.mgL, L), n = idx - q * L, b0 = 8 * q;
+    const int sc = line_pad_src(n, a.Win, a.pad, a.mode);
+    const float* xc = a.x + max(sc, 0);
+    float va[8], vb[8];
+    int64_t oa[8], ob[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      oa[k] = src[2 * (b0 + k)];
+      ob[k] = src[2 * (b0 + k) + 1];
+      va[k] = xc[oa[k] < 0 ? 0 : oa[k]];
+      vb[k] = xc[ob[k] < 0 ? 0 : ob[k]];
+    }
+    if (i0 == tid) line_tables(a.plan, a.tw, ipos, tw, tid, nth);
+    if (i0 < nitem) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        buf[n * LD + b0 + k] =
+            make_float2(sc < 0 || src[2 * (b0 + k)] < 0 ? 0.f : va[k], sc < 0 || src[2 * (b0 + k) + 1] < 0 ? 0.f : vb[k]);
+    }
+  }
+  __syncthreads();
+  line_fft<true>(a.plan, smem, tw, tid, nth);
+  // Ya = (Z[v] + conj Z[-v]) / 2, Yb = (Z[v] - conj Z[-v]) / (2 i)
+  const int b = tid % NB, gp = g0 + b;
+  if (gp >= a.total) return;
+  const int plane = gp / a.npair, r = 2 * (gp - plane * a.npair);
+  float2* out = a.S + (int64_t)plane * a.NC * a.h + r;
+  const bool two = r + 1 < a.h;
+  const int step = nth / NB;
+  for (int v0 = tid / NB; v0 < a.NC; v0 += 4 * step) {
+    float2 z[4], zm[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int v = min(v0 + k * step, a.NC - 1);
+      z[k] = buf[ipos[v] * LD + b];
+      zm[k] = buf[ipos[v ? L - v : 0] * LD + b];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int v = v0 + k * step;
+      if (v >= a.NC) break;
+      const float2 ya = make_float2(0.5f * (z[k].x + zm[k].x), 0.5f * (z[k].y - zm[k].y));
+      const float2 yb = make_float2(0.5f * (z[k].y + zm[k].y), 0.5f * (zm[k].x - z[k].x));
+      float2* o = out + (int64_t)v * a.h;
+      if (a.vec) {
+        *(float4*)o = make_float4(ya.x, ya.y, yb.x, yb.y);
+      } else {
+        o[0] = ya;
+        if (two) o[1] = yb;
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Module column pass: forward LR column transform, times Phi, inverse HR column transform.
+// ------------------------------------------------------------------------------------------------
+struct ColsArgs {
+  const float2* S;    // (P, NC, h)
+  const float2* phi;  // (Cp, NCs, Hs)
+  float2* SH;         // (P, NCs, Hs); S itself at scale 1
+  const float2 *tw_h, *tw_H;
+  int B, C, psf_batch;
+  int w, Hs, NC, NCs, total, nblk;
+  LinePlan ph, pH;    // column lengths h and Hs (pH unused at scale 1)
+};
+
+template <bool ONE>  // ONE: scale 1, in place
+__global__ void __launch_bounds__(kLineThreads) k_lines_cols(ColsArgs) {
+  const CVN_KARG ColsArgs& a = *(const CVN_KARG ColsArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int NB = kLines, LD = kLineLd;
+  const int tid = threadIdx.x, nth = blockDim.x, h = a.ph.L, Hs = ONE ? h : a.Hs;
+  float2* X = (float2*)smem;  // the HR lines
+  char* p = smem + ((size_t)Hs * LD * sizeof(float2) + 15) / 16 * 16;
+  float2* Y = ONE ? X : (float2*)p;  // the LR lines
+  if (!ONE) p += ((size_t)h * LD * sizeof(float2) + 15) / 16 * 16;
+  int64_t* in = (int64_t*)p;  // per line: offset in S (complemented: the conjugate), in Phi, in SH
+  int64_t *fi = in + NB, *oo = fi + NB;
+  float2* twh = (float2*)(oo + NB);
+  float2* twH = ONE ? twh : twh + a.ph.T;
+  unsigned short* ih = (unsigned short*)(twH + (ONE ? a.ph.T : a.pH.T));
+  unsigned short* iH = ONE ? ih : ih + h;
+  const int g0 = line_item(blockIdx.x, a.nblk) * NB;
+  const int nb = min(NB, a.total - g0);
+  if (tid < NB) {
+    // lines channel by channel: the planes that share a psf follow each other
+    const int gc = min(g0 + tid, a.total - 1);
+    const int q = gc / a.NCs, v = gc - q * a.NCs;
+    const int c = q / a.B;
+    const int64_t plane = (int64_t)(q - c * a.B) * a.C + c;
+    const int64_t cp = a.psf_batch == 1 ? c : plane;
+    oo[tid] = (plane * a.NCs + v) * Hs;
+    fi[tid] = (cp * a.NCs + v) * Hs;
+    const int vv = ONE ? v : v % a.w;  // a real row's spectrum is Hermitian in the column
+    in[tid] = vv < a.NC ? (plane * a.NC + vv) * h : ~((plane * a.NC + (a.w - vv)) * h);
+  }
+  __syncthreads();
+  const int nin = h * (NB / 8), nout = Hs * (NB / 8);
+  for (int i0 = tid; i0 < nin || i0 == tid; i0 += nth) {
+    const int idx = min(i0, nin - 1);
+    const int q = mg_div(idx, a.ph.mgL, h), u = idx - q * h, b0 = 8 * q;
+    float2 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t o = in[b0 + k];
+      v[k] = a.S[(o < 0 ? ~o : o) + u];
+      if (!ONE && o < 0) v[k].y = -v[k].y;
+    }
+    if (i0 == tid) {
+      line_tables(a.ph, a.tw_h, ih, twh, tid, nth);
+      if (!ONE) line_tables(a.pH, a.tw_H, iH, twH, tid, nth);
+    }
+    if (i0 < nin) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) Y[u * LD + b0 + k] = v[k];
+    }
+  }
+  __syncthreads();
+  line_fft<true>(a.ph, (char*)Y, twh, tid, nth);
+  for (int idx = tid; idx < nout; idx += nth) {
+    const int q = mg_div(idx, ONE ? a.ph.mgL : a.pH.mgL, Hs), u = idx - q * Hs, b0 = 8 * q;
+    float2 f[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) f[k] = a.phi[fi[b0 + k] + u];
+    const int us = ONE ? u : u - mg_div(u, a.ph.mgL, h) * h;
+    const float2* y = Y + ih[us] * LD + b0;
+    float2* x = X + iH[u] * LD + b0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float2 t = cmul(y[k], f[k]);
+      x[k] = make_float2(t.y, t.x);
+    }
+  }
+  __syncthreads();
+  line_fft<false>(ONE ? a.ph : a.pH, smem, twH, tid, nth);
+  for (int idx = tid; idx < nout; idx += nth) {
+    const int q = mg_div(idx, ONE ? a.ph.mgL : a.pH.mgL, Hs), u = idx - q * Hs, b0 = 8 * q;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (b0 + k < nb) {
+        const float2 t = X[u * LD + b0 + k];
+        a.SH[oo[b0 + k] + u] = make_float2(t.y, t.x);
+      }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Inverse row pass: half spectra SH[plane][v][row] -> real rows; crop and activation on store, or the
+// padding adjoint (pad >= 0, see k_rows_inv).
+// ------------------------------------------------------------------------------------------------
+struct RowsInvArgs {
+  const float2* SH;
+  float* out;
+  float* side;
+  const float2* tw;
+  int Hs, NCs, row0, nrows, col0, ncols, act, npair, total, nblk;
+  int vec;          // 16-byte loads of a row pair (Hs and row0 even, SH 16-byte aligned)
+  int pad, pmode, dst_off;
+  uint32_t mg_cols;
+  LinePlan plan;
+};
+
+__global__ void __launch_bounds__(kLineThreads) k_lines_rows_inv(RowsInvArgs) {
+  const CVN_KARG RowsInvArgs& a = *(const CVN_KARG RowsInvArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int NB = kLines, LD = kLineLd;
+  const int tid = threadIdx.x, nth = blockDim.x, L = a.plan.L;
+  float2* buf = (float2*)smem;
+  float2* tw = (float2*)(smem + ((size_t)L * LD * sizeof(float2) + 15) / 16 * 16);
+  unsigned short* ipos = (unsigned short*)(tw + a.plan.T);
+  float** dst = (float**)(smem + a.dst_off);  // 2 NB: each row's destination, null: none
+  int* csrc = (int*)(dst + 2 * NB);
+  const int g0 = line_item(blockIdx.x, a.nblk) * NB;
+  const int Hd = a.nrows - 2 * a.pad, Wd = a.ncols - 2 * a.pad;  // the unpadded grid (pad >= 0)
+  const int cols = a.pad >= 0 ? Wd : a.ncols, c0 = a.pad >= 0 ? a.pad : a.col0;
+  const int nbd = (a.pad < 0 || a.pmode == CVN_PAD_ZEROS) ? 0 : 2 * a.pad;
+  if (tid < 2 * NB) {
+    const int gp = g0 + (tid >> 1);
+    const int plane = gp / a.npair, r = 2 * (gp - plane * a.npair) + (tid & 1);
+    float* d = nullptr;
+    if (gp < a.total && r < a.nrows) {
+      if (a.pad < 0) d = a.out + ((int64_t)plane * a.nrows + r) * cols;
+      else if (r >= a.pad && r < a.pad + Hd) d = a.out + ((int64_t)plane * Hd + (r - a.pad)) * cols;
+      else if (nbd > 0) d = a.side + ((int64_t)plane * nbd + (r < a.pad ? r : r - Hd)) * cols;
+    }
+    dst[tid] = d;
+  }
+  line_tables(a.plan, a.tw, ipos, tw, tid, nth);
+  for (int q = tid; q < nbd; q += nth)
+    csrc[q] = line_pad_src(q < a.pad ? q : Wd + q, Wd, a.pad, a.pmode);
+  __syncthreads();
+  {
+    const int b = tid % NB, gp = min(g0 + b, a.total - 1);
+    const int plane = gp / a.npair, r = 2 * (gp - plane * a.npair);
+    const float2* in = a.SH + (int64_t)plane * a.NCs * a.Hs + a.row0 + r;
+    const bool two = r + 1 < a.nrows;
+    for (int v0 = tid / NB; v0 < a.NCs; v0 += 4 * (nth / NB)) {
+      float2 fa[4], fb[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int v = min(v0 + k * (nth / NB), a.NCs - 1);
+        const float2* s = in + (int64_t)v * a.Hs;
+        if (a.vec) {
+          const float4 t = *(const float4*)s;
+          fa[k] = make_float2(t.x, t.y);
+          fb[k] = make_float2(t.z, t.w);
+        } else {
+          fa[k] = s[0];
+          fb[k] = two ? s[1] : make_float2(0.f, 0.f);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int v = v0 + k * (nth / NB);
+        if (v >= a.NCs) break;
+        if (v == 0 || 2 * v == L) fa[k].y = fb[k].y = 0.f;
+        // Z = Fa + i Fb and its mirror conj Fa + i conj Fb, real and imaginary parts exchanged
+        buf[ipos[v] * LD + b] = make_float2(fa[k].y + fb[k].x, fa[k].x - fb[k].y);
+        if (v > 0 && 2 * v < L) buf[ipos[L - v] * LD + b] = make_float2(fb[k].x - fa[k].y, fa[k].x + fb[k].y);
+      }
+    }
+  }
+  __syncthreads();
+  line_fft<false>(a.plan, smem, tw, tid, nth);
+  // buf[n LD + b] = (row 2 t + 1, row 2 t) of line b
+  if (nbd > 0) {
+    // border columns onto their padding sources: columns j <= pad or j >= Wd - 1 - pad
+    const bool all = Wd <= 2 * a.pad + 2;
+    const int ne = all ? Wd : 2 * a.pad + 2, b = tid % NB;
+    for (int e = tid / NB; e < ne; e += nth / NB) {
+      const int j = (all || e <= a.pad) ? e : Wd - 1 - a.pad + (e - a.pad - 1);
+      float2 v = buf[(j + a.pad) * LD + b];
+      for (int q = 0; q < nbd; ++q)
+        if (csrc[q] == j) {
+          const float2 z = buf[(q < a.pad ? q : Wd + q) * LD + b];
+          v.x += z.x;
+          v.y += z.y;
+        }
+      buf[(j + a.pad) * LD + b] = v;
+    }
+    __syncthreads();
+  }
+  for (int idx = tid; idx < cols * (NB / 4); idx += nth) {
+    const int q = mg_div(idx, a.mg_cols, cols), j = idx - q * cols, b0 = 4 * q;
+    float2 z[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      z[k] = buf[(c0 + j) * LD + b0 + k];
+      if (a.act == CVN_ACT_GELU) z[k] = make_float2(gelu_fast(z[k].x), gelu_fast(z[k].y));
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float *da = dst[2 * (b0 + k)], *db = dst[2 * (b0 + k) + 1];
+      if (da) da[j] = z[k].y;
+      if (db) db[j] = z[k].x;
+    }
+  }
+}
+
+std::atomic<uint64_t> g_line_attr{0};
+void line_attrs() {
+  once_per_device(g_line_attr, [] {
+    for (const void* k : {(const void*)k_lines_rows_fwd, (const void*)k_lines_rows_inv, (const void*)k_lines_cols<true>,
+                          (const void*)k_lines_cols<false>})
+      (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLineLds);
+    (void)hipGetLastError();
+  });
+}
+
+// Threads per block.  The kernels take up to 128 VGPRs, so a CU holds 16 waves.  Measured over 27 lengths
+// from 24 to 560 (1 to 16 waves per block): a power of two near one wave per 64 elements of length (16
+// elements per thread) is the fastest or within 6 % of it, and an uneven share of the 16 waves (3, 5) up to
+// 30 % slower.  Where the blocks are too few to fill the chip, waves are doubled while all blocks stay
+// resident and the widest pass still gives every wave a butterfly per lane (64 planes of 136 x 136: 37 -> 28 us).
+int line_threads(const LinePlan& p, int nblk) {
+  int w = 1, most = 1;
+  while (w < 16 && w * 64 * 1.41421 < p.L) w *= 2;
+  for (int t = 0; t < p.np; ++t) most = std::max(most, p.ps[t].nl * kLines);
+  while (2 * w <= 16 && (int64_t)nblk * 2 * w <= 256 * 16 && 64 * w < most) w *= 2;
+  return std::max(64 * w, line_min_threads(p));
+}
+
+}  // namespace
+
+bool lines_rows_ok(int64_t P, int h, int w) { return w <= kLineMax && P * ((h + 1) / 2) < (1 << 30); }
+
+int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, int mode, int h, int w,
+                          const float2* tw, float2* S, hipStream_t st) {
+  RowsFwdArgs a;
+  const LinePlan* lp = line_plan(w);
+  if (!lp) return fail(CVN_ERR_UNSUPPORTED, "no plan for length %d", w);
+  a.plan = *lp;
+  line_attrs();
+  a.x = x; a.S = S; a.tw = tw; a.Hin = Hin; a.Win = Win; a.h = h; a.pad = pad; a.mode = mode;
+  a.NC = w / 2 + 1;
+  a.npair = (h + 1) / 2;
+  a.total = (int)(P * a.npair);
+  a.vec = h % 2 == 0 && ((uintptr_t)S & 15) == 0;
+  const size_t lds = line_buf_bytes(w) + line_tab_bytes(a.plan) + 2 * kLines * sizeof(int64_t);
+  a.nblk = (a.total + kLines - 1) / kLines;
+  hipLaunchKernelGGL(k_lines_rows_fwd, dim3((unsigned)a.nblk), dim3(line_threads(a.plan, a.nblk)), lds, st, a);
+  return check_launch("row forward pass");
+}
+
+bool lines_cols_ok(int64_t P, int h, int Hs, int NCs) {
+  if (Hs > kLineMax || P * NCs >= (1 << 30)) return false;
+  if (Hs == h) return true;
+  return line_buf_bytes(h) + line_buf_bytes(Hs) + line_tab_bytes(*line_plan(h)) + line_tab_bytes(*line_plan(Hs)) +
+                 3 * kLines * sizeof(int64_t) <= kLineLds;
+}
+
+int launch_lines_cols(const float2* S, const float2* phi, float2* SH, int64_t B, int64_t C, int64_t psf_batch, int h,
+                      int w, int Hs, int Ws, const float2* tw_h, const float2* tw_H, hipStream_t st) {
+  ColsArgs a;
+  const LinePlan *lh = line_plan(h), *lH = line_plan(Hs);
+  if (!lh || !lH) return fail(CVN_ERR_UNSUPPORTED, "no plan for column length");
+  a.ph = *lh;
+  a.pH = *lH;
+  line_attrs();
+  const bool one = Hs == h;
+  a.S = S; a.phi = phi; a.SH = SH; a.tw_h = tw_h; a.tw_H = tw_H;
+  a.B = (int)B; a.C = (int)C; a.psf_batch = (int)psf_batch;
+  a.w = w; a.Hs = Hs; a.NC = w / 2 + 1; a.NCs = Ws / 2 + 1;
+  a.total = (int)(B * C * a.NCs);
+  size_t lds = line_buf_bytes(Hs) + line_tab_bytes(a.ph) + 3 * kLines * sizeof(int64_t);
+  if (!one) lds += line_buf_bytes(h) + line_tab_bytes(a.pH);
+  a.nblk = (a.total + kLines - 1) / kLines;
+  const dim3 grid((unsigned)a.nblk), block(std::max(line_threads(a.ph, a.nblk), line_threads(a.pH, a.nblk)));
+  if (one) hipLaunchKernelGGL(k_lines_cols<true>, grid, block, lds, st, a);
+  else hipLaunchKernelGGL(k_lines_cols<false>, grid, block, lds, st, a);
+  return check_launch("column pass");
+}
+
+int launch_lines_rows_inv(const float2* SH, int64_t P, int Hs, int Ws, int row0, int nrows, int col0, int ncols, int act,
+                          const float2* tw, float* out, hipStream_t st, int pad, int pmode, float* side) {
+  RowsInvArgs a;
+  const LinePlan* lp = line_plan(Ws);
+  if (!lp) return fail(CVN_ERR_UNSUPPORTED, "no plan for length %d", Ws);
+  a.plan = *lp;
+  line_attrs();
+  a.SH = SH; a.out = out; a.side = side; a.tw = tw; a.Hs = Hs; a.NCs = Ws / 2 + 1;
+  a.row0 = row0; a.nrows = nrows; a.col0 = col0; a.ncols = ncols; a.act = act;
+  a.pad = pad; a.pmode = pmode;
+  a.npair = (nrows + 1) / 2;
+  a.total = (int)(P * a.npair);
+  a.vec = Hs % 2 == 0 && row0 % 2 == 0 && nrows % 2 == 0 && ((uintptr_t)SH & 15) == 0;
+  a.mg_cols = line_magic(pad >= 0 ? ncols - 2 * pad : ncols);
+  a.dst_off = (int)(line_buf_bytes(Ws) + line_tab_bytes(a.plan));
+  const size_t lds = a.dst_off + 2 * kLines * sizeof(float*) + sizeof(int) * 2 * std::max(pad, 0);
+  a.nblk = (a.total + kLines - 1) / kLines;
+  hipLaunchKernelGGL(k_lines_rows_inv, dim3((unsigned)a.nblk), dim3(line_threads(a.plan, a.nblk)), lds, st, a);
+  return check_launch("row inverse pass");
+}
+
+}  // namespace cvn

@@ -206,4 +206,15 @@ int launch_module_ct(const float* x, int64_t P, int64_t C, int64_t psf_batch, in
                      const float2* tw_w, const float2* tw_h, const float2* tw_Hs, const float2* tw_Ws,
                      const float2* phi, float2* S, float2* SH, float* out, hipStream_t st);
 
+// Row and column passes on the in-place prime-factor engine (converse2d_lines.hip), lengths up to 1024.
+// Same scratch, table and twiddle layouts as the runtime-plan passes; tw_*: exp(-2 pi i m / L), m < L.
+bool lines_rows_ok(int64_t P, int h, int w);
+int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, int mode, int h, int w,
+                          const float2* tw, float2* S, hipStream_t st);
+bool lines_cols_ok(int64_t P, int h, int Hs, int NCs);
+int launch_lines_cols(const float2* S, const float2* phi, float2* SH, int64_t B, int64_t C, int64_t psf_batch, int h,
+                      int w, int Hs, int Ws, const float2* tw_h, const float2* tw_H, hipStream_t st);
+int launch_lines_rows_inv(const float2* SH, int64_t P, int Hs, int Ws, int row0, int nrows, int col0, int ncols, int act,
+                          const float2* tw, float* out, hipStream_t st, int pad, int pmode, float* side);
+
 }  // namespace cvn

@@ -1,0 +1,99 @@
+"""The in-place prime-factor row and column passes (csrc/fft_lines.h) against the fp64 oracle: every length
+up to 1024, so every radix, every Cooley-Tukey part and every dense prime, in rows and in columns.
+
+Tolerance (relative 2-norm): a call makes four transforms, each of at most 5 rounded operations per pass and
+element, 3 passes; at 6e-8 per rounding and independent errors that is 4 sqrt(15) 6e-8 = 9e-7.  A dense prime adds
+chunked sums of up to 512 terms, sqrt((32 + 512 / 32) / 6) roundings, 4 * 2.8 * 6e-8 = 7e-7.  Gate: 3e-6, above the
+sum of both."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import converse_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+TOL = 3e-6
+
+
+def _t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def _inputs(B, C, H, W, k, seed, pb=1):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((B, C, H, W)).astype(np.float32)
+    w = rng.random((pb, C, k, k))
+    w = (w / w.sum(axis=(2, 3), keepdims=True)).astype(np.float32)
+    b = (0.3 * rng.standard_normal((1, C, 1, 1))).astype(np.float32)
+    return x, w, b
+
+
+def _check(x, w, b, s, p, mode, what):
+    from conversenet_amd import functional as Fh
+
+    ref = O.converse2d_module(x, w, b, s, p, mode, 1e-5)
+    got = Fh.converse2d_fused(_t(x), _t(w), _t(b).reshape(-1), s, p, mode, 1e-5, cache=False).cpu().numpy()
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= TOL, (what, err)
+
+
+@pytest.mark.parametrize("first", range(1, 1025, 128))
+def test_every_length(first):
+    """Rows of L samples (5 rows: an odd count leaves half a pair) and columns of L samples."""
+    for L in range(first, first + 128):
+        for H, W in ((5, L), (L, 3)):
+            x, w, b = _inputs(1, 2, H, W, 1 if min(H, W) < 3 else 3, L)
+            _check(x, w, b, 1, 0, "circular", (H, W))
+
+
+# (B, C, H, W, k, s, p, mode, psf batch): blocks that straddle planes and channels, odd rows and crops, a
+# mirrored LR column at s > 1, dense primes (37, 61, 127) and staged parts (49, 64, 81, 343) in both directions
+CASES = [
+    (3, 5, 31, 29, 3, 1, 4, "circular", 1),     # 39 x 37
+    (2, 3, 33, 57, 5, 1, 2, "reflect", 2),      # 37 x 61
+    (2, 3, 55, 123, 7, 1, 3, "replicate", 1),   # 61 x 129
+    (1, 2, 115, 331, 7, 1, 6, "constant", 1),   # 127 x 343
+    (2, 7, 20, 23, 2, 2, 2, "replicate", 1),    # 48 x 54
+    (1, 3, 15, 25, 3, 3, 1, "circular", 1),     # 51 x 81
+    (2, 2, 12, 33, 5, 4, 2, "reflect", 2),      # 64 x 148
+    (1, 2, 60, 41, 3, 2, 1, "constant", 1),     # 124 x 86
+    (2, 2, 130, 91, 3, 5, 2, "circular", 1),    # 670 x 475: two column buffers, scale above 4
+    (1, 1, 250, 1, 3, 4, 2, "replicate", 1),    # 1016 x 20: LR and HR columns exceed LDS together
+]
+
+
+@pytest.mark.parametrize("B,C,H,W,k,s,p,mode,pb", CASES)
+def test_shapes_modes_scales(B, C, H, W, k, s, p, mode, pb):
+    x, w, b = _inputs(B, C, H, W, k, 7 * H + W, pb)
+    _check(x, w, b, s, p, mode, (H, W, s, p))
+
+
+def test_misaligned_scratch_and_infinite_plane():
+    """Spectra scratch at 8 bytes past a 16-byte boundary (no 16-byte accesses), and a plane of infinities and
+    NaN that shares its blocks with finite planes, which it must not touch."""
+    from conversenet_amd import _lib
+    from conversenet_amd import functional as Fh
+
+    x, w, b = _inputs(3, 2, 34, 44, 3, 5)
+    x[1, 0] = np.nan
+    x[1, 1, 3, 4] = np.inf
+    ref = O.converse2d_module(np.where(np.isfinite(x), x, 0), w, b, 1, 1, "circular", 1e-5)
+    xt, wt, bt = _t(x), _t(w), _t(b).reshape(-1)
+    got = Fh.converse2d_fused(xt, wt, bt, 1, 1, "circular", 1e-5, cache=False).cpu().numpy()
+    lib = _lib.load()
+    geo = (3, 2, 34, 44, 1, 3, 3, 1, 1)
+    route, mode = lib.cvn_converse2d_route(*geo), _lib.PAD_MODES["circular"]
+    tb, sb = lib.cvn_converse2d_table_bytes(*geo, route), lib.cvn_converse2d_scratch_bytes(*geo, route)
+    table = torch.empty(tb, dtype=torch.uint8, device=DEV)
+    scratch = torch.empty(sb + 8, dtype=torch.uint8, device=DEV)
+    out = torch.empty(3, 2, 34, 44, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib.cvn_converse2d_table_f32(wt.data_ptr(), 1, 3, 3, bt.data_ptr(), 1e-5, 3, 2, 34, 44, 1, 1, route,
+                                        table.data_ptr(), tb, st) == 0
+    assert lib.cvn_converse2d_apply_f32(xt.data_ptr(), 3, 2, 34, 44, 1, 3, 3, 1, 1, mode, 0, route, table.data_ptr(), tb,
+                                        scratch.data_ptr() + 8, sb, out.data_ptr(), st) == 0
+    for y in (got, out.cpu().numpy()):
+        for i in (0, 2):
+            assert np.linalg.norm(y[i] - ref[i]) / np.linalg.norm(ref[i]) <= TOL
+        assert np.isnan(y[1]).all()

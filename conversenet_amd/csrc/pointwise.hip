@@ -241,10 +241,10 @@ __device__ __forceinline__ void zero_acc(v4f (&acc)[COUT / 16][Q]) {
 
 // Epilogue: bias, activation, optional alpha-scaled residual, vector store.  yw / rw: output and
 // residual at channel 0 and the wave's first pixel; yoff: lane offset of channel 4 g, pixel Q j;
-// bias / res_scale: per-channel vectors staged in LDS.
+// bias / res_scale: per-channel vectors staged in LDS; inv: the weights' scale undone (StageF16; 1 without).
 template <int COUT, int Q>
 __device__ __forceinline__ void store_tile(v4f (&acc)[COUT / 16][Q], float* yw, const float* rw, int64_t HW,
-                                           bool inb, uint32_t yoff, int g, const float* bias, int act,
+                                           bool inb, uint32_t yoff, int g, float inv, const float* bias, int act,
                                            const float* res_scale) {
   if (!inb) return;
 #pragma unroll
@@ -257,7 +257,7 @@ __device__ __forceinline__ void store_tile(v4f (&acc)[COUT / 16][Q], float* yw, 
       float v[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        v[q] = acc[rb][q][r] + bo;
+        v[q] = fmaf(acc[rb][q][r], inv, bo);
         if (act == CVN_ACT_GELU) v[q] = gelu_f(v[q]);
       }
       if (rw) {
@@ -284,10 +284,12 @@ __device__ __forceinline__ int64_t tile_px(int64_t t, int64_t tpb, int Q, int NW
 
 // ------------------------------------------------------------------------------------------------
 // fp32 products on the fp16 matrix cores ("split fp16").  Every operand x is split as x = x_h + x_l,
-// x_h = fp16(x) and x_l = fp16(x - x_h), both rounded toward zero (x - x_h is exact in fp32), so
-// |x - x_h - x_l| < 2^-20 |x|; a product is formed as a_l b_h + a_h b_l + a_h b_h (three
-// v_mfma_f32_16x16x32_f16, each product exact in the fp32 accumulator), dropping a_l b_l (< 2^-20
-// |a b|).  fp16 inputs below the normal range are kept by the matrix cores (gradual underflow), so
+// x_h = fp16(x) and x_l = fp16(x - x_h), both rounded to nearest (x - x_h is exact in fp32), so
+// |x - x_h - x_l| <= 2^-22 |x|; a product is formed as a_l b_h + a_h b_l + a_h b_h (three
+// v_mfma_f32_16x16x32_f16, each product exact in the fp32 accumulator), dropping a_l b_l (<= 2^-22
+// |a b|).  The errors have random signs (rounded toward zero, as these splits were at first, they are
+// 2^-20 and one-sided: a ConverseBlock's relative error against fp64 was 1.1e-6, now 2.9e-7; with torch's
+// fp32 1x1 convolutions it is 3.1e-7).  fp16 inputs below the normal range are kept by the matrix cores (gradual underflow), so
 // small values lose no relative accuracy beyond 2^-24 absolute.  A 16 x 16 x 32 block update then
 // takes three of these MFMAs (8192 multiply-adds each, half the issue time of one 16x16x4 fp32 MFMA)
 // instead of eight fp32 MFMAs.  fp16's range ends at 65504: a k-chunk whose activations exceed it in
@@ -300,6 +302,8 @@ __device__ __forceinline__ int64_t tile_px(int64_t t, int64_t tpb, int Q, int NW
 // a layer's accumulators feed the next layer's B operand directly.
 // ------------------------------------------------------------------------------------------------
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 constexpr float kF16Max = 65504.f;
 
@@ -307,8 +311,9 @@ __device__ __forceinline__ void split_f16(const float (&x)[8], f16x8& h, f16x8& 
   u32x4_t H, L;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const auto hp = __builtin_amdgcn_cvt_pkrtz(x[2 * i], x[2 * i + 1]);
-    const auto lp = __builtin_amdgcn_cvt_pkrtz(x[2 * i] - (float)hp[0], x[2 * i + 1] - (float)hp[1]);
+    const f16x2 hp = __builtin_convertvector((f32x2){x[2 * i], x[2 * i + 1]}, f16x2);  // v_cvt_pk_f16_f32
+    const f16x2 lp =
+        __builtin_convertvector((f32x2){x[2 * i] - (float)hp[0], x[2 * i + 1] - (float)hp[1]}, f16x2);
     H[i] = __builtin_bit_cast(unsigned, hp);
     L[i] = __builtin_bit_cast(unsigned, lp);
   }
@@ -319,19 +324,52 @@ __device__ __forceinline__ void split_f16(const float (&x)[8], f16x8& h, f16x8& 
 // Weights (N outputs x K inputs, row-major fp32) in LDS for gemm_f16s: for input chunk c, output
 // block ob and lane 16 g + j, 16 bytes of high parts (W[16 ob + j][channel of k slot 8 g + e], e < 8),
 // and 1 KB further on the 16 bytes of low parts: consecutive lanes read consecutive 16-byte words.
-template <int N, int K>
-__device__ __forceinline__ void stage_f16s(const float* __restrict__ W, _Float16* Wl) {
-  for (int e = threadIdx.x; e < N * K; e += blockDim.x) {
+// The matrix is scaled by a power of two that brings its largest entry to [64, 128): a weight of 0.1 has
+// its low part below fp16's normal range (2^-14), where the spacing of 2^-24 is 3e-7 of it, several times
+// the split's own error.  The caller multiplies the sums by the returned reciprocal, in the fma that
+// adds the bias.  load() reads the block's share into registers and joins the matrix' maximum, put()
+// writes it; between the two the block synchronises (after put() too, before the first use).
+template <int N, int K, int T>
+struct StageF16 {
+  static constexpr int PER = (N * K + T - 1) / T;
+  float w[PER];
+  __device__ __forceinline__ static int src(int e) {
     const int e8 = e & 7, lj = (e >> 3) & 63, cob = e >> 9;
     const int g = lj >> 4, j = lj & 15, hf = e8 >> 2, r = e8 & 3;
     const int ob = cob % (N / 16), c = cob / (N / 16);
-    const float w = W[(16 * ob + j) * K + 16 * (2 * c + hf) + 4 * g + r];
-    const auto hp = __builtin_amdgcn_cvt_pkrtz(w, 0.f);
-    const auto lp = __builtin_amdgcn_cvt_pkrtz(w - (float)hp[0], 0.f);
-    Wl[cob * 1024 + lj * 8 + e8] = (_Float16)hp[0];
-    Wl[cob * 1024 + 512 + lj * 8 + e8] = (_Float16)lp[0];
+    return (16 * ob + j) * K + 16 * (2 * c + hf) + 4 * g + r;
   }
-}
+  __device__ __forceinline__ void load(const float* __restrict__ W, unsigned* top) {
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = threadIdx.x + i * T;
+      w[i] = (N * K % T == 0 || e < N * K) ? W[src(e)] : 0.f;
+      m = fmaxf(m, fabsf(w[i]));
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
+    if ((threadIdx.x & 63) == 0) atomicMax(top, __float_as_uint(m));  // m >= 0: ordered as its bits
+  }
+  __device__ __forceinline__ float put(const unsigned* top, _Float16* Wl) const {
+    // exponent of the largest entry, kept inside +-100; zero or infinite entries alone scale by 1
+    const int e2 = (int)(*top >> 23) - 127;
+    const int s = *top == 0 || e2 == 128 ? 0 : 6 - max(-100, min(e2, 100));
+    const float sc = ldexpf(1.f, s);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = threadIdx.x + i * T;
+      if (N * K % T == 0 || e < N * K) {
+        const int d = (e >> 9) * 1024 + (e & 511);
+        const float v = w[i] * sc;
+        const _Float16 h = (_Float16)v;
+        Wl[d] = h;
+        Wl[d + 512] = (_Float16)(v - (float)h);
+      }
+    }
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(ldexpf(1.f, -s))));
+  }
+};
 
 // acc[ob][q] += W[16 ob + j][k] v[k] over all K input channels; v in the accumulator layout.
 template <int K, int N, int Q>
@@ -372,7 +410,7 @@ __device__ __forceinline__ void gemm_f16s(const v4f (&v)[K / 16][Q], const _Floa
         const f16x8 ah = __builtin_bit_cast(f16x8, wp[0]), al = __builtin_bit_cast(f16x8, wp[64]);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float w = (float)ah[e] + (float)al[e];
+          const float w = (float)ah[e] + (float)al[e];  // (scaled like the fp16 products)
 #pragma unroll
           for (int q = 0; q < Q; ++q) acc[ob][q] = mfma4(w, xb[q][e], acc[ob][q]);
         }
@@ -453,8 +491,18 @@ __global__ void __launch_bounds__(64 * NW) k_conv1x1_mfma(const float* __restric
   constexpr int LD = COUT + 16;  // (4 ks + g) LD + j + 16 rb: 16 g + j distinct banks
   __shared__ __align__(16) float Wt[F16S ? COUT * CIN : CIN * LD];
   __shared__ float prm[2 * COUT + 2 * CIN];  // bias, residual scale, LN weight, LN bias
-  if constexpr (F16S) stage_f16s<COUT, CIN>(W, (_Float16*)Wt);
-  else stage_wt<COUT, CIN, LD>(W, Wt);
+  float inv = 1.f;
+  if constexpr (F16S) {
+    __shared__ unsigned top;
+    if (threadIdx.x == 0) top = 0;
+    __syncthreads();
+    StageF16<COUT, CIN, 64 * NW> sw;
+    sw.load(W, &top);
+    __syncthreads();
+    inv = sw.put(&top, (_Float16*)Wt);
+  } else {
+    stage_wt<COUT, CIN, LD>(W, Wt);
+  }
   stage_vec<COUT>(bias, 0.f, prm);
   stage_vec<COUT>(res_scale, 1.f, prm + COUT);
   if (LN) {
@@ -490,7 +538,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv1x1_mfma(const float* __restric
       gemm_tile<CIN, COUT, Q>(xv, Wt, LD, g, j, acc);
     }
     store_tile<COUT, Q>(acc, y + b * COUT * hw + pw, residual ? residual + b * COUT * hw + pw : nullptr, hw, inb,
-                        yoff, g, prm, act, prm + COUT);
+                        yoff, g, inv, prm, act, prm + COUT);
   }
 }
 
@@ -503,11 +551,18 @@ __global__ void __launch_bounds__(64 * NW) k_ln_mlp_mfma(const float* x, int64_t
                                                      const float* __restrict__ b2,
                                                      const float* __restrict__ res_scale, float* y) {
   static_assert(C % 32 == 0 && CM % 32 == 0, "split-fp16 GEMM chunks");
-  __shared__ __align__(16) _Float16 W1l[2 * CM * C];  // stage_f16s layouts
+  __shared__ __align__(16) _Float16 W1l[2 * CM * C];  // StageF16 layouts
   __shared__ __align__(16) _Float16 W2l[2 * C * CM];
   __shared__ float prm[CM + 4 * C];  // b1, b2, residual scale, LN weight, LN bias
-  stage_f16s<CM, C>(W1, W1l);
-  stage_f16s<C, CM>(W2, W2l);
+  __shared__ unsigned top[2];
+  if (threadIdx.x < 2) top[threadIdx.x] = 0;
+  __syncthreads();
+  StageF16<CM, C, 64 * NW> s1;
+  StageF16<C, CM, 64 * NW> s2;
+  s1.load(W1, top);
+  s2.load(W2, top + 1);
+  __syncthreads();
+  const float inv1 = s1.put(top, W1l), inv2 = s2.put(top + 1, W2l);
   stage_vec<CM>(b1, 0.f, prm);
   stage_vec<C>(b2, 0.f, prm + CM);
   stage_vec<C>(res_scale, 1.f, prm + CM + C);
@@ -539,12 +594,12 @@ __global__ void __launch_bounds__(64 * NW) k_ln_mlp_mfma(const float* x, int64_t
       for (int r = 0; r < 4; ++r) {
         const float bo = prm[16 * rb + 4 * g + r];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(h[rb][q][r] + bo);
+        for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(fmaf(h[rb][q][r], inv1, bo));
       }
     v4f acc[C / 16][Q];
     zero_acc<C, Q>(acc);
     gemm_f16s<CM, C, Q>(h, W2l, lane, acc);
-    store_tile<C, Q>(acc, y + b * C * hw + pw, xw, hw, inb, yoff, g, prm + CM, CVN_ACT_NONE, prm + CM + C);
+    store_tile<C, Q>(acc, y + b * C * hw + pw, xw, hw, inb, yoff, g, inv2, prm + CM, CVN_ACT_NONE, prm + CM + C);
   }
 }
 
@@ -586,14 +641,26 @@ template <int CIN, int C, int CM, int Q, int NW, bool HEAD, bool GIN>
 __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
   static_assert(CIN % 32 == 0 && C % 32 == 0 && CM % 32 == 0, "split-fp16 GEMM chunks");
   constexpr int NP = 6 * C + CM + (HEAD ? 2 * C + CIN : 0);
-  __shared__ __align__(16) _Float16 W0l[2 * C * CIN];  // stage_f16s layouts
+  __shared__ __align__(16) _Float16 W0l[2 * C * CIN];  // StageF16 layouts
   __shared__ __align__(16) _Float16 W1l[2 * CM * C];
   __shared__ __align__(16) _Float16 W2l[2 * C * CM];
   __shared__ __align__(16) _Float16 Whl[HEAD ? 2 * CIN * C : 8];
   __shared__ float prm[NP];  // b0, s1, LN weight, LN bias, b2, s2, b1 [, head LN weight, bias, head bias]
-  stage_f16s<C, CIN>(a.W0, W0l);
-  stage_f16s<CM, C>(a.W1, W1l);
-  stage_f16s<C, CM>(a.W2, W2l);
+  __shared__ unsigned top[4];
+  if (threadIdx.x < 4) top[threadIdx.x] = 0;
+  __syncthreads();
+  StageF16<C, CIN, 64 * NW> sw0;
+  StageF16<CM, C, 64 * NW> sw1;
+  StageF16<C, CM, 64 * NW> sw2;
+  StageF16<CIN, HEAD ? C : 16, 64 * NW> swh;
+  sw0.load(a.W0, top);
+  sw1.load(a.W1, top + 1);
+  sw2.load(a.W2, top + 2);
+  if constexpr (HEAD) swh.load(a.Wh, top + 3);
+  __syncthreads();
+  const float inv0 = sw0.put(top, W0l), inv1 = sw1.put(top + 1, W1l), inv2 = sw2.put(top + 2, W2l);
+  float invh = 1.f;
+  if constexpr (HEAD) invh = swh.put(top + 3, Whl);
   stage_vec<C>(a.b0, 0.f, prm);
   stage_vec<C>(a.s1, 1.f, prm + C);
   stage_vec<C>(a.lw, 1.f, prm + 2 * C);
@@ -602,7 +669,6 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
   stage_vec<C>(a.s2, 1.f, prm + 5 * C);
   stage_vec<CM>(a.b1, 0.f, prm + 6 * C);
   if (HEAD) {
-    stage_f16s<CIN, C>(a.Wh, Whl);
     stage_vec<C>(a.hlw, 1.f, prm + 6 * C + CM);
     stage_vec<C>(a.hlb, 0.f, prm + 7 * C + CM);
     stage_vec<CIN>(a.bh, 0.f, prm + 8 * C + CM);
@@ -649,7 +715,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         }
         const float bo = prm[o], sc = prm[C + o];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) acc[rb][q][r] = fmaf(sc, acc[rb][q][r] + bo, rr[q]);
+        for (int q = 0; q < Q; ++q) acc[rb][q][r] = fmaf(sc, fmaf(acc[rb][q][r], inv0, bo), rr[q]);
       }
     // out = y' + s2 (W2 GELU(W1 LN(y') + b1) + b2)
     v4f acc2[C / 16][Q];
@@ -667,7 +733,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         for (int r = 0; r < 4; ++r) {
           const float bo = prm[6 * C + 16 * rb + 4 * g + r];
 #pragma unroll
-          for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(h[rb][q][r] + bo);
+          for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(fmaf(h[rb][q][r], inv1, bo));
         }
       zero_acc<C, Q>(acc2);
       gemm_f16s<CM, C, Q>(h, W2l, lane, acc2);
@@ -679,7 +745,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         const int o = 16 * rb + 4 * g + r;
         const float bo = prm[4 * C + o], sc = prm[5 * C + o];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) acc2[rb][q][r] = fmaf(sc, acc2[rb][q][r] + bo, acc[rb][q][r]);
+        for (int q = 0; q < Q; ++q) acc2[rb][q][r] = fmaf(sc, fmaf(acc2[rb][q][r], inv2, bo), acc[rb][q][r]);
       }
     if (inb) store_acc<C, Q>(acc2, a.y + b * C * hw + pw, hw, yoff);
     if (HEAD) {
@@ -697,7 +763,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         for (int r = 0; r < 4; ++r) {
           const float bo = prm[8 * C + CM + 16 * rb + 4 * g + r];
 #pragma unroll
-          for (int q = 0; q < Q; ++q) hh[rb][q][r] = gelu_f(hh[rb][q][r] + bo);
+          for (int q = 0; q < Q; ++q) hh[rb][q][r] = gelu_f(fmaf(hh[rb][q][r], invh, bo));
         }
       if (inb) store_acc<CIN, Q>(hh, a.th + b * CIN * hw + pw, hw, yoff);
     }
@@ -813,11 +879,12 @@ unsigned persistent_grid(K kernel, int threads, int64_t ntiles) {
   return (unsigned)std::min<int64_t>(ntiles, r);
 }
 
-template <int CIN, int COUT, bool LN>
+// ONE: one pixel per lane and 16-pixel tile, dword accesses only: any pixel count and alignment
+template <int CIN, int COUT, bool LN, bool ONE>
 int launch_mfma(const float* x, int64_t B, int64_t HW, const float* W, const float* bias, const float* lw,
                 const float* lb, float eps, int act, const float* residual, const float* res_scale, float* y,
                 hipStream_t st) {
-  constexpr int Q = ConvTile<CIN, COUT, LN>::Q, NW = ConvTile<CIN, COUT, LN>::NW;
+  constexpr int Q = ONE ? 1 : ConvTile<CIN, COUT, LN>::Q, NW = ConvTile<CIN, COUT, LN>::NW;
   const int64_t tpb = (HW + 16 * NW * Q - 1) / (16 * NW * Q), ntiles = B * tpb;
   auto kern = k_conv1x1_mfma<CIN, COUT, LN, Q, NW, ConvTile<CIN, COUT, LN>::F16S>;
   hipLaunchKernelGGL(kern, dim3(persistent_grid(kern, 64 * NW, ntiles)), dim3(64 * NW), 0, st, x, HW, tpb, ntiles,
@@ -854,16 +921,25 @@ int launch_tail(TailArgs a, int64_t B, hipStream_t st) {
   return check_launch("fused block tail");
 }
 
+// vec: pixel count a multiple of 4 and 16-byte aligned buffers.  Otherwise the shapes whose tile is one
+// pixel per lane anyway, and every LayerNorm shape (there is no other kernel for those), run with ONE; the
+// remaining shapes run on the VALU kernel (*done = false).
 template <bool LN>
 int dispatch_mfma(int64_t Cin, int64_t Cout, const float* x, int64_t B, int64_t HW, const float* W,
                   const float* bias, const float* lw, const float* lb, float eps, int act, const float* residual,
-                  const float* res_scale, float* y, hipStream_t st, bool* done) {
+                  const float* res_scale, float* y, hipStream_t st, bool vec, bool* done) {
   *done = true;
-#define CVN_CASE(ci, co) \
-  if (Cin == ci && Cout == co) return launch_mfma<ci, co, LN>(x, B, HW, W, bias, lw, lb, eps, act, residual, res_scale, y, st);
+#define CVN_ARGS x, B, HW, W, bias, lw, lb, eps, act, residual, res_scale, y, st
+#define CVN_CASE(ci, co)                                                                              \
+  if (Cin == ci && Cout == co) {                                                                      \
+    if (vec) return launch_mfma<ci, co, LN, false>(CVN_ARGS);                                         \
+    if constexpr (ConvTile<ci, co, LN>::F16S && (LN || ConvTile<ci, co, LN>::Q == 1))                 \
+      return launch_mfma<ci, co, LN, true>(CVN_ARGS);                                                 \
+  }
   CVN_CASE(64, 64) CVN_CASE(64, 128) CVN_CASE(128, 64) CVN_CASE(128, 128) CVN_CASE(16, 64) CVN_CASE(64, 16)
   CVN_CASE(32, 32) CVN_CASE(32, 64) CVN_CASE(64, 32)
 #undef CVN_CASE
+#undef CVN_ARGS
   *done = false;
   return CVN_OK;
 }
@@ -902,22 +978,20 @@ static int conv_impl(const float* x, int64_t B, int64_t Cin, int64_t HW, const f
   int rc = conv_args_ok(x, B, Cin, HW, weight, Cout, act, y);
   if (rc != CVN_OK) return rc;
   if (B == 0 || HW == 0) return CVN_OK;
+  const bool vec = HW % 4 == 0 && aligned16(x) && aligned16(y) && (!residual || aligned16(residual));
   // the MFMA kernels address a lane's pixels with 32-bit byte offsets within 16 channel rows
-  const bool vec_ok = (HW % 4 == 0) && HW <= kMaxMfmaHW && aligned16(x) && aligned16(y) &&
-                      (!residual || aligned16(residual));
-  if (vec_ok) {
+  if (HW <= kMaxMfmaHW) {
     bool done = false;
     if (ln_w)
       rc = dispatch_mfma<true>(Cin, Cout, x, B, HW, weight, bias, ln_w, ln_b, ln_eps, act, residual, res_scale, y,
-                               st, &done);
+                               st, vec, &done);
     else
       rc = dispatch_mfma<false>(Cin, Cout, x, B, HW, weight, bias, nullptr, nullptr, 0.f, act, residual,
-                                res_scale, y, st, &done);
+                                res_scale, y, st, vec, &done);
     if (done) return rc;
   }
   if (ln_w) return fail(CVN_ERR_UNSUPPORTED, "LayerNorm-fused 1x1 conv needs an MFMA tile shape");
   if ((Cout + kOutGroup - 1) / kOutGroup > 65535) return fail(CVN_ERR_UNSUPPORTED, "too many output channels");
-  const bool vec = HW % 4 == 0 && aligned16(x) && aligned16(y) && (!residual || aligned16(residual));
   const int px = vec ? 4 : 1;
   dim3 grid((unsigned)((HW / px + 255) / 256), (unsigned)B, (unsigned)((Cout + kOutGroup - 1) / kOutGroup));
   if (vec)
@@ -953,9 +1027,8 @@ extern "C" int cvn_ln_mlp_residual_f32(const float* x, int64_t B, int64_t C, int
   if (B < 0 || HW < 0) return fail(CVN_ERR_ARG, "bad shape");
   if (B > 65535) return fail(CVN_ERR_UNSUPPORTED, "batch exceeds 65535");
   if (B == 0 || HW == 0) return CVN_OK;
-  if (HW % 4 != 0 || HW > kMaxMfmaHW || !aligned16(x) || !aligned16(y))
-    return fail(CVN_ERR_UNSUPPORTED,
-                "fused branch needs HW %% 4 == 0, HW <= 2^26 and 16-byte aligned buffers");
+  static_assert(MlpTile<64, 128>::Q == 1 && MlpTile<32, 64>::Q == 1, "dword accesses: any HW and alignment");
+  if (HW > kMaxMfmaHW) return fail(CVN_ERR_UNSUPPORTED, "fused branch needs HW <= 2^26");
   hipStream_t st = (hipStream_t)stream;
   if (C == 64 && Cmid == 128)
     return launch_mlp<64, 128>(x, B, HW, ln_w, ln_b, ln_eps, w1, b1, w2, b2, res_scale, y, st);
@@ -974,9 +1047,8 @@ static int tail_impl(TailArgs a, int64_t B, int64_t Ct, int64_t C, int64_t Cmid,
   if (a.t == a.y || (a.th && (a.th == a.x || a.th == a.y)))
     return fail(CVN_ERR_ARG, "the output may alias x only; the next block's input must be a separate buffer");
   if (B == 0 || a.HW == 0) return CVN_OK;
-  if (a.HW % 4 != 0 || a.HW > kMaxMfmaHW || !aligned16(a.t) || !aligned16(a.x) || !aligned16(a.y) ||
-      (a.th && !aligned16(a.th)))
-    return fail(CVN_ERR_UNSUPPORTED, "fused tail needs HW %% 4 == 0, HW <= 2^26 and 16-byte aligned buffers");
+  // (one pixel per lane and tile, dword accesses: any HW and alignment)
+  if (a.HW > kMaxMfmaHW) return fail(CVN_ERR_UNSUPPORTED, "fused tail needs HW <= 2^26");
   if (Ct == 128 && C == 64 && Cmid == 128) return launch_tail<128, 64, 128>(a, B, st);
   return fail(CVN_ERR_UNSUPPORTED, "fused tail supports (Ct, C, Cmid) = (128, 64, 128)");
 }

@@ -252,7 +252,7 @@ def _gelu_in_tail(parts, t_shape, x):
     inverse row pass is bound by VALU issue at three waves per SIMD (there the GELU costs about 24 us
     of a 0.47 ms layer at Converse-DnCNN's shape; in the tail, about 10 us)."""
     _, _, cv, c15, _, c21, _, _ = parts
-    if (c15.in_channels, c15.out_channels, c21.out_channels) not in functional.TAIL_SHAPES or x.data_ptr() % 16:
+    if (c15.in_channels, c15.out_channels, c21.out_channels) not in functional.TAIL_SHAPES:
         return False
     return functional.module_route(t_shape, cv.weight, cv.scale, cv.padding) == _lib.ROUTE_PFA268
 
@@ -263,8 +263,7 @@ def _block_tail(parts, t, x, next_parts=None, t_act=None):
     Returns (block output, next block's Converse2D input or None)."""
     _, _, _, c15, ln2, c21, c23, (s1, s2) = parts
     mid, C = c15.in_channels, c15.out_channels
-    aligned = t.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
-    if (mid, C, c21.out_channels) in functional.TAIL_SHAPES and aligned:
+    if (mid, C, c21.out_channels) in functional.TAIL_SHAPES:
         if next_parts is not None and next_parts[1].out_channels == mid:
             nln, nc11 = next_parts[0], next_parts[1]
             return functional.conv_ln_mlp_residual(t, x, c15.weight, c15.bias, ln2.weight, ln2.bias, ln2.eps,
@@ -293,7 +292,7 @@ def _fused_block_forward(blk, x, alpha1=None, alpha2=None):
     """LN+1x1+GELU -> Converse2D+GELU -> 1x1+residual and the LN-MLP branch + residual.
     Returns None when a shape is outside the instantiated HIP tiles or the library's limits."""
     parts = _block_parts(blk)
-    if parts is None or (x.shape[2] * x.shape[3]) % 4 != 0 or not _parts_supported(parts, x):
+    if parts is None or not _parts_supported(parts, x):
         return None
     t = _block_head(parts, x)
     gin = _gelu_in_tail(parts, t.shape, x)
@@ -309,8 +308,7 @@ def run_blocks(blocks, x):
     if not blocks:
         return x
     parts = [_block_parts(b) if _hip_eligible(x, *_block_params(b)) else None for b in blocks]
-    if (any(p is None for p in parts) or (x.shape[2] * x.shape[3]) % 4 != 0
-            or not all(_parts_supported(p, x) for p in parts)):
+    if any(p is None for p in parts) or not all(_parts_supported(p, x) for p in parts):
         for b in blocks:
             x = b(x)
         return x

@@ -186,10 +186,11 @@ int cvn_layernorm_cf_f32(const float* x, int64_t B, int64_t C, int64_t HW, const
  * y = (res_scale ? res_scale[o] : 1) * y + residual[b,o,p].  x: (B,Cin,HW), W: (Cout,Cin),
  * bias: (Cout) or NULL, residual: (B,Cout,HW) or NULL, res_scale: (Cout) or NULL.
  * y may alias residual.  Channel counts with a matrix-core tile run on the MFMA units: in whole
- * 32-channel chunks as split-fp16 products (each fp32 operand x = x_h + x_l, two fp16 parts; three
- * fp16 MFMAs accumulating in fp32; relative error per product below 2^-20, a chunk whose activations
- * leave fp16's range falls back to fp32 MFMAs), otherwise as fp32 MFMAs; 1 or 3 channels, and pixel
- * counts not a multiple of 4, run on a VALU kernel in fp32. */
+ * 32-channel chunks as split-fp16 products (each fp32 operand x = x_h + x_l, two fp16 parts rounded to
+ * nearest, the weights scaled by a power of two; three fp16 MFMAs accumulating in fp32; relative error per
+ * product at most 2^-20.4, 2^-23 rms; a chunk whose activations leave fp16's range falls back to fp32
+ * MFMAs), otherwise as fp32 MFMAs; 1 or 3 channels run on a VALU kernel in fp32, as do pixel counts not a
+ * multiple of 4 and misaligned buffers except for 64 <-> 128 channels. */
 int cvn_conv1x1_f32(const float* x, int64_t B, int64_t Cin, int64_t HW, const float* weight,
                     const float* bias, int64_t Cout, int act, const float* residual,
                     const float* res_scale, float* y, cvn_stream_t stream);

@@ -1,0 +1,114 @@
+"""The channel-mixing kernels on pixel counts that are no multiple of 4, on buffers at any 4-byte alignment, and
+on weights far from 1 (their split-fp16 parts are scaled per matrix), against the fp64 oracle.
+
+Tolerance (relative 2-norm): a split-fp16 product is off by at most 3 * 2^-22 = 7e-7 of itself, with random signs;
+GELU by 3.3e-7 absolute.  Through the three layers of a tail: 3 (7e-7 + 3.3e-7) = 3e-6 at most; fp32 rounding of the
+sums adds 1e-7 each."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import converse_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+TOL = 3e-6
+
+
+def _t(a):
+    """On the device, one float past a 16-byte boundary."""
+    a = np.ascontiguousarray(a)
+    buf = torch.empty(a.size + 1, device=DEV)
+    v = buf[1:].view(a.shape)
+    v.copy_(torch.from_numpy(a))
+    return v
+
+
+def _close(got, ref, what):
+    got = got.cpu().numpy()
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= TOL, (what, err)
+
+
+def _params(C, mid, seed, ws=1.0):
+    r = np.random.default_rng(seed)
+    f = lambda *s: r.standard_normal(s).astype(np.float32)  # noqa: E731
+    return dict(lw=1 + 0.1 * f(C), lb=0.1 * f(C), w1=ws * f(mid, C, 1, 1) / np.float32(np.sqrt(C)), b1=f(mid),
+                w2=f(C, mid, 1, 1) / np.float32(np.sqrt(mid) * ws), b2=f(C), w0=f(C, mid, 1, 1) / np.float32(np.sqrt(mid)),
+                b0=f(C), a1=f(C), a2=f(C))
+
+
+def _branch(y, p):
+    return O.conv1x1(O.gelu(O.conv1x1(O.layernorm_cf(y, p["lw"], p["lb"], 1e-5), p["w1"], p["b1"])), p["w2"], p["b2"])
+
+
+# pixel counts around one 16-pixel tile, one 256-pixel block and several blocks
+SIZES = [(1, 1), (3, 5), (1, 17), (15, 17), (7, 37), (33, 65)]
+
+
+@pytest.mark.parametrize("H,W", SIZES)
+@pytest.mark.parametrize("head", [False, True])
+def test_tail(H, W, head):
+    from conversenet_amd import functional as Fh
+
+    p = _params(64, 128, H * W)
+    r = np.random.default_rng(W)
+    t = r.standard_normal((2, 128, H, W)).astype(np.float32)
+    x = r.standard_normal((2, 64, H, W)).astype(np.float32)
+    s = lambda v: v[None, :, None, None]  # noqa: E731
+    y1 = x + s(p["a1"]) * O.conv1x1(O.gelu(t), p["w0"], p["b0"])
+    ref = y1 + s(p["a2"]) * _branch(y1, p)
+    d = {k: _t(v) for k, v in p.items()}
+    out = Fh.conv_ln_mlp_residual(_t(t), _t(x), d["w0"], d["b0"], d["lw"], d["lb"], 1e-5, d["w1"], d["b1"], d["w2"],
+                                  d["b2"], d["a1"], d["a2"], t_act="gelu",
+                                  head=(d["lw"], d["lb"], 1e-5, d["w1"], d["b1"]) if head else None)
+    _close(out[0] if head else out, ref, "tail")
+    if head:
+        _close(out[1], O.gelu(O.conv1x1(O.layernorm_cf(ref, p["lw"], p["lb"], 1e-5), p["w1"], p["b1"])), "head")
+
+
+@pytest.mark.parametrize("H,W", SIZES)
+@pytest.mark.parametrize("C,mid", [(64, 128), (32, 64)])
+def test_ln_conv_and_mlp(H, W, C, mid):
+    from conversenet_amd import functional as Fh
+
+    p = _params(C, mid, H + W)
+    x = np.random.default_rng(H).standard_normal((2, C, H, W)).astype(np.float32)
+    d = {k: _t(v) for k, v in p.items()}
+    got = Fh.conv1x1(_t(x), d["w1"], d["b1"], act="gelu", ln=(d["lw"], d["lb"], 1e-5))
+    _close(got, O.gelu(O.conv1x1(O.layernorm_cf(x, p["lw"], p["lb"], 1e-5), p["w1"], p["b1"])), "ln conv")
+    got = Fh.ln_mlp_residual(_t(x), d["lw"], d["lb"], 1e-5, d["w1"], d["b1"], d["w2"], d["b2"], d["a2"])
+    _close(got, x + p["a2"][None, :, None, None] * _branch(x, p), "mlp")
+
+
+@pytest.mark.parametrize("ws", [1e-30, 1e-6, 300.0, 1e6])
+def test_weight_scale(ws):
+    """Weights whose fp16 parts would vanish or overflow without the per-matrix scale (1x1, no bias)."""
+    from conversenet_amd import functional as Fh
+
+    r = np.random.default_rng(3)
+    x = r.standard_normal((1, 64, 9, 11)).astype(np.float32)
+    w = (ws * r.standard_normal((128, 64, 1, 1)) / 8).astype(np.float32)
+    _close(Fh.conv1x1(_t(x), _t(w)), O.conv1x1(x, w, np.zeros(128, np.float32)), ws)
+    z = Fh.conv1x1(_t(x), _t(0 * w))
+    assert not z.cpu().numpy().any()
+
+
+@pytest.mark.parametrize("mode,k,pad", [("circular", 7, 6), ("replicate", 5, 4)])
+def test_block_and_chain_on_odd_images(mode, k, pad):
+    """A block and a chain of blocks on 45 x 41 pixels (padded planes 57 x 53 and 53 x 49)."""
+    from conversenet_amd.util_converse import ConverseBlock, run_blocks
+
+    torch.manual_seed(1)
+    blks = [ConverseBlock(64, 64, kernel_size=k, padding=pad, padding_mode=mode).to(DEV).eval() for _ in range(3)]
+    x = np.random.default_rng(2).standard_normal((2, 64, 45, 41)).astype(np.float32)
+    ref = x
+    for b in blks:
+        sd = {n: v.detach().cpu().numpy() for n, v in b.state_dict().items()}
+        ref = O.converse_block(ref, sd, "", k, 1, pad, mode, 1e-5, False)
+    with torch.no_grad():
+        _close(run_blocks(blks, _t(x)), ref, "chain")
+        y = _t(x)
+        for b in blks:
+            y = b(y)
+    _close(y, ref, "blocks")

@@ -2280,6 +2280,12 @@ extern "C" int cvn_converse2d_op_apply_f32(const float* x, const float* x0, int6
   if ((rc = launch_rows_fwd(x0, g.P, g.Hs, g.Ws, 0, CVN_PAD_ZEROS, g.Hs, g.Ws, tabs + L.t.off[kTabWs], S0, st)) !=
       CVN_OK)
     return rc;
+  if (lines_cols_op_ok(g.P, g.h, g.Hs, g.s, g.w)) {
+    rc = launch_lines_cols_op(S, S0, kf, Am, SH, g.B, g.C, g.h, g.w, g.s, (const float2*)(tabs + L.t.off[kTabH]),
+                              (const float2*)(tabs + L.t.off[kTabHs]), st);
+    if (rc != CVN_OK) return rc;
+    return launch_rows_inv(SH, g, 0, g.Hs, 0, g.Ws, CVN_ACT_NONE, tabs + L.t.off[kTabWs], out, st);
+  }
   ColOpArgs ca;
   ca.S = S; ca.S0 = S0; ca.kf = kf; ca.A = Am; ca.SH = SH; ca.C = g.C;
   ca.h = g.h; ca.w = g.w; ca.s = g.s; ca.Hs = g.Hs; ca.Ws = g.Ws; ca.NC = g.NC; ca.NCs = g.NCs;
@@ -2368,7 +2374,14 @@ extern "C" int cvn_converse2d_bwd_f32(const float* grad_out, const float* x, int
                 CVN_OK)
     return rc;
   // column pass: dS (in place over Sx) and dPhi
-  {
+  // (132, 256 and 260 points at scale 1 keep the compile-time kernel, whose dPhi sums stay in registers
+  // through its smaller transforms: 340 us against 690 at cfg3)
+  const bool ct = g.s == 1 && (g.h == 132 || g.h == 256 || g.h == 260);
+  if (!ct && lines_cols_bwd_ok(g.P, g.h, g.Hs, g.s, g.NC)) {
+    rc = launch_lines_cols_bwd(Sg, Sx, phi, wg ? (float2*)(base + ws.dphi) : nullptr, g.B, g.C, g.Cp / g.C, g.h, g.w,
+                               g.s, (const float2*)(tabs + t.off[kTabH]), (const float2*)(tabs + t.off[kTabHs]), st);
+    if (rc != CVN_OK) return rc;
+  } else {
     ColBwdArgs a;
     a.Sg = Sg; a.Sx = Sx; a.phi = phi; a.dphi = wg ? (float2*)(base + ws.dphi) : nullptr;
     a.B = g.B; a.C = g.C; a.psf_batch = g.Cp / g.C;

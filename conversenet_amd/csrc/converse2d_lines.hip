@@ -10,7 +10,9 @@
 // byte of plane and pass), overlapped by the 2 to 16 blocks of a CU with two or three LDS passes.  Measured
 // (one layer, us, runtime-plan passes -> these): 128 planes 333 x 493: 679 -> 210 (rows 214 -> 58, columns
 // 282 -> 90, inverse rows 214 -> 58); 512 planes 136 x 136: 282 -> 90; 256 planes 499 x 509 (primes):
-// 1283 ms -> 1.7 ms; the backward's 1024 x 260 rows of 260, compile-time plan before: 172 -> 127.
+// 1283 ms -> 1.7 ms; the backward's 1024 x 260 rows of 260, compile-time plan before: 172 -> 127; the
+// backward's column pass at 1024 planes 108 x 108: 240 -> 127; the operator's 192 planes 63 x 88 at scale 3:
+// 336 -> 176 (whole call).
 #include <algorithm>
 
 #include "cvn_common.h"
@@ -334,11 +336,300 @@ __global__ void __launch_bounds__(kLineThreads) k_lines_rows_inv(RowsInvArgs) {
   }
 }
 
+// ------------------------------------------------------------------------------------------------
+// Backward column pass (see k_cols_bwd): 16 LR column classes v0 per block, numbered through the psf
+// groups; the block loops over the planes that share a psf.  Per plane: Y (LR columns of pad x) and, member
+// by member, dZ (HR columns v0 + b w of the output gradient's rows) are transformed; dY = alias sum of
+// conj(Phi') dZ goes back through the inverse LR transform to dS, in place over Sx; dPhi += conj(Y) dZ.
+// dPhi is summed in global memory: every entry belongs to one thread, which adds its planes in order (no
+// atomics, the same bits each time), and the block's 16 columns stay in L2; in registers the sums would
+// have to live across the transforms, in LDS they would halve the blocks per CU.
+// ------------------------------------------------------------------------------------------------
+struct ColsBwdArgs {
+  const float2* Sg;   // (P, NCs, Hs)
+  float2* Sx;         // (P, NC, h): in (dphi != null) and out
+  const float2* phi;  // (Cp, NCs, Hs)
+  float2* dphi;       // (Cp, Ws, Hs) or null
+  const float2 *tw_h, *tw_H;
+  int nplanes, C;     // planes per psf: B (shared psf) or 1
+  int w, s, Hs, Ws, NC, NCs, total, nblk;
+  LinePlan ph, pH;
+};
+
+template <bool ONE>  // ONE: scale 1 (dY in place of dZ)
+__global__ void __launch_bounds__(kLineThreads) k_lines_cols_bwd(ColsBwdArgs) {
+  const CVN_KARG ColsBwdArgs& a = *(const CVN_KARG ColsBwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int NB = kLines, LD = kLineLd;
+  const int tid = threadIdx.x, nth = blockDim.x, h = a.ph.L, Hs = ONE ? h : a.Hs;
+  const bool wg = a.dphi != nullptr;
+  const size_t nh = ((size_t)h * LD * sizeof(float2) + 15) / 16 * 16;
+  float2* Y = (float2*)smem;             // LR lines of pad x
+  float2* X = (float2*)(smem + nh);      // HR lines of one member
+  char* p = smem + nh + ((size_t)Hs * LD * sizeof(float2) + 15) / 16 * 16;
+  float2* D = ONE ? X : (float2*)p;      // dY
+  if (!ONE) p += nh;
+  // per line, for the current plane and member: offsets in Sx, Sg and Phi' (complemented: the mirrored
+  // column, conjugated) and dPhi
+  int64_t* xo = (int64_t*)p;
+  int64_t *go = xo + NB, *fo = go + NB, *po = fo + NB;
+  float2* twh = (float2*)(po + NB);
+  float2* twH = ONE ? twh : twh + a.ph.T;
+  unsigned short* ih = (unsigned short*)(twH + (ONE ? a.ph.T : a.pH.T));
+  unsigned short* iH = ONE ? ih : ih + h;
+  const int g0 = line_item(blockIdx.x, a.nblk) * NB;
+  const int nb = min(NB, a.total - g0);
+  line_tables(a.ph, a.tw_h, ih, twh, tid, nth);
+  if (!ONE) line_tables(a.pH, a.tw_H, iH, twH, tid, nth);
+  const int members = ONE ? 1 : a.s;
+  for (int ib = 0; ib < a.nplanes; ++ib) {
+    for (int b = 0; b < members; ++b) {
+      // the index arithmetic of each phase is formed again per plane: hoisted out of the loop, it would be
+      // held (spilled) across the transforms
+      int tl = tid;
+      asm volatile("" : "+v"(tl));
+      const int nih = h * (NB / 4), niH = Hs * (NB / 4);  // items of 4 lines at one row, rows fastest
+      const uint32_t mgh = a.ph.mgL, mgH = ONE ? mgh : a.pH.mgL;
+      __syncthreads();  // the previous member's product and the previous plane's stores have read theirs
+      if (tl < NB) {
+        const int gc = min(g0 + tl, a.total - 1), grp = gc / a.NC, col = gc - grp * a.NC, vb = col + b * a.w;
+        const int64_t plane = (int64_t)ib * a.C + grp;
+        const bool mir = !ONE && vb > a.Ws / 2;  // a real row's spectrum is Hermitian in the column
+        const int vm = mir ? a.Ws - vb : vb;
+        const int64_t g = (plane * a.NCs + vm) * Hs, f = ((int64_t)grp * a.NCs + vm) * Hs;
+        xo[tl] = (plane * a.NC + col) * h;
+        go[tl] = mir ? ~g : g;
+        fo[tl] = mir ? ~f : f;
+        po[tl] = ((int64_t)grp * a.Ws + vb) * Hs;
+      }
+      __syncthreads();
+      if (wg && b == 0)
+        for (int idx = tl; idx < nih; idx += nth) {
+          const int q = mg_div(idx, mgh, h), u = idx - q * h;
+          float2 v[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = a.Sx[xo[4 * q + j] + u];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) Y[u * LD + 4 * q + j] = v[j];
+        }
+      for (int idx = tl; idx < niH; idx += nth) {
+        const int q = mg_div(idx, mgH, Hs), u = idx - q * Hs;
+        float2 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int64_t o = go[4 * q + j];
+          v[j] = a.Sg[(!ONE && o < 0 ? ~o : o) + u];
+          if (!ONE && o < 0) v[j].y = -v[j].y;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) X[u * LD + 4 * q + j] = v[j];
+      }
+      __syncthreads();
+      for (int t = wg && b == 0 ? 0 : 1; t < 2; ++t) {
+        const CVN_KARG LinePlan* pl = (ONE || t == 0) ? &a.ph : &a.pH;
+        line_fft<true>(*pl, (char*)(t ? X : Y), t ? twH : twh, tl, nth);
+      }
+      // dY (+)= sum over the member's rows of a class of conj(Phi') dZ, real and imaginary parts exchanged
+      // for the inverse transform; dPhi (+)= conj(Y) dZ / (Hs Ws).  Items of 2 lines at one LR row.
+      const float norm = 1.0f / ((float)Hs * (float)a.Ws);
+      int tp = tid;
+      asm volatile("" : "+v"(tp));
+      for (int idx = tp; idx < 2 * nih; idx += nth) {
+        const int q = mg_div(idx, mgh, h), u0 = idx - q * h;
+        const int py = ih[u0] * LD + 2 * q;
+        float2 m[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) m[j] = make_float2(0.f, 0.f);
+        for (int e = 0; e < members; ++e) {
+          const int u = ONE ? u0 : u0 + e * h;
+          const float2* xz = X + iH[u] * LD + 2 * q;
+          float2 f[2], d[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int64_t o = fo[2 * q + j];
+            f[j] = !ONE && o < 0 ? a.phi[~o + (u ? Hs - u : 0)] : a.phi[o + u];
+            if (!ONE && o < 0) f[j].y = -f[j].y;
+            d[j] = make_float2(0.f, 0.f);
+            if (wg && ib > 0) d[j] = a.dphi[po[2 * q + j] + u];
+          }
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const float2 z = xz[j];
+            const float2 t = cmul(cconj(f[j]), z);
+            m[j].x += t.x;
+            m[j].y += t.y;
+            if (wg && 2 * q + j < nb) {
+              const float2 g = cmul(cconj(Y[py + j]), z);
+              a.dphi[po[2 * q + j] + u] = make_float2(fmaf(g.x, norm, d[j].x), fmaf(g.y, norm, d[j].y));
+            }
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          float2 t = make_float2(m[j].y, m[j].x);
+          if (!ONE && b > 0) {
+            const float2 o = D[py + j];
+            t.x += o.x;
+            t.y += o.y;
+          }
+          D[py + j] = t;
+        }
+      }
+    }
+    __syncthreads();
+    int ts = tid;
+    asm volatile("" : "+v"(ts));
+    line_fft<false>(a.ph, (char*)D, twh, ts, nth);
+    for (int idx = ts; idx < h * (NB / 4); idx += nth) {
+      const int q = mg_div(idx, a.ph.mgL, h), u = idx - q * h;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * q + j < nb) {
+          const float2 t = D[u * LD + 4 * q + j];
+          a.Sx[xo[4 * q + j] + u] = make_float2(t.y, t.x);
+        }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Operator column pass (arbitrary x0, see k_cols_op): 16 alias classes v0 in [0, w / 2] per block with all
+// their members v0 + b w in LDS.  Rows are real, so column Ws - v of a row spectrum is the conjugate of
+// column v: the members past Ws / 2 are read from, and written to, the mirrored stored columns, which
+// covers the classes above w / 2 too (half the column transforms of one block per class).
+// ------------------------------------------------------------------------------------------------
+struct ColsOpArgs {
+  const float2* S;   // (P, NC, h)    row spectra of y
+  const float2* S0;  // (P, NCs, Hs)  row spectra of x0
+  const float2* kf;  // (C, Ws, Hs)
+  const float2* A;   // (C, Ws, Hs)   conj(K) / D / (Hs Ws)
+  float2* SH;        // (P, NCs, Hs)
+  const float2 *tw_h, *tw_H;
+  int B, C, w, s, Hs, Ws, NC, NCs, total, nblk;
+  LinePlan ph, pH;
+};
+constexpr int64_t kNoCol = INT64_MIN;
+
+__global__ void __launch_bounds__(kLineThreads) k_lines_cols_op(ColsOpArgs) {
+  const CVN_KARG ColsOpArgs& a = *(const CVN_KARG ColsOpArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int NB = kLines, LD = kLineLd;
+  const int tid = threadIdx.x, nth = blockDim.x, h = a.ph.L, Hs = a.Hs;
+  const size_t nh = ((size_t)h * LD * sizeof(float2) + 15) / 16 * 16;
+  const size_t nH = ((size_t)Hs * LD * sizeof(float2) + 15) / 16 * 16;
+  float2* Y = (float2*)smem;
+  char* X = smem + nh;  // member b at X + b nH
+  // per line: offset in S; per member and line: offsets in S0 (complemented: mirrored and conjugated), the
+  // tables, and SH (complemented: conjugated; kNoCol: a member whose mirror is another member, which stores it)
+  int64_t* yo = (int64_t*)(X + a.s * nH);
+  int64_t *xo = yo + NB, *ko = xo + a.s * NB, *oo = ko + a.s * NB;
+  float2* twh = (float2*)(oo + a.s * NB);
+  float2* twH = twh + a.ph.T;
+  unsigned short* ih = (unsigned short*)(twH + a.pH.T);
+  unsigned short* iH = ih + h;
+  const int g0 = line_item(blockIdx.x, a.nblk) * NB;
+  const int nb = min(NB, a.total - g0);
+  for (int i = tid; i < a.s * NB; i += nth) {
+    const int b = i / NB, gc = min(g0 + i - b * NB, a.total - 1);
+    const int q = gc / a.NC, v0 = gc - q * a.NC, c = q / a.B;  // planes of a channel follow each other
+    const int64_t plane = (int64_t)(q - c * a.B) * a.C + c;
+    const int vb = v0 + b * a.w;
+    const bool mir = vb > a.Ws / 2;
+    const int64_t o = (plane * a.NCs + (mir ? a.Ws - vb : vb)) * Hs;
+    if (b == 0) yo[i] = (plane * a.NC + v0) * h;
+    xo[i] = mir ? ~o : o;
+    ko[i] = ((int64_t)c * a.Ws + vb) * Hs;
+    oo[i] = !mir ? o : (v0 == 0 || 2 * v0 == a.w) ? kNoCol : ~o;
+  }
+  line_tables(a.ph, a.tw_h, ih, twh, tid, nth);
+  line_tables(a.pH, a.tw_H, iH, twH, tid, nth);
+  __syncthreads();
+  const int nih = h * (NB / 4), niH = Hs * (NB / 4);  // items of 4 lines at one row, rows fastest
+  for (int idx = tid; idx < nih; idx += nth) {
+    const int q = mg_div(idx, a.ph.mgL, h), u = idx - q * h;
+    float2 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = a.S[yo[4 * q + j] + u];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) Y[u * LD + 4 * q + j] = v[j];
+  }
+  for (int b = 0; b < a.s; ++b)
+    for (int idx = tid; idx < niH; idx += nth) {
+      const int q = mg_div(idx, a.pH.mgL, Hs), u = idx - q * Hs;
+      float2 v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t o = xo[b * NB + 4 * q + j];
+        v[j] = a.S0[(o < 0 ? ~o : o) + u];
+        if (o < 0) v[j].y = -v[j].y;
+      }
+      float2* d = (float2*)(X + b * nH) + u * LD + 4 * q;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[j] = v[j];
+    }
+  __syncthreads();
+  for (int t = 0; t <= a.s; ++t) {
+    const CVN_KARG LinePlan* pl = t == 0 ? &a.ph : &a.pH;
+    line_fft<true>(*pl, t == 0 ? (char*)Y : X + (t - 1) * nH, t == 0 ? twh : twH, tid, nth);
+  }
+  // X = X0 + A (Y - mean(K X0)) of every class, real and imaginary parts exchanged for the inverse
+  {
+    int ts = tid;
+    asm volatile("" : "+v"(ts));  // (its index arithmetic is not to be held across the transforms)
+    const float inv_s2 = 1.0f / (float)(a.s * a.s), norm = 1.0f / ((float)Hs * (float)a.Ws);
+    for (int idx = ts; idx < 2 * nih; idx += nth) {
+      const int q = mg_div(idx, a.ph.mgL, h), u0 = idx - q * h;
+      float2 m[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+      for (int b = 0; b < a.s; ++b)
+        for (int e = 0; e < a.s; ++e) {
+          const int u = u0 + e * h;
+          const float2* x = (const float2*)(X + b * nH) + iH[u] * LD + 2 * q;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const float2 t = cmul(a.kf[ko[b * NB + 2 * q + j] + u], x[j]);
+            m[j].x += t.x;
+            m[j].y += t.y;
+          }
+        }
+      const float2* y = Y + ih[u0] * LD + 2 * q;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) m[j] = make_float2(y[j].x - m[j].x * inv_s2, y[j].y - m[j].y * inv_s2);
+      for (int b = 0; b < a.s; ++b)
+        for (int e = 0; e < a.s; ++e) {
+          const int u = u0 + e * h;
+          float2* x = (float2*)(X + b * nH) + iH[u] * LD + 2 * q;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const float2 t = cmul(a.A[ko[b * NB + 2 * q + j] + u], m[j]), x0 = x[j];
+            x[j] = make_float2(fmaf(x0.y, norm, t.y), fmaf(x0.x, norm, t.x));
+          }
+        }
+    }
+  }
+  __syncthreads();
+  for (int b = 0; b < a.s; ++b) line_fft<false>(a.pH, X + b * nH, twH, tid, nth);
+  int ts = tid;
+  asm volatile("" : "+v"(ts));
+  for (int b = 0; b < a.s; ++b)
+    for (int idx = ts; idx < niH; idx += nth) {
+      const int q = mg_div(idx, a.pH.mgL, Hs), u = idx - q * Hs;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t o = oo[b * NB + 4 * q + j];
+        if (4 * q + j < nb && o != kNoCol) {
+          const float2 t = ((const float2*)(X + b * nH))[u * LD + 4 * q + j];
+          a.SH[(o < 0 ? ~o : o) + u] = make_float2(t.y, o < 0 ? -t.x : t.x);
+        }
+      }
+    }
+}
+
 std::atomic<uint64_t> g_line_attr{0};
 void line_attrs() {
   once_per_device(g_line_attr, [] {
     for (const void* k : {(const void*)k_lines_rows_fwd, (const void*)k_lines_rows_inv, (const void*)k_lines_cols<true>,
-                          (const void*)k_lines_cols<false>})
+                          (const void*)k_lines_cols<false>, (const void*)k_lines_cols_bwd<true>,
+                          (const void*)k_lines_cols_bwd<false>, (const void*)k_lines_cols_op})
       (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLineLds);
     (void)hipGetLastError();
   });
@@ -349,10 +640,13 @@ void line_attrs() {
 // elements per thread) is the fastest or within 6 % of it, and an uneven share of the 16 waves (3, 5) up to
 // 30 % slower.  Where the blocks are too few to fill the chip, waves are doubled while all blocks stay
 // resident and the widest pass still gives every wave a butterfly per lane (64 planes of 136 x 136: 37 -> 28 us).
-int line_threads(const LinePlan& p, int nblk) {
+// lds: the block's LDS, where it holds more than one line buffer (fewer blocks per CU, more waves each).
+int line_threads(const LinePlan& p, int nblk, size_t lds = 0) {
   int w = 1, most = 1;
   while (w < 16 && w * 64 * 1.41421 < p.L) w *= 2;
   for (int t = 0; t < p.np; ++t) most = std::max(most, p.ps[t].nl * kLines);
+  if (lds) most = std::max(most, p.L * 8);  // the product's items
+  while (lds && 2 * w * (int)(kLineLds / lds) <= 16 && 64 * w < most) w *= 2;
   while (2 * w <= 16 && (int64_t)nblk * 2 * w <= 256 * 16 && 64 * w < most) w *= 2;
   return std::max(64 * w, line_min_threads(p));
 }
@@ -406,6 +700,73 @@ int launch_lines_cols(const float2* S, const float2* phi, float2* SH, int64_t B,
   if (one) hipLaunchKernelGGL(k_lines_cols<true>, grid, block, lds, st, a);
   else hipLaunchKernelGGL(k_lines_cols<false>, grid, block, lds, st, a);
   return check_launch("column pass");
+}
+
+namespace {
+size_t cols_bwd_lines_lds(int h, int Hs, int s) {
+  size_t n = 2 * line_buf_bytes(h) + line_tab_bytes(*line_plan(h)) + 4 * kLines * sizeof(int64_t);
+  if (s > 1) n += line_buf_bytes(Hs) + line_tab_bytes(*line_plan(Hs));
+  return n;
+}
+}  // namespace
+
+bool lines_cols_bwd_ok(int64_t P, int h, int Hs, int s, int NC) {
+  return Hs <= kLineMax && P * NC < (1 << 30) && cols_bwd_lines_lds(h, Hs, s) <= kLineLds;
+}
+
+int launch_lines_cols_bwd(const float2* Sg, float2* Sx, const float2* phi, float2* dphi, int64_t B, int64_t C,
+                          int64_t psf_batch, int h, int w, int s, const float2* tw_h, const float2* tw_H, hipStream_t st) {
+  ColsBwdArgs a;
+  const LinePlan *lh = line_plan(h), *lH = line_plan(h * s);
+  if (!lh || !lH) return fail(CVN_ERR_UNSUPPORTED, "no plan for column length");
+  a.ph = *lh;
+  a.pH = *lH;
+  line_attrs();
+  a.Sg = Sg; a.Sx = Sx; a.phi = phi; a.dphi = dphi; a.tw_h = tw_h; a.tw_H = tw_H;
+  a.nplanes = psf_batch == 1 ? (int)B : 1;
+  a.C = (int)C;
+  a.w = w; a.s = s; a.Hs = h * s; a.Ws = w * s; a.NC = w / 2 + 1; a.NCs = w * s / 2 + 1;
+  a.total = (int)(psf_batch == 1 ? C : B * C) * a.NC;
+  a.nblk = (a.total + kLines - 1) / kLines;
+  const size_t lds = cols_bwd_lines_lds(h, h * s, s);
+  const dim3 grid((unsigned)a.nblk), block(std::max(line_threads(a.ph, a.nblk, lds), line_threads(a.pH, a.nblk, lds)));
+  if (s == 1) hipLaunchKernelGGL(k_lines_cols_bwd<true>, grid, block, lds, st, a);
+  else hipLaunchKernelGGL(k_lines_cols_bwd<false>, grid, block, lds, st, a);
+  return check_launch("backward column pass");
+}
+
+namespace {
+size_t cols_op_lines_lds(int h, int Hs, int s) {
+  return line_buf_bytes(h) + s * line_buf_bytes(Hs) + line_tab_bytes(*line_plan(h)) + line_tab_bytes(*line_plan(Hs)) +
+         (1 + 3 * (size_t)s) * kLines * sizeof(int64_t);
+}
+}  // namespace
+
+// A block runs s + 1 transforms and s^2 bins per class one after another, k_cols_op one block per class: with
+// few blocks that one is faster (us, this / that: 36 blocks at s = 4 50 / 40, 24 at s = 3 52 / 47, 36 and 42 at
+// s = 2 40 / 38 and 36 / 42, 33 at s = 1 37 / 44; 104 at s = 3 45 / 65, 216 at s = 4 57 / 104).
+bool lines_cols_op_ok(int64_t P, int h, int Hs, int s, int w) {
+  if (P * (w / 2 + 1) < (int64_t)kLines * 20 * s) return false;
+  return Hs <= kLineMax && P * (w / 2 + 1) < (1 << 30) && cols_op_lines_lds(h, Hs, s) <= kLineLds;
+}
+
+int launch_lines_cols_op(const float2* S, const float2* S0, const float2* kf, const float2* A, float2* SH, int64_t B,
+                         int64_t C, int h, int w, int s, const float2* tw_h, const float2* tw_H, hipStream_t st) {
+  ColsOpArgs a;
+  const LinePlan *lh = line_plan(h), *lH = line_plan(h * s);
+  if (!lh || !lH) return fail(CVN_ERR_UNSUPPORTED, "no plan for column length");
+  a.ph = *lh;
+  a.pH = *lH;
+  line_attrs();
+  a.S = S; a.S0 = S0; a.kf = kf; a.A = A; a.SH = SH; a.tw_h = tw_h; a.tw_H = tw_H;
+  a.B = (int)B; a.C = (int)C;
+  a.w = w; a.s = s; a.Hs = h * s; a.Ws = w * s; a.NC = w / 2 + 1; a.NCs = w * s / 2 + 1;
+  a.total = (int)(B * C * a.NC);
+  a.nblk = (a.total + kLines - 1) / kLines;
+  const size_t lds = cols_op_lines_lds(h, h * s, s);
+  const dim3 block(std::max(line_threads(a.ph, a.nblk, lds), line_threads(a.pH, a.nblk, lds)));
+  hipLaunchKernelGGL(k_lines_cols_op, dim3((unsigned)a.nblk), block, lds, st, a);
+  return check_launch("op column pass");
 }
 
 int launch_lines_rows_inv(const float2* SH, int64_t P, int Hs, int Ws, int row0, int nrows, int col0, int ncols, int act,

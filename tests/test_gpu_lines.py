@@ -69,6 +69,56 @@ def test_shapes_modes_scales(B, C, H, W, k, s, p, mode, pb):
     _check(x, w, b, s, p, mode, (H, W, s, p))
 
 
+# (B, C, h, w, k, s): enough classes for the lines pass; even and odd w (self-mirrored classes 0 and w / 2),
+# dense and staged lengths, a length (500 rows at s = 2) whose members exceed LDS and stay on the class-per-block pass
+OP_CASES = [
+    (2, 40, 21, 37, 3, 1),
+    (3, 33, 15, 26, 3, 2),
+    (2, 30, 49, 17, 5, 3),
+    (2, 80, 10, 12, 7, 4),
+    (1, 97, 37, 31, 2, 2),
+    (2, 4, 250, 44, 3, 2),
+]
+
+
+@pytest.mark.parametrize("B,C,h,w,k,s", OP_CASES)
+def test_operator_arbitrary_x0(B, C, h, w, k, s):
+    from conversenet_amd import functional as Fh
+
+    x, psf, b = _inputs(B, C, h, w, k, h * w)
+    x0 = np.random.default_rng(w).standard_normal((B, C, h * s, w * s)).astype(np.float32)
+    ref = O.converse2d_op_stable(x, x0, psf, b, s, 1e-5)
+    got = Fh.converse2d_op(_t(x), _t(x0), _t(psf), _t(b), s, 1e-5, cache=False).cpu().numpy()
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= TOL, err
+
+
+# (B, C, H, W, k, s, p, mode, psf batch): several planes per psf and blocks that straddle psf groups
+BWD_CASES = [
+    (3, 5, 31, 29, 3, 1, 4, "circular", 1),     # 39 x 37
+    (2, 3, 33, 57, 5, 1, 2, "reflect", 2),      # 37 x 61
+    (4, 3, 94, 43, 3, 1, 3, "replicate", 1),    # 100 x 49
+    (3, 4, 15, 26, 3, 2, 1, "constant", 1),     # 34 x 56
+    (2, 3, 17, 13, 5, 3, 2, "circular", 2),     # 63 x 51
+    (3, 2, 10, 21, 2, 4, 1, "reflect", 1),      # 48 x 92
+]
+
+
+@pytest.mark.parametrize("B,C,H,W,k,s,p,mode,pb", BWD_CASES)
+@pytest.mark.parametrize("weights", [True, False])
+def test_backward(B, C, H, W, k, s, p, mode, pb, weights):
+    from conversenet_amd import functional as Fh
+
+    x, w, b = _inputs(B, C, H, W, k, H + W, pb)
+    go = np.random.default_rng(W).standard_normal((B, C, H * s, W * s)).astype(np.float32)
+    ref = O.converse2d_module_backward(x, w, b, go, s, p, mode, 1e-5)
+    got = Fh.converse2d_backward(_t(go), _t(x), _t(w), _t(b), s, p, mode, 1e-5, True, weights, weights)
+    for g, r in zip(got[:3 if weights else 1], ref):
+        r = np.asarray(r).reshape(g.shape)
+        # the weight gradients are sums over all bins in fp64 of products that are right to TOL
+        assert np.linalg.norm(g.cpu().numpy() - r) / np.linalg.norm(r) <= TOL
+
+
 def test_misaligned_scratch_and_infinite_plane():
     """Spectra scratch at 8 bytes past a 16-byte boundary (no 16-byte accesses), and a plane of infinities and
     NaN that shares its blocks with finite planes, which it must not touch."""

@@ -1772,7 +1772,9 @@ bool plan_tabs(const Geo& g, PlanTabs* t) {
   const int len[4] = {g.w, g.h, g.Hs, g.Ws};
   size_t o = 0;
   for (int i = 0; i < 4; ++i) {
-    if (!make_plan(len[i], &t->plan[i])) return false;
+    const FftPlan* p = fft_plan(len[i]);
+    if (!p) return false;
+    t->plan[i] = *p;
     t->off[i] = o;
     o += align_up(plan_tab_bytes(t->plan[i]), 256);
   }

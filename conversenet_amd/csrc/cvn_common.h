@@ -131,6 +131,23 @@ inline bool make_plan(int L, FftPlan* plan) {
   return true;
 }
 
+// make_plan of length L, made once per process; null outside 1 .. kMaxFftLen or without a plan.  (A call
+// asks for four lengths several times; factoring them costs as much host time as a kernel launch.)
+inline const FftPlan* fft_plan(int L) {
+  static std::atomic<const FftPlan*> memo[kMaxFftLen + 1] = {};
+  if (L < 1 || L > kMaxFftLen) return nullptr;
+  const FftPlan* p = memo[L].load(std::memory_order_acquire);
+  if (p) return p;
+  FftPlan* made = new FftPlan;
+  if (!make_plan(L, made)) {
+    delete made;
+    return nullptr;
+  }
+  if (memo[L].compare_exchange_strong(p, made, std::memory_order_acq_rel)) return made;
+  delete made;  // another thread was first
+  return p;
+}
+
 // Fused single-kernel path (converse2d_fused.hip): returns 1 and the workspace it needs when the
 // padded plane (H + 2 pad, W + 2 pad) at this scale has an instantiated plan (at scale > 1: when the
 // upsampled plane has one).

@@ -22,7 +22,9 @@ _ws_lock = threading.Lock()
 
 
 def _stream(dev):
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The current stream's handle.  (torch.cuda.current_stream builds a Stream object around it: 2 us, as much
+    host time as a kernel launch.)"""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def _need_hip(*ts):
@@ -38,7 +40,7 @@ def _need_hip(*ts):
 def _workspace(dev, nbytes: int, stream=None):
     """A reusable uint8 scratch tensor per (device, stream); grows monotonically.  stream: the current
     stream's handle when the caller has it already."""
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream if stream is None else stream)
+    key = (dev.index, _stream(dev) if stream is None else stream)
     with _ws_lock:
         buf = _ws_cache.get(key)
         if buf is None or buf.numel() < nbytes:
@@ -140,6 +142,7 @@ def _cache_key(kind, weight, bias, eps, geo, route, dev):
 
 
 _plan_memo: dict = {}
+_supported_memo: dict = {}  # the library's answers by geometry, as in _plan_memo
 _plan_lock = threading.Lock()
 
 
@@ -233,9 +236,17 @@ def supported(x, weight, scale, padding, grad_x=False, grad_weight=False, shape=
     if weight.dim() != 4 or (shape is None and x.dim() != 4):
         return False
     B, C, H, W = shape if shape is not None else x.shape
-    return lib.cvn_converse2d_supported(B, C, H, W, int(weight.shape[0]), int(weight.shape[2]),
-                                        int(weight.shape[3]), int(scale), int(padding), int(bool(grad_x)),
-                                        int(bool(grad_weight))) == _lib.CVN_OK
+    pb, _, kh, kw = weight.shape
+    key = (B, C, H, W, pb, kh, kw, int(scale), int(padding), bool(grad_x), bool(grad_weight),
+           os.environ.get("CVN_DISABLE_FUSED"))
+    ok = _supported_memo.get(key)
+    if ok is None:
+        ok = lib.cvn_converse2d_supported(*key[:9], int(key[9]), int(key[10])) == _lib.CVN_OK
+        with _plan_lock:
+            if len(_supported_memo) >= 1024:
+                _supported_memo.clear()
+            _supported_memo[key] = ok
+    return ok
 
 
 def op_supported(x, x0, weight, scale) -> bool:

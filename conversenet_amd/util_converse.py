@@ -188,7 +188,7 @@ class Converse2D(nn.Module):
         """act='gelu' applies exact GELU to the output (fused on store on the HIP path)."""
         if self._use_hip(x):
             self.biaseps = None  # read lazily from the current bias
-            return functional.converse2d_fused(x, self.weight, self.bias.reshape(-1), self.scale, self.padding,
+            return functional.converse2d_fused(x, self.weight, self.bias, self.scale, self.padding,
                                                self.padding_mode, self.eps, act)
         if self._use_hip_grad(x):
             self.biaseps = None
@@ -242,8 +242,7 @@ def _block_head(parts, x):
 def _block_converse(parts, t, act="gelu"):
     cv = parts[2]
     cv.biaseps = None  # read lazily from the current bias
-    return functional.converse2d_fused(t, cv.weight, cv.bias.reshape(-1), cv.scale, cv.padding, cv.padding_mode,
-                                       cv.eps, act=act)
+    return functional.converse2d_fused(t, cv.weight, cv.bias, cv.scale, cv.padding, cv.padding_mode, cv.eps, act=act)
 
 
 def _gelu_in_tail(parts, t_shape, x):

@@ -653,7 +653,7 @@ int line_threads(const LinePlan& p, int nblk, size_t lds = 0) {
 
 }  // namespace
 
-bool lines_rows_ok(int64_t P, int h, int w) { return w <= kLineMax && P * ((h + 1) / 2) < (1 << 30); }
+bool lines_rows_ok(int64_t P, int h, int w) { return line_plan(w) && P * ((h + 1) / 2) < (1 << 30); }
 
 int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, int mode, int h, int w,
                           const float2* tw, float2* S, hipStream_t st) {
@@ -674,7 +674,7 @@ int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, 
 }
 
 bool lines_cols_ok(int64_t P, int h, int Hs, int NCs) {
-  if (Hs > kLineMax || P * NCs >= (1 << 30)) return false;
+  if (!line_plan(h) || !line_plan(Hs) || P * NCs >= (1 << 30)) return false;
   if (Hs == h) return true;
   return line_buf_bytes(h) + line_buf_bytes(Hs) + line_tab_bytes(*line_plan(h)) + line_tab_bytes(*line_plan(Hs)) +
                  3 * kLines * sizeof(int64_t) <= kLineLds;
@@ -711,7 +711,7 @@ size_t cols_bwd_lines_lds(int h, int Hs, int s) {
 }  // namespace
 
 bool lines_cols_bwd_ok(int64_t P, int h, int Hs, int s, int NC) {
-  return Hs <= kLineMax && P * NC < (1 << 30) && cols_bwd_lines_lds(h, Hs, s) <= kLineLds;
+  return line_plan(h) && line_plan(Hs) && P * NC < (1 << 30) && cols_bwd_lines_lds(h, Hs, s) <= kLineLds;
 }
 
 int launch_lines_cols_bwd(const float2* Sg, float2* Sx, const float2* phi, float2* dphi, int64_t B, int64_t C,
@@ -747,7 +747,7 @@ size_t cols_op_lines_lds(int h, int Hs, int s) {
 // s = 2 40 / 38 and 36 / 42, 33 at s = 1 37 / 44; 104 at s = 3 45 / 65, 216 at s = 4 57 / 104).
 bool lines_cols_op_ok(int64_t P, int h, int Hs, int s, int w) {
   if (P * (w / 2 + 1) < (int64_t)kLines * 20 * s) return false;
-  return Hs <= kLineMax && P * (w / 2 + 1) < (1 << 30) && cols_op_lines_lds(h, Hs, s) <= kLineLds;
+  return line_plan(h) && line_plan(Hs) && P * (w / 2 + 1) < (1 << 30) && cols_op_lines_lds(h, Hs, s) <= kLineLds;
 }
 
 int launch_lines_cols_op(const float2* S, const float2* S0, const float2* kf, const float2* A, float2* SH, int64_t B,

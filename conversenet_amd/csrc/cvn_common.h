@@ -7,6 +7,7 @@
 #include <stdio.h>
 
 #include <atomic>
+#include <new>
 #include <string>
 
 #include "../../include/converse2d.h"
@@ -138,8 +139,8 @@ inline const FftPlan* fft_plan(int L) {
   if (L < 1 || L > kMaxFftLen) return nullptr;
   const FftPlan* p = memo[L].load(std::memory_order_acquire);
   if (p) return p;
-  FftPlan* made = new FftPlan;
-  if (!make_plan(L, made)) {
+  FftPlan* made = new (std::nothrow) FftPlan;
+  if (!made || !make_plan(L, made)) {
     delete made;
     return nullptr;
   }

@@ -613,10 +613,9 @@ __device__ __forceinline__ float2* fft_lds(const FftPlan& plan, float2* a, float
 
 // The fixed-radix decomposition of a compile-time length L: the odd radices first, largest first
 // (13, 11, 7, 5, 3), then 8s and 4 / 2 for the power of two; count 0 when L has another factor.
-// Measured on the 260-point passes of the backward (13, 5, 4 against 4, 5, 13): the column pass
-// 452 -> 398 us (LDS bank conflicts 2.0 -> 1.6 cycles per LDS instruction: the first pass writes
-// each butterfly's R outputs to R consecutive elements, which an odd R spreads over more banks),
-// the row passes 170 -> 167 and 172 -> 165 us (fewer instructions).
+// Measured on the 260-point column pass of the backward (13, 5, 4 against 4, 5, 13): 452 -> 398 us (LDS
+// bank conflicts 2.0 -> 1.6 cycles per LDS instruction: the first pass writes each butterfly's R
+// outputs to R consecutive elements, which an odd R spreads over more banks).
 struct FixedRadices {
   int n;
   int r[kMaxStages];

@@ -22,6 +22,7 @@
 // exchanged before and after, which the callers fold into their stores and loads.
 #pragma once
 #include <atomic>
+#include <new>
 
 #include "fft_device.h"
 
@@ -553,13 +554,14 @@ inline bool make_line_plan(int L, LinePlan* p) {
 }
 
 // The plan of length L, made once per process (at most kLineMax of them; the planner takes microseconds,
-// as much as a small launch); null outside 1 .. kLineMax.
+// as much as a small launch); null outside 1 .. kLineMax (and without memory).
 inline const LinePlan* line_plan(int L) {
   static std::atomic<const LinePlan*> memo[kLineMax + 1] = {};
   if (L < 1 || L > kLineMax) return nullptr;
   const LinePlan* p = memo[L].load(std::memory_order_acquire);
   if (p) return p;
-  LinePlan* made = new LinePlan;
+  LinePlan* made = new (std::nothrow) LinePlan;
+  if (!made) return nullptr;
   make_line_plan(L, made);
   if (memo[L].compare_exchange_strong(p, made, std::memory_order_acq_rel)) return made;
   delete made;  // another thread was first

@@ -58,8 +58,9 @@ class TableCache:
     """LRU cache of transfer tables, the counterpart of the reference's OTF cache (converse2d.cpp:52-102).
 
     Key: the psf and bias tensors (data pointer and version counter), eps, the geometry, the route
-    (which fixes the table's layout) and the device.  Entries hold strong references to psf and bias,
-    so a cached address cannot be reused by another tensor while the entry lives.  An in-place update
+    (which fixes the table's layout) and the device.  Entries hold the memory of psf and bias (detached
+    views: a parameter itself drops its memory when `.data` is assigned, as Module.to does, and keeps its
+    version), so a cached address cannot be reused by another tensor while the entry lives.  An in-place update
     (optimizer step, load_state_dict) bumps the version and misses; the entry of the older version is
     dropped then, so updates leave no dead tables behind.  Writes through `.data` (p.data.copy_(...),
     p.data.mul_(...)) do not bump the version counter: call torch.ops.converse2d.clear_cache() after such
@@ -102,6 +103,7 @@ class TableCache:
             del self.latest[stem]
 
     def put(self, key, table, refs):
+        refs = tuple(t.detach() for t in refs)
         with self._lock:
             old = self.latest.get(self._stem(key))
             if old is not None and old in self.entries:

@@ -42,6 +42,22 @@ def test_lru_bounds():
     assert c.bytes == 0 and not c.entries and not c.latest
 
 
+def test_entries_keep_the_memory_of_reassigned_parameters():
+    """p.data = t (Module.to, weight swaps) leaves the version as it is: an address that returned to the
+    allocator could come back with other values under the same key."""
+    c = Fh.TableCache()
+    w = torch.nn.Parameter(torch.ones(1, 4, 3, 3))
+    b = torch.nn.Parameter(torch.zeros(1, 4, 1, 1))
+    old = [(t.data_ptr(), t.detach().clone()) for t in (w, b)]
+    k = _key(w, b)
+    c.put(k, torch.empty(100, dtype=torch.uint8), (w, b))
+    for t in (w, b):
+        t.data = torch.full_like(t, 2.0)
+    held = {t.data_ptr(): t for t in c.entries[k][1]}
+    assert all(p in held and torch.equal(held[p], v) for p, v in old)
+    assert c.get(_key(w, b)) is None
+
+
 def test_cacheable_rules():
     w = torch.nn.Parameter(torch.ones(1, 4, 3, 3))
     b = torch.nn.Parameter(torch.zeros(1, 4, 1, 1))

@@ -131,8 +131,12 @@ __global__ void __launch_bounds__(kLineThreads) k_lines_rows_fwd(RowsFwdArgs) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Module column pass: forward LR column transform, times Phi, inverse HR column transform.
+// Module column pass: forward LR column transform, times Phi, inverse HR column transform.  Above scale 1
+// the LR bins pass through registers, so that one line buffer serves both transforms: 4 instead of 3 blocks per
+// CU at 132 -> 264 points (layer call, us, two buffers -> one: 256 planes 132 -> 264: 114 -> 97; 64 planes
+// 330 -> 990: 566 -> 372; 128 planes 16 -> 32, where the waves limit the blocks: 53 -> 54).
 // ------------------------------------------------------------------------------------------------
+constexpr int kUpRounds = 6;  // items of 2 lines per thread: 6 nth >= 8 h (launch_lines_cols)
 struct ColsArgs {
   const float2* S;    // (P, NC, h)
   const float2* phi;  // (Cp, NCs, Hs)
@@ -149,10 +153,8 @@ __global__ void __launch_bounds__(kLineThreads) k_lines_cols(ColsArgs) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int NB = kLines, LD = kLineLd;
   const int tid = threadIdx.x, nth = blockDim.x, h = a.ph.L, Hs = ONE ? h : a.Hs;
-  float2* X = (float2*)smem;  // the HR lines
+  float2* X = (float2*)smem;  // the LR lines, then the HR lines
   char* p = smem + ((size_t)Hs * LD * sizeof(float2) + 15) / 16 * 16;
-  float2* Y = ONE ? X : (float2*)p;  // the LR lines
-  if (!ONE) p += ((size_t)h * LD * sizeof(float2) + 15) / 16 * 16;
   int64_t* in = (int64_t*)p;  // per line: offset in S (complemented: the conjugate), in Phi, in SH
   int64_t *fi = in + NB, *oo = fi + NB;
   float2* twh = (float2*)(oo + NB);
@@ -191,23 +193,57 @@ __global__ void __launch_bounds__(kLineThreads) k_lines_cols(ColsArgs) {
     }
     if (i0 < nin) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) Y[u * LD + b0 + k] = v[k];
+      for (int k = 0; k < 8; ++k) X[u * LD + b0 + k] = v[k];
     }
   }
   __syncthreads();
-  line_fft<true>(a.ph, (char*)Y, twh, tid, nth);
-  for (int idx = tid; idx < nout; idx += nth) {
-    const int q = mg_div(idx, ONE ? a.ph.mgL : a.pH.mgL, Hs), u = idx - q * Hs, b0 = 8 * q;
-    float2 f[8];
+  line_fft<true>(a.ph, smem, twh, tid, nth);
+  if constexpr (ONE) {
+    for (int idx = tid; idx < nout; idx += nth) {
+      const int q = mg_div(idx, a.ph.mgL, h), u = idx - q * h, b0 = 8 * q;
+      float2 f[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) f[k] = a.phi[fi[b0 + k] + u];
-    const int us = ONE ? u : u - mg_div(u, a.ph.mgL, h) * h;
-    const float2* y = Y + ih[us] * LD + b0;
-    float2* x = X + iH[u] * LD + b0;
+      for (int k = 0; k < 8; ++k) f[k] = a.phi[fi[b0 + k] + u];
+      float2* x = X + ih[u] * LD + b0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const float2 t = cmul(y[k], f[k]);
-      x[k] = make_float2(t.y, t.x);
+      for (int k = 0; k < 8; ++k) {
+        const float2 t = cmul(x[k], f[k]);
+        x[k] = make_float2(t.y, t.x);
+      }
+    }
+  } else {
+    // each LR bin times Phi at its s aliases u + e h; items of 2 lines at one LR row, rows fastest
+    const int n = h * (NB / 2);
+    float2 y[kUpRounds][2];
+    int ul[kUpRounds], bl[kUpRounds];
+#pragma unroll
+    for (int r = 0; r < kUpRounds; ++r) {
+      if (r * nth >= n) break;
+      const int idx = min(tid + r * nth, n - 1), q = mg_div(idx, a.ph.mgL, h);
+      ul[r] = idx - q * h;
+      bl[r] = 2 * q;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) y[r][j] = X[ih[ul[r]] * LD + bl[r] + j];
+    }
+    __syncthreads();
+    for (int u0 = 0; u0 < Hs; u0 += h) {
+      float2 f[kUpRounds][2];
+#pragma unroll
+      for (int r = 0; r < kUpRounds; ++r) {
+        if (r * nth >= n) break;  // (a wave's last rounds may hold nothing)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) f[r][j] = a.phi[fi[bl[r] + j] + u0 + ul[r]];
+      }
+#pragma unroll
+      for (int r = 0; r < kUpRounds; ++r)
+        if (tid + r * nth < n) {
+          float2* x = X + iH[u0 + ul[r]] * LD + bl[r];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const float2 t = cmul(y[r][j], f[r][j]);
+            x[j] = make_float2(t.y, t.x);
+          }
+        }
     }
   }
   __syncthreads();
@@ -675,8 +711,7 @@ int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, 
 
 bool lines_cols_ok(int64_t P, int h, int Hs, int NCs) {
   if (!line_plan(h) || !line_plan(Hs) || P * NCs >= (1 << 30)) return false;
-  if (Hs == h) return true;
-  return line_buf_bytes(h) + line_buf_bytes(Hs) + line_tab_bytes(*line_plan(h)) + line_tab_bytes(*line_plan(Hs)) +
+  return line_buf_bytes(Hs) + line_tab_bytes(*line_plan(h)) + line_tab_bytes(*line_plan(Hs)) +
                  3 * kLines * sizeof(int64_t) <= kLineLds;
 }
 
@@ -694,9 +729,11 @@ int launch_lines_cols(const float2* S, const float2* phi, float2* SH, int64_t B,
   a.w = w; a.Hs = Hs; a.NC = w / 2 + 1; a.NCs = Ws / 2 + 1;
   a.total = (int)(B * C * a.NCs);
   size_t lds = line_buf_bytes(Hs) + line_tab_bytes(a.ph) + 3 * kLines * sizeof(int64_t);
-  if (!one) lds += line_buf_bytes(h) + line_tab_bytes(a.pH);
+  if (!one) lds += line_tab_bytes(a.pH);
   a.nblk = (a.total + kLines - 1) / kLines;
-  const dim3 grid((unsigned)a.nblk), block(std::max(line_threads(a.ph, a.nblk), line_threads(a.pH, a.nblk)));
+  int nth = std::max(line_threads(a.ph, a.nblk), line_threads(a.pH, a.nblk));
+  if (!one) nth = std::max(nth, ((kLines / 2 * h + kUpRounds - 1) / kUpRounds + 63) / 64 * 64);  // at most 704
+  const dim3 grid((unsigned)a.nblk), block(nth);
   if (one) hipLaunchKernelGGL(k_lines_cols<true>, grid, block, lds, st, a);
   else hipLaunchKernelGGL(k_lines_cols<false>, grid, block, lds, st, a);
   return check_launch("column pass");

@@ -58,8 +58,11 @@ CASES = [
     (1, 3, 15, 25, 3, 3, 1, "circular", 1),     # 51 x 81
     (2, 2, 12, 33, 5, 4, 2, "reflect", 2),      # 64 x 148
     (1, 2, 60, 41, 3, 2, 1, "constant", 1),     # 124 x 86
-    (2, 2, 130, 91, 3, 5, 2, "circular", 1),    # 670 x 475: two column buffers, scale above 4
-    (1, 1, 250, 1, 3, 4, 2, "replicate", 1),    # 1016 x 20: LR and HR columns exceed LDS together
+    (2, 2, 130, 91, 3, 5, 2, "circular", 1),    # 670 x 475: scale above 4
+    (1, 1, 250, 1, 3, 4, 2, "replicate", 1),    # 1016 x 20
+    (1, 2, 508, 3, 3, 2, 2, "circular", 1),     # 1024 x 14: the largest column buffer, most LR rows per thread
+    (2, 3, 3, 4, 3, 3, 0, "circular", 1),       # 9 x 12: LR rows fewer than a wave's items
+    (3, 2, 41, 6, 2, 2, 1, "reflect", 1),       # 86 x 16: 43 LR rows, items in an uneven last round
 ]
 
 

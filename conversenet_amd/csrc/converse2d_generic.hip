@@ -2379,7 +2379,7 @@ extern "C" int cvn_converse2d_bwd_f32(const float* grad_out, const float* x, int
   // (132, 256 and 260 points at scale 1 keep the compile-time kernel, whose dPhi sums stay in registers
   // through its smaller transforms: 340 us against 690 at cfg3)
   const bool ct = g.s == 1 && (g.h == 132 || g.h == 256 || g.h == 260);
-  if (!ct && lines_cols_bwd_ok(g.P, g.h, g.Hs, g.s, g.NC)) {
+  if (!ct && lines_cols_bwd_ok(g.P, g.Cp == g.C ? g.B : 1, g.h, g.Hs, g.s, g.NC)) {
     rc = launch_lines_cols_bwd(Sg, Sx, phi, wg ? (float2*)(base + ws.dphi) : nullptr, g.B, g.C, g.Cp / g.C, g.h, g.w,
                                g.s, (const float2*)(tabs + t.off[kTabH]), (const float2*)(tabs + t.off[kTabHs]), st);
     if (rc != CVN_OK) return rc;

@@ -747,7 +747,34 @@ size_t cols_bwd_lines_lds(int h, int Hs, int s) {
 }
 }  // namespace
 
-bool lines_cols_bwd_ok(int64_t P, int h, int Hs, int s, int NC) {
+namespace {
+// Whether k_cols_bwd (1 to 8 columns per block) is the faster one: with less than about a block per CU, the lines
+// pass is a serial chain over the planes of a psf beside idle CUs.  k_cols_bwd's plan must hold no prime above
+// 13 (34 rows, scale 1: 412 us against 205).  Whole backward, us, that / this, B planes per psf:
+//   scale > 1: 32 rows, 18 blocks, B 2 74 / 82, B 16 175 / 269; 128 rows, 98 blocks, B 16 313 / 363, 392 blocks, B 4
+//     265 / 213; 192 rows, 132 blocks, B 16 523 / 643; 400 rows, 42 blocks, B 4 163 / 185; 200 rows, 102 blocks, B 4
+//     184 / 177, 204 blocks, B 16 747 / 537; B 1 within 5 %.
+//   scale 1, where a block holds one column buffer less: only if the lines pass has a radix that leaves most of a
+//     block idle (24 rows in one radix, 34 blocks, B 4 77 / 81, B 16 150 / 180) or that one has two stages (64 rows, 98 blocks,
+//     B 16 200 / 210), or at few blocks of long columns (320 rows, 42 blocks, B 4 125 / 134); otherwise 36 rows, 38
+//     blocks, B 16 180 / 160; 120 rows, 62 blocks, B 16 235 / 217; 200 rows 282 / 288.
+bool few_bwd_blocks(int64_t nblk, int64_t nplanes, int h, int s) {
+  const FftPlan *p = fft_plan(h), *pH = fft_plan(h * s);
+  if (!p || !pH) return false;
+  for (const FftPlan* q : {p, pH})
+    for (int i = 0; i < q->nst; ++i)
+      if (q->radix[i] > 13) return false;
+  if (s > 1) return nblk < (h * s <= 192 ? 200 : 100) && nplanes > 1;
+  int narrow = h;  // butterflies of the widest radix
+  const LinePlan* lp = line_plan(h);
+  for (int t = 0; t < lp->np; ++t) narrow = std::min(narrow, lp->ps[t].nl);
+  return (nblk < 100 && nplanes >= 8 && (narrow < 4 || p->nst <= 2)) ||
+         (nblk < 50 && nplanes >= 4 && (narrow < 4 || h >= 256));
+}
+}  // namespace
+
+bool lines_cols_bwd_ok(int64_t P, int64_t nplanes, int h, int Hs, int s, int NC) {
+  if (line_plan(h) && few_bwd_blocks((P / nplanes * NC + kLines - 1) / kLines, nplanes, h, s)) return false;
   return line_plan(h) && line_plan(Hs) && P * NC < (1 << 30) && cols_bwd_lines_lds(h, Hs, s) <= kLineLds;
 }
 

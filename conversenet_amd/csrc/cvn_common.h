@@ -232,7 +232,7 @@ int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, 
 bool lines_cols_ok(int64_t P, int h, int Hs, int NCs);
 int launch_lines_cols(const float2* S, const float2* phi, float2* SH, int64_t B, int64_t C, int64_t psf_batch, int h,
                       int w, int Hs, int Ws, const float2* tw_h, const float2* tw_H, hipStream_t st);
-bool lines_cols_bwd_ok(int64_t P, int h, int Hs, int s, int NC);
+bool lines_cols_bwd_ok(int64_t P, int64_t nplanes, int h, int Hs, int s, int NC);
 int launch_lines_cols_bwd(const float2* Sg, float2* Sx, const float2* phi, float2* dphi, int64_t B, int64_t C,
                           int64_t psf_batch, int h, int w, int s, const float2* tw_h, const float2* tw_H, hipStream_t st);
 bool lines_cols_op_ok(int64_t P, int h, int Hs, int s, int w);

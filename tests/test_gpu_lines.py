@@ -104,6 +104,11 @@ BWD_CASES = [
     (3, 4, 15, 26, 3, 2, 1, "constant", 1),     # 34 x 56
     (2, 3, 17, 13, 5, 3, 2, "circular", 2),     # 63 x 51
     (3, 2, 10, 21, 2, 4, 1, "reflect", 1),      # 48 x 92
+    (1, 5, 16, 20, 3, 2, 0, "circular", 1),     # 32 x 40: one plane per psf, the lines pass
+    (2, 60, 14, 110, 3, 2, 0, "circular", 1),   # 28 x 220: blocks for most of the chip, the lines pass
+    (8, 3, 24, 10, 3, 1, 0, "circular", 1),     # 24 x 10: few blocks, a column class or more per block
+    (4, 2, 100, 9, 3, 3, 1, "replicate", 1),    # 306 x 33 (17 a factor): the lines pass at few blocks
+    (3, 3, 70, 9, 3, 3, 0, "constant", 1),      # 210 x 27: few blocks of long columns
 ]
 
 

@@ -57,7 +57,7 @@ def release_workspace():
 class TableCache:
     """LRU cache of transfer tables, the counterpart of the reference's OTF cache (converse2d.cpp:52-102).
 
-    Key: the psf and bias tensors (data pointer and version counter), eps, the geometry, the route
+    Key: the psf and bias tensors (data pointer, strides and version counter), eps, the geometry, the route
     (which fixes the table's layout) and the device.  Entries hold the memory of psf and bias (detached
     views: a parameter itself drops its memory when `.data` is assigned, as Module.to does, and keeps its
     version), so a cached address cannot be reused by another tensor while the entry lives.  An in-place update
@@ -139,8 +139,9 @@ def cacheable(weight, bias) -> bool:
 
 
 def _cache_key(kind, weight, bias, eps, geo, route, dev):
+    # with the strides: a transposed or expanded view starts at its base's address and shares its version
     return (kind, weight.data_ptr(), weight._version, bias.data_ptr(), bias._version, float(eps), geo, route,
-            dev.index)
+            dev.index, weight.stride(), bias.stride())
 
 
 _plan_memo: dict = {}

@@ -31,6 +31,19 @@ def test_route_and_geometry_are_part_of_the_key():
     assert len(c.entries) == 2 and c.bytes == 30
 
 
+def test_views_of_one_address_have_tables_of_their_own():
+    """A transposed square psf, and rows of one psf expanded, start at the address of the tensor they view."""
+    c = Fh.TableCache()
+    w, b = torch.rand(1, 4, 3, 3), torch.zeros(1, 4, 1, 1)
+    views = [(w, b), (w.transpose(2, 3), b), (w[:, :1].expand(1, 4, 3, 3), b), (w, b[:, :1].expand(1, 4, 1, 1))]
+    assert len({(v.data_ptr(), v._version, u.data_ptr(), u._version) for v, u in views}) == 1
+    for n, (v, u) in enumerate(views):
+        assert c.get(_key(v, u)) is None, n
+        c.put(_key(v, u), torch.full((10,), n, dtype=torch.uint8), (v, u))
+    for n, (v, u) in enumerate(views):
+        assert int(c.get(_key(v, u))[0]) == n
+
+
 def test_lru_bounds():
     c = Fh.TableCache(max_entries=3, max_bytes=250)
     ts = [(torch.ones(1, 1, 1, 1), torch.zeros(1, 1, 1, 1)) for _ in range(5)]

@@ -116,22 +116,35 @@ def _conv(m, x):
     return m(x)
 
 
+def _psf_stack(convs):
+    """The convolutions' weights and biases, each stacked along the output channels.  Kept in the transfer-table
+    cache while the parameters are unchanged (their memory is held there, and clear_cache drops it)."""
+    ws, bs = [m.weight for m in convs], [m.bias for m in convs]
+    ps = ws + bs
+    n, dev = sum(w.numel() for w in ws), ws[0].device
+    key = stack = None
+    if all(functional.cacheable(w, b) for w, b in zip(ws, bs)):
+        key = ("psf stack", tuple(t.data_ptr() for t in ps), tuple(t._version for t in ps), None, None, None,
+               tuple(t.shape for t in ps), None, dev.index, tuple(t.stride() for t in ps))
+        stack = functional.table_cache.get(key)
+    if stack is None:
+        stack = torch.cat([t.reshape(-1) for t in ps]).view(torch.uint8)
+        if key is not None:
+            functional.table_cache.put(key, stack, ps)
+    f = stack.view(torch.float32)
+    return f[:n].view(-1, *ws[0].shape[1:]), f[n:]
+
+
 def _psf_maps(model, k, b, h, w):
     """Every iteration's psf convs[i](k).view(b, 64, h, w) (converse_usrnet.py:203-211 computes each in
     its loop; they depend on k only).  On HIP the 1x1 convolutions (16 -> 64 channels on psf-sized maps,
     a few microseconds of work each, bound by launch and memory latency) run as one launch with the
-    weights stacked (kept while the parameters are unchanged), and one transposing copy lays the
-    output out iteration-major, so that each iteration's psf is a contiguous (b, 64, h, w) view."""
+    weights stacked, and one transposing copy lays the output out iteration-major, so that each iteration's
+    psf is a contiguous (b, 64, h, w) view."""
     convs = model.convs
     if all(_hip_eligible(k, m.weight, m.bias) for m in convs):
-        params = [t for m in convs for t in (m.weight, m.bias)]
-        key = tuple((t.data_ptr(), t._version) for t in params)
-        cached = getattr(model, "_psf_stack", None)
-        if cached is None or cached[0] != key:
-            cached = (key, torch.cat([m.weight for m in convs]), torch.cat([m.bias for m in convs]))
-            model._psf_stack = cached
         n, m_ = convs[0].weight.shape[0], len(convs)
-        y = functional.conv1x1(k, cached[1], cached[2])  # (b, m n, kh, kw)
+        y = functional.conv1x1(k, *_psf_stack(convs))  # (b, m n, kh, kw)
         z = y.view(b, m_, n * y.shape[2] * y.shape[3]).transpose(0, 1).contiguous()
         return [z[i].view(b, n, h, w) for i in range(m_)]
     return [_conv(m, k).view(b, 64, h, w) for m in convs]

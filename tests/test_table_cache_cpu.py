@@ -71,6 +71,48 @@ def test_entries_keep_the_memory_of_reassigned_parameters():
     assert c.get(_key(w, b)) is None
 
 
+def test_psf_stack_follows_the_convolutions(monkeypatch):
+    """The weights that ConverseUSRNet stacks: reassigned through .data (the version stays, and the old memory may
+    come back under the same address with other values), updated in place, and made in inference mode."""
+    from conversenet_amd import converse_usrnet as M
+
+    seen = []  # the stacked weights and biases that each forward used
+    monkeypatch.setattr(M, "_hip_eligible", lambda *ts: True)
+    monkeypatch.setattr(Fh, "conv1x1", lambda k, w, b: (seen.append((w.clone(), b.clone())),
+                                                        torch.nn.functional.conv2d(k, w, b))[1])
+    monkeypatch.setattr(Fh, "table_cache", Fh.TableCache())
+
+    class Net:
+        pass
+
+    def check(net):
+        k = torch.rand(2, 16, 3, 3)
+        with torch.no_grad():
+            maps = M._psf_maps(net, k, 2, 3, 3)
+            for c, got in zip(net.convs, maps):
+                assert torch.equal(got, c(k).view(2, 64, 3, 3)) or torch.allclose(got, c(k).view(2, 64, 3, 3), atol=1e-6)
+        w, b = seen[-1]
+        assert torch.equal(w, torch.cat([c.weight for c in net.convs]))
+        assert torch.equal(b, torch.cat([c.bias for c in net.convs]))
+
+    net = Net()
+    net.convs = [torch.nn.Conv2d(16, 64, 1) for _ in range(3)]
+    check(net)
+    ps = [t for c in net.convs for t in (c.weight, c.bias)]
+    old = [(t.data_ptr(), t.detach().clone()) for t in ps]
+    for t in ps:
+        t.data = torch.rand_like(t)
+    held = {t.data_ptr(): t for _, refs in Fh.table_cache.entries.values() for t in refs}
+    assert all(p in held and torch.equal(held[p], v) for p, v in old)
+    check(net)
+    with torch.no_grad():
+        net.convs[1].weight.mul_(2)
+    check(net)
+    with torch.inference_mode():
+        net.convs = [torch.nn.Conv2d(16, 64, 1) for _ in range(3)]
+        check(net)
+
+
 def test_cacheable_rules():
     w = torch.nn.Parameter(torch.ones(1, 4, 3, 3))
     b = torch.nn.Parameter(torch.zeros(1, 4, 1, 1))

@@ -123,14 +123,15 @@ def _psf_stack(convs):
     ps = ws + bs
     n, dev = sum(w.numel() for w in ws), ws[0].device
     key = stack = None
+    st = functional._stream(dev)
     if all(functional.cacheable(w, b) for w, b in zip(ws, bs)):
         key = ("psf stack", tuple(t.data_ptr() for t in ps), tuple(t._version for t in ps), None, None, None,
                tuple(t.shape for t in ps), None, dev.index, tuple(t.stride() for t in ps))
-        stack = functional.table_cache.get(key)
+        stack = functional.table_cache.get(key, st)
     if stack is None:
         stack = torch.cat([t.reshape(-1) for t in ps]).view(torch.uint8)
         if key is not None:
-            functional.table_cache.put(key, stack, ps)
+            functional.table_cache.put(key, stack, ps, st)
     f = stack.view(torch.float32)
     return f[:n].view(-1, *ws[0].shape[1:]), f[n:]
 

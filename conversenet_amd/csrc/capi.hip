@@ -31,6 +31,18 @@ extern "C" const char* cvn_last_error(void) { return last_error_slot().c_str(); 
 
 extern "C" int cvn_clear_cache(void) { return CVN_OK; }
 
+extern "C" int cvn_event_wait(void* event) {
+  if (!event) return fail(CVN_ERR_ARG, "null event");
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+  if (e == hipSuccess) {
+    e = hipEventSynchronize((hipEvent_t)event);
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) e = back;
+  }
+  return e == hipSuccess ? CVN_OK : fail(CVN_ERR_HIP, "event wait: %s", hipGetErrorString(e));
+}
+
 extern "C" int cvn_copy_f32(const float* src, float* dst, int64_t n, cvn_stream_t stream) {
   if (n < 0 || (n > 0 && (!src || !dst))) return fail(CVN_ERR_ARG, "bad copy arguments");
   if (n == 0) return CVN_OK;

@@ -11,6 +11,7 @@ import os
 import threading
 
 import torch
+from torch.multiprocessing.reductions import StorageWeakRef
 
 from . import _lib, composite
 
@@ -54,6 +55,44 @@ def release_workspace():
         _ws_cache.clear()
 
 
+def _capturing(stream) -> bool:
+    """Whether the current stream (its handle) records a graph; the null stream cannot."""
+    return bool(stream) and torch.cuda.is_current_stream_capturing()
+
+
+class _Made:
+    """Where the kernels that made a table were enqueued, and what other streams need before they read it."""
+
+    __slots__ = ("dev", "event", "streams")
+
+    def __init__(self, dev, stream):
+        self.dev = dev
+        self.streams = {stream}  # streams that may use the table and its memory in their own order
+        self.event = torch.cuda.Event()  # None once it is known to have passed
+        self.event.record(torch.cuda.current_stream(dev))
+
+    def join(self, table, stream):
+        """Orders the current stream (its handle) after the making of the table, and the release of the table's
+        memory after what that stream has enqueued by then."""
+        if stream in self.streams:
+            return
+        cur = torch.cuda.current_stream(self.dev)
+        if self.event is not None:
+            cur.wait_event(self.event)
+        table.record_stream(cur)
+        self.streams.add(stream)
+
+    def finish(self):
+        """Waits on the host.  (A stream that records a graph cannot wait for an event from outside it.)"""
+        if self.event is not None:
+            _lib.check(_lib.load().cvn_event_wait(self.event.cuda_event), "transfer table")
+            self.event = None
+
+
+class _Entry(tuple):
+    """(table, memory of psf and bias), with `made` (None without a stream)."""
+
+
 class TableCache:
     """LRU cache of transfer tables, the counterpart of the reference's OTF cache (converse2d.cpp:52-102).
 
@@ -67,7 +106,13 @@ class TableCache:
     a write, as with the reference's cache, which keys on the data pointer alone.
 
     Callers cache only tables that can be hit again (see `cacheable`).  Bounded by the reference's
-    64 entries and by bytes."""
+    64 entries and by bytes.
+
+    Tables are read on any stream: a hit on another stream than the one that made the table waits for it there.
+    A table made while its stream records a graph exists once the graph has run, so it is not kept; one from
+    before that the graph reads stays until the psf's memory is released (the graph goes on reading it after an
+    update of the parameters and clear_cache: record it again then).  At most max_entries tables stay that way;
+    past that, a graph makes its own."""
 
     def __init__(self, max_entries=64, max_bytes=4 << 30):
         from collections import OrderedDict
@@ -80,15 +125,35 @@ class TableCache:
         self.bytes = 0
         self.hits = 0
         self.misses = 0
+        self.recorded = []  # (psf storage, table) read by recorded graphs
 
     @staticmethod
     def _stem(key):
         return key[:2] + key[3:4] + key[5:]
 
-    def get(self, key):
+    def _keep_recorded(self, e):  # caller holds self._lock
+        self.recorded = [r for r in self.recorded if not r[0].expired()]
+        if any(t is e[0] for _, t in self.recorded):
+            return True
+        if len(self.recorded) >= self.max_entries or sum(t.numel() for _, t in self.recorded) > self.max_bytes:
+            return False
+        self.recorded.append((StorageWeakRef(e[1][0].untyped_storage()), e[0]))
+        return True
+
+    def _usable(self, e, stream):  # caller holds self._lock
+        if e.made is None or stream is None:
+            return True
+        if _capturing(stream):
+            e.made.finish()
+            return self._keep_recorded(e)
+        e.made.join(e[0], stream)
+        return True
+
+    def get(self, key, stream=None):
+        """The table of `key` or None.  stream: the current stream's handle, where the table is to be read."""
         with self._lock:
             e = self.entries.get(key)
-            if e is None:
+            if e is None or not self._usable(e, stream):
                 self.misses += 1
                 return None
             self.entries.move_to_end(key)
@@ -102,8 +167,12 @@ class TableCache:
         if self.latest.get(stem) == key:
             del self.latest[stem]
 
-    def put(self, key, table, refs):
-        refs = tuple(t.detach() for t in refs)
+    def put(self, key, table, refs, stream=None):
+        """Keeps `table`.  stream: the current stream's handle, where its kernels have been enqueued."""
+        if stream is not None and _capturing(stream):
+            return
+        e = _Entry((table, tuple(t.detach() for t in refs)))
+        e.made = None if stream is None else _Made(table.device, stream)
         with self._lock:
             old = self.latest.get(self._stem(key))
             if old is not None and old in self.entries:
@@ -111,7 +180,7 @@ class TableCache:
             prev = self.entries.pop(key, None)
             if prev is not None:  # another thread built the same table meanwhile: keep one copy
                 self.bytes -= prev[0].numel()
-            self.entries[key] = (table, refs)
+            self.entries[key] = e
             self.latest[self._stem(key)] = key
             self.bytes += table.numel()
             while self.entries and (len(self.entries) > self.max_entries or self.bytes > self.max_bytes):
@@ -213,7 +282,7 @@ def converse2d_fused(x, weight, bias, scale=1, padding=2, padding_mode="circular
     table = None
     if cache and pb == 1 and cacheable(weight, bias):
         key = _cache_key("module", weight, bias, eps, (C, H, W, kh, kw, s, p), route, dev)
-        table = table_cache.get(key)
+        table = table_cache.get(key, st)
     if table is None:
         wc = weight.contiguous()
         bc = bias.contiguous()
@@ -221,7 +290,7 @@ def converse2d_fused(x, weight, bias, scale=1, padding=2, padding_mode="circular
         _lib.check(lib.cvn_converse2d_table_f32(wc.data_ptr(), pb, kh, kw, bc.data_ptr(), float(eps), B, C, H, W,
                                                 s, p, route, table.data_ptr(), tb, st), "converse2d transfer table")
         if key is not None:
-            table_cache.put(key, table, (weight, bias))
+            table_cache.put(key, table, (weight, bias), st)
     scratch = _workspace(dev, sb, st) if sb > 0 else None
     rc = lib.cvn_converse2d_apply_f32(
         x.data_ptr(), B, C, H, W, pb, kh, kw, s, p, _lib.PAD_MODES[padding_mode],
@@ -373,14 +442,14 @@ def converse2d_op(x, x0, weight, bias, scale, eps=1e-5, cache=True):
     table = None
     if cache and cacheable(weight, bias):
         key = _cache_key("op", weight, bias, eps, (C, h, w, kh, kw, s), 0, dev)
-        table = table_cache.get(key)
+        table = table_cache.get(key, st)
     if table is None:
         wc, bc = weight.contiguous(), bias.contiguous()
         table = torch.empty(tb, dtype=torch.uint8, device=dev)
         _lib.check(lib.cvn_converse2d_op_table_f32(wc.data_ptr(), kh, kw, bc.data_ptr(), float(eps), C, h, w, s,
                                                    table.data_ptr(), tb, st), "converse2d op table")
         if key is not None:
-            table_cache.put(key, table, (weight, bias))
+            table_cache.put(key, table, (weight, bias), st)
     ws = _workspace(dev, sb)
     rc = lib.cvn_converse2d_op_apply_f32(x.data_ptr(), x0.data_ptr(), B, C, h, w, s, table.data_ptr(), tb,
                                          ws.data_ptr(), sb, out.data_ptr(), st)

@@ -177,6 +177,11 @@ int cvn_converse2d_op_apply_f32(const float* x, const float* x0, int64_t B, int6
  * it is kept so that a binding of the reference's clear_cache has a symbol to call. */
 int cvn_clear_cache(void);
 
+/* Waits on the host until a HIP event (hipEvent_t, recorded outside any graph) has passed.  Unlike a plain
+ * hipEventSynchronize it may be called by a thread whose stream records a graph, so that a table built before
+ * the recording is complete before the graph reads it. */
+int cvn_event_wait(void* event);
+
 /* y = weight[c] * (x - mean_c) / sqrt(var_c + eps) + bias[c], statistics over C per pixel.
  * x, y: (B,C,HW). */
 int cvn_layernorm_cf_f32(const float* x, int64_t B, int64_t C, int64_t HW, const float* weight,

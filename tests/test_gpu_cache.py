@@ -37,3 +37,55 @@ def test_views_of_one_psf(entry):
             x0 = x.repeat_interleave(2, 2).repeat_interleave(2, 3)
             got = Fh.converse2d_op(x, x0, v, b, 2, 1e-5)
         assert np.abs(got.cpu().numpy() - _ref(x, v, b, 2)).max() <= TOL
+
+
+def test_table_made_on_another_stream():
+    """A hit waits for a table that is still being made on another stream (delayed there by a spinning kernel)."""
+    from conversenet_amd import functional as Fh
+
+    x, w, b = _case("streams", C=64, H=40, W=40)
+    refs = [_ref(x, w, b, 2), _ref(x, w, b, 1)]
+    a, s = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(20_000_000)
+        Fh.converse2d_fused(x, w, b, 2, 0, "circular", 1e-5)
+        Fh.converse2d_fused(x, w, b, 1, 0, "circular", 1e-5)
+    with torch.cuda.stream(s):
+        hits = Fh.table_cache.hits
+        got = [Fh.converse2d_fused(x, w, b, n, 0, "circular", 1e-5) for n in (2, 1)]
+        assert Fh.table_cache.hits == hits + 2
+    torch.cuda.synchronize()
+    for g, r in zip(got, refs):
+        assert np.abs(g.cpu().numpy() - r).max() <= TOL
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_recorded_graph(warm):
+    """A recorded call without its table makes one in the graph, for itself alone; with one from before, the table
+    outlives the cache's entry.  Replays between other work, each against the eager result."""
+    from conversenet_amd import functional as Fh
+
+    x, w, b = _case(("graph", warm), C=16, H=36, W=28)
+    ref = _ref(x, w, b, 2)
+    if warm:
+        Fh.converse2d_fused(x, w, b, 2, 0, "circular", 1e-5)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = Fh.converse2d_fused(x, w, b, 2, 0, "circular", 1e-5)
+    misses = Fh.table_cache.misses
+    got = Fh.converse2d_fused(x, w, b, 2, 0, "circular", 1e-5)  # eager, the graph has not run yet
+    assert Fh.table_cache.misses == misses + (not warm)
+    assert np.abs(got.cpu().numpy() - ref).max() <= TOL
+    torch.ops.converse2d.clear_cache()
+    for n in range(3):
+        junk = [torch.full((1 << 18,), float("nan"), device=DEV) for _ in range(40)]  # takes over what was released
+        x2 = x * (n + 1)
+        eager = Fh.converse2d_fused(x2, w, b, 2, 0, "circular", 1e-5)
+        keep = x.clone()
+        x.copy_(x2)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), n
+        x.copy_(keep)
+        del junk

@@ -81,6 +81,7 @@ def test_psf_stack_follows_the_convolutions(monkeypatch):
     monkeypatch.setattr(Fh, "conv1x1", lambda k, w, b: (seen.append((w.clone(), b.clone())),
                                                         torch.nn.functional.conv2d(k, w, b))[1])
     monkeypatch.setattr(Fh, "table_cache", Fh.TableCache())
+    monkeypatch.setattr(Fh, "_stream", lambda dev: None)
 
     class Net:
         pass
@@ -111,6 +112,60 @@ def test_psf_stack_follows_the_convolutions(monkeypatch):
     with torch.inference_mode():
         net.convs = [torch.nn.Conv2d(16, 64, 1) for _ in range(3)]
         check(net)
+
+
+def _fake_streams(monkeypatch):
+    """Tables' stream ordering written down instead of enqueued; state["capturing"]: the streams that record a graph."""
+    log, state = [], {"capturing": set()}
+
+    class Made:
+        def __init__(self, dev, stream):
+            self.made_on = stream
+            log.append(("made", stream))
+
+        def join(self, table, stream):
+            if stream != self.made_on:
+                log.append(("wait and hold", stream))
+
+        def finish(self):
+            log.append(("host wait",))
+
+    monkeypatch.setattr(Fh, "_Made", Made)
+    monkeypatch.setattr(Fh, "_capturing", lambda s: s in state["capturing"])
+    return log, state
+
+
+def test_hits_wait_for_the_stream_that_made_the_table(monkeypatch):
+    log, state = _fake_streams(monkeypatch)
+    c = Fh.TableCache()
+    w, b = torch.ones(1, 4, 3, 3), torch.zeros(1, 4, 1, 1)
+    c.put(_key(w, b), torch.empty(8, dtype=torch.uint8), (w, b), 7)
+    assert c.get(_key(w, b), 7) is not None and log == [("made", 7)]
+    assert c.get(_key(w, b), 9) is not None and log[1:] == [("wait and hold", 9)]
+
+
+def test_tables_and_recorded_graphs(monkeypatch):
+    """A table made while its stream records a graph is not kept; one made before is waited for, and stays while a
+    graph may read it: until the psf's memory is released."""
+    log, state = _fake_streams(monkeypatch)
+    c = Fh.TableCache(max_entries=2)
+    state["capturing"] = {5}
+    w, b = torch.ones(1, 4, 3, 3), torch.zeros(1, 4, 1, 1)
+    c.put(_key(w, b), torch.empty(8, dtype=torch.uint8), (w, b), 5)
+    assert not c.entries and c.get(_key(w, b), 0) is None
+    c.put(_key(w, b), torch.empty(8, dtype=torch.uint8), (w, b), 0)
+    t = c.get(_key(w, b), 5)
+    assert t is not None and ("host wait",) in log and len(c.recorded) == 1
+    w.add_(1)
+    c.put(_key(w, b), torch.empty(8, dtype=torch.uint8), (w, b), 0)
+    c.clear()
+    assert any(r is t for _, r in c.recorded)  # replaced, then cleared: the graph still reads it
+    others = [(torch.ones(1, 1, 3, 3), b) for _ in range(2)]
+    for n, (v, u) in enumerate(others):
+        c.put(_key(v, u), torch.empty(8, dtype=torch.uint8), (v, u), 0)
+        assert (c.get(_key(v, u), 5) is not None) == (n == 0)  # at most max_entries: then a graph makes its own
+    del w
+    assert c.get(_key(*others[1]), 5) is not None and not any(r is t for _, r in c.recorded)
 
 
 def test_cacheable_rules():

@@ -31,12 +31,14 @@ extern "C" const char* cvn_last_error(void) { return last_error_slot().c_str(); 
 
 extern "C" int cvn_clear_cache(void) { return CVN_OK; }
 
-extern "C" int cvn_event_wait(void* event) {
+extern "C" int cvn_event_wait(void* event, cvn_stream_t stream) {
   if (!event) return fail(CVN_ERR_ARG, "null event");
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
   if (e == hipSuccess) {
-    e = hipEventSynchronize((hipEvent_t)event);
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (stream) e = hipStreamIsCapturing((hipStream_t)stream, &status);
+    if (e == hipSuccess && status == hipStreamCaptureStatusNone) e = hipEventSynchronize((hipEvent_t)event);
     const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
     if (e == hipSuccess) e = back;
   }

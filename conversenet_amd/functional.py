@@ -17,7 +17,8 @@ from . import _lib, composite
 
 # The op is callable from any host thread (the reference guards its OTF cache with a mutex,
 # converse2d.cpp:56,70,90): the workspace map, the plan memo and the table cache each take a lock
-# around their dict updates.  Kernel launches and table builds run outside the locks.
+# around their dict updates.  Table builds run outside the locks, launches that use a stream's scratch under
+# that scratch's own lock.
 _ws_cache: dict = {}
 _ws_lock = threading.Lock()
 
@@ -38,16 +39,35 @@ def _need_hip(*ts):
             raise RuntimeError("conversenet_amd HIP path computes in float32")
 
 
-def _workspace(dev, nbytes: int, stream=None):
-    """A reusable uint8 scratch tensor per (device, stream); grows monotonically.  stream: the current
-    stream's handle when the caller has it already."""
-    key = (dev.index, _stream(dev) if stream is None else stream)
-    with _ws_lock:
-        buf = _ws_cache.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
-            _ws_cache[key] = buf
-    return buf
+class _Scratch:
+    """A uint8 buffer that grows; `lock` is held while a call that uses it enqueues its kernels."""
+
+    __slots__ = ("dev", "lock", "buf")
+
+    def __init__(self, dev):
+        self.dev, self.lock, self.buf = dev, threading.Lock(), None
+
+    def ptr(self, nbytes):
+        if nbytes == 0:
+            return None
+        if self.buf is None or self.buf.numel() < nbytes:
+            self.buf = torch.empty(nbytes, dtype=torch.uint8, device=self.dev)
+        return self.buf.data_ptr()
+
+
+def _scratch(dev, stream):
+    """The scratch of the calls on a device's stream (its handle; the current one).  Its lock keeps the kernels of
+    two threads' calls on one stream from alternating: one call's would overwrite what the other's still read.  A
+    recorded graph gets a buffer of its own, in the graph's memory: it runs at any time, on any stream, and a kept
+    buffer may be replaced by a larger one."""
+    if _capturing(stream):
+        return _Scratch(dev)
+    key = (dev.index, stream)
+    s = _ws_cache.get(key)
+    if s is None:
+        with _ws_lock:
+            s = _ws_cache.setdefault(key, _Scratch(dev))
+    return s
 
 
 def release_workspace():
@@ -57,16 +77,16 @@ def release_workspace():
 
 def _capturing(stream) -> bool:
     """Whether the current stream (its handle) records a graph; the null stream cannot."""
-    return bool(stream) and torch.cuda.is_current_stream_capturing()
+    return stream != 0 and torch._C._cuda_isCurrentStreamCapturing()
 
 
 class _Made:
     """Where the kernels that made a table were enqueued, and what other streams need before they read it."""
 
-    __slots__ = ("dev", "event", "streams")
+    __slots__ = ("dev", "stream", "event", "streams")
 
     def __init__(self, dev, stream):
-        self.dev = dev
+        self.dev, self.stream = dev, stream
         self.streams = {stream}  # streams that may use the table and its memory in their own order
         self.event = torch.cuda.Event()  # None once it is known to have passed
         self.event.record(torch.cuda.current_stream(dev))
@@ -74,8 +94,6 @@ class _Made:
     def join(self, table, stream):
         """Orders the current stream (its handle) after the making of the table, and the release of the table's
         memory after what that stream has enqueued by then."""
-        if stream in self.streams:
-            return
         cur = torch.cuda.current_stream(self.dev)
         if self.event is not None:
             cur.wait_event(self.event)
@@ -83,9 +101,9 @@ class _Made:
         self.streams.add(stream)
 
     def finish(self):
-        """Waits on the host.  (A stream that records a graph cannot wait for an event from outside it.)"""
+        """Waits on the host: a stream that records a graph cannot wait for an event from outside it."""
         if self.event is not None:
-            _lib.check(_lib.load().cvn_event_wait(self.event.cuda_event), "transfer table")
+            _lib.check(_lib.load().cvn_event_wait(self.event.cuda_event, self.stream), "transfer table")
             self.event = None
 
 
@@ -141,19 +159,18 @@ class TableCache:
         return True
 
     def _usable(self, e, stream):  # caller holds self._lock
-        if e.made is None or stream is None:
-            return True
         if _capturing(stream):
             e.made.finish()
             return self._keep_recorded(e)
-        e.made.join(e[0], stream)
+        if stream not in e.made.streams:
+            e.made.join(e[0], stream)
         return True
 
     def get(self, key, stream=None):
         """The table of `key` or None.  stream: the current stream's handle, where the table is to be read."""
         with self._lock:
             e = self.entries.get(key)
-            if e is None or not self._usable(e, stream):
+            if e is None or not (e.made is None or stream is None or self._usable(e, stream)):
                 self.misses += 1
                 return None
             self.entries.move_to_end(key)
@@ -208,11 +225,14 @@ def cacheable(weight, bias) -> bool:
 
 
 def _cache_key(kind, weight, bias, eps, geo, route, dev):
-    # with the strides: a transposed or expanded view starts at its base's address and shares its version
+    # with the strides of a view: a transposed or expanded one starts at its base's address and shares its version
     return (kind, weight.data_ptr(), weight._version, bias.data_ptr(), bias._version, float(eps), geo, route,
-            dev.index, weight.stride(), bias.stride())
+            dev.index, None if weight.is_contiguous() else weight.stride(),
+            None if bias.is_contiguous() else bias.stride())
 
 
+# os.environ's own mapping: a name that is not set costs 0.6 us through os.environ, which raises for it twice
+_ENV = os.environ._data
 _plan_memo: dict = {}
 _supported_memo: dict = {}  # the library's answers by geometry, as in _plan_memo
 _plan_lock = threading.Lock()
@@ -222,7 +242,7 @@ def _module_plan(lib, B, C, H, W, pb, kh, kw, s, p):
     """(route, table bytes, scratch bytes) of a module-level call: the library's answers depend only on
     the geometry and CVN_DISABLE_FUSED, so they are asked once per geometry (three queries cost about as
     much host time as a small layer's kernels)."""
-    key = (B, C, H, W, pb, kh, kw, s, p, os.environ.get("CVN_DISABLE_FUSED"))
+    key = (B, C, H, W, pb, kh, kw, s, p, _ENV.get(b"CVN_DISABLE_FUSED"))
     plan = _plan_memo.get(key)
     if plan is None:
         route = lib.cvn_converse2d_route(B, C, H, W, pb, kh, kw, s, p)
@@ -291,11 +311,12 @@ def converse2d_fused(x, weight, bias, scale=1, padding=2, padding_mode="circular
                                                 s, p, route, table.data_ptr(), tb, st), "converse2d transfer table")
         if key is not None:
             table_cache.put(key, table, (weight, bias), st)
-    scratch = _workspace(dev, sb, st) if sb > 0 else None
-    rc = lib.cvn_converse2d_apply_f32(
-        x.data_ptr(), B, C, H, W, pb, kh, kw, s, p, _lib.PAD_MODES[padding_mode],
-        _lib.ACT_GELU if act == "gelu" else _lib.ACT_NONE, route, table.data_ptr(), tb,
-        scratch.data_ptr() if scratch is not None else None, sb, out.data_ptr(), st)
+    ws = _scratch(dev, st)
+    with ws.lock:
+        rc = lib.cvn_converse2d_apply_f32(
+            x.data_ptr(), B, C, H, W, pb, kh, kw, s, p, _lib.PAD_MODES[padding_mode],
+            _lib.ACT_GELU if act == "gelu" else _lib.ACT_NONE, route, table.data_ptr(), tb, ws.ptr(sb), sb,
+            out.data_ptr(), st)
     _lib.check(rc, "converse2d_fused")
     return out
 
@@ -310,7 +331,7 @@ def supported(x, weight, scale, padding, grad_x=False, grad_weight=False, shape=
     B, C, H, W = shape if shape is not None else x.shape
     pb, _, kh, kw = weight.shape
     key = (B, C, H, W, pb, kh, kw, int(scale), int(padding), bool(grad_x), bool(grad_weight),
-           os.environ.get("CVN_DISABLE_FUSED"))
+           _ENV.get(b"CVN_DISABLE_FUSED"))
     ok = _supported_memo.get(key)
     if ok is None:
         ok = lib.cvn_converse2d_supported(*key[:9], int(key[9]), int(key[10])) == _lib.CVN_OK
@@ -375,11 +396,13 @@ def converse2d_backward(grad_out, x, weight, bias, scale=1, padding=2, padding_m
     nb = lib.cvn_converse2d_bwd_workspace(B, C, H, W, pb, kh, kw, s, p)
     if nb == 0:
         _lib.check(_lib.CVN_ERR_ARG, "converse2d_backward")
-    ws = _workspace(dev, nb)
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
-    rc = lib.cvn_converse2d_bwd_f32(go.data_ptr(), xc.data_ptr(), B, C, H, W, wc.data_ptr(), pb, kh, kw,
-                                    bc.data_ptr(), float(eps), s, p, _lib.PAD_MODES[padding_mode], ptr(gx), ptr(gw),
-                                    ptr(gb), ws.data_ptr(), nb, _stream(dev))
+    st = _stream(dev)
+    ws = _scratch(dev, st)
+    with ws.lock:
+        rc = lib.cvn_converse2d_bwd_f32(go.data_ptr(), xc.data_ptr(), B, C, H, W, wc.data_ptr(), pb, kh, kw,
+                                        bc.data_ptr(), float(eps), s, p, _lib.PAD_MODES[padding_mode], ptr(gx),
+                                        ptr(gw), ptr(gb), ws.ptr(nb), nb, st)
     _lib.check(rc, "converse2d_backward")
     return gx, gw, gb.reshape(bias.shape) if gb is not None else None
 
@@ -450,9 +473,10 @@ def converse2d_op(x, x0, weight, bias, scale, eps=1e-5, cache=True):
                                                    table.data_ptr(), tb, st), "converse2d op table")
         if key is not None:
             table_cache.put(key, table, (weight, bias), st)
-    ws = _workspace(dev, sb)
-    rc = lib.cvn_converse2d_op_apply_f32(x.data_ptr(), x0.data_ptr(), B, C, h, w, s, table.data_ptr(), tb,
-                                         ws.data_ptr(), sb, out.data_ptr(), st)
+    ws = _scratch(dev, st)
+    with ws.lock:
+        rc = lib.cvn_converse2d_op_apply_f32(x.data_ptr(), x0.data_ptr(), B, C, h, w, s, table.data_ptr(), tb,
+                                             ws.ptr(sb), sb, out.data_ptr(), st)
     _lib.check(rc, "converse2d_op")
     return out
 
@@ -470,10 +494,13 @@ def converse2d_fwd_oneshot(x, weight, bias, scale=1, padding=2, padding_mode="ci
         x = x.clone()
     out = torch.empty((B, C, H * s, W * s), dtype=torch.float32, device=x.device)
     nb = lib.cvn_converse2d_fwd_workspace(B, C, H, W, pb, kh, kw, s, p)
-    ws = _workspace(x.device, max(nb, 1))
-    rc = lib.cvn_converse2d_fwd_f32(x.data_ptr(), B, C, H, W, wc.data_ptr(), pb, kh, kw, bc.data_ptr(), float(eps), s,
-                                    p, _lib.PAD_MODES[padding_mode], _lib.ACT_GELU if act == "gelu" else _lib.ACT_NONE,
-                                    out.data_ptr(), ws.data_ptr(), nb, _stream(x.device))
+    st = _stream(x.device)
+    ws = _scratch(x.device, st)
+    with ws.lock:
+        rc = lib.cvn_converse2d_fwd_f32(x.data_ptr(), B, C, H, W, wc.data_ptr(), pb, kh, kw, bc.data_ptr(), float(eps),
+                                        s, p, _lib.PAD_MODES[padding_mode],
+                                        _lib.ACT_GELU if act == "gelu" else _lib.ACT_NONE, out.data_ptr(),
+                                        ws.ptr(max(nb, 1)), nb, st)
     _lib.check(rc, "converse2d_fwd")
     return out
 

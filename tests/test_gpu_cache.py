@@ -89,3 +89,52 @@ def test_recorded_graph(warm):
         assert torch.equal(out, eager), n
         x.copy_(keep)
         del junk
+
+
+def test_two_threads_on_one_stream():
+    """Calls of two threads on the default stream, on the multi-pass route: each thread's results are its own."""
+    import threading
+
+    from conversenet_amd import functional as Fh
+
+    cases = [_case(("threads", n), C=8, H=40 + 4 * n, W=36) for n in range(2)]
+    want = [Fh.converse2d_fused(*c, 2, 0, "circular", 1e-5) for c in cases]
+    wrong, start = [], threading.Barrier(2)
+
+    def work(n):
+        start.wait()
+        for i in range(50):
+            got = Fh.converse2d_fused(*cases[n], 2, 0, "circular", 1e-5)
+            if not torch.equal(got, want[n]):
+                wrong.append((n, i))
+
+    ts = [threading.Thread(target=work, args=(n,)) for n in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not wrong, wrong[:5]
+
+
+def test_graph_keeps_its_scratch():
+    """A graph recorded on the stream of the calls before it, which grow that stream's scratch afterwards."""
+    from conversenet_amd import functional as Fh
+
+    x, w, b = _case("graph scratch", C=8, H=36, W=36)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        want = Fh.converse2d_fused(x, w, b, 2, 0, "circular", 1e-5)
+    with torch.cuda.graph(g, stream=s):
+        out = Fh.converse2d_fused(x, w, b, 2, 0, "circular", 1e-5)
+    big = torch.randn(4, 8, 96, 96, device=DEV)
+    for n in range(3):
+        with torch.cuda.stream(s):
+            Fh.converse2d_fused(big[: n + 2], w, b, 2, 0, "circular", 1e-5)
+            canary = [torch.zeros(1 << 16, device=DEV) for _ in range(20)]
+        s.synchronize()
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and not any(c.any() for c in canary)

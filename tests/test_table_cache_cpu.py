@@ -120,12 +120,12 @@ def _fake_streams(monkeypatch):
 
     class Made:
         def __init__(self, dev, stream):
-            self.made_on = stream
+            self.streams = {stream}
             log.append(("made", stream))
 
         def join(self, table, stream):
-            if stream != self.made_on:
-                log.append(("wait and hold", stream))
+            self.streams.add(stream)
+            log.append(("wait and hold", stream))
 
         def finish(self):
             log.append(("host wait",))
@@ -224,3 +224,43 @@ def test_concurrent_callers_keep_the_cache_consistent():
     assert len(c.entries) <= 16
     assert c.bytes == sum(t.numel() for t, _ in c.entries.values())
     assert all(c.latest[c._stem(k)] == k for k in c.entries)
+
+
+def test_scratch_belongs_to_one_call_at_a_time(monkeypatch):
+    """Two threads on one stream: the second call's kernels follow the first's; a graph's call has its own buffer."""
+    import threading
+
+    dev = torch.device("cpu")
+    monkeypatch.setattr(Fh, "_capturing", lambda s: s == 5)
+    inside, go_on, order = threading.Event(), threading.Event(), []
+
+    def first():
+        ws = Fh._scratch(dev, 0)
+        with ws.lock:
+            order.append(("first in", ws.ptr(1000)))
+            inside.set()
+            go_on.wait(10)
+            order.append(("first out", ws.ptr(500)))
+
+    def second():
+        inside.wait(10)
+        ws = Fh._scratch(dev, 0)
+        with ws.lock:
+            order.append(("second in", ws.ptr(1000)))
+
+    ts = [threading.Thread(target=f) for f in (first, second)]
+    for t in ts:
+        t.start()
+    inside.wait(10)
+    ts[1].join(0.2)
+    assert ts[1].is_alive()  # waits for the first
+    assert Fh._scratch(dev, 9).lock.acquire(blocking=False)  # another stream does not
+    go_on.set()
+    for t in ts:
+        t.join(10)
+    assert [n for n, _ in order] == ["first in", "first out", "second in"] and len({p for _, p in order}) == 1
+    g, g2 = Fh._scratch(dev, 5), Fh._scratch(dev, 5)
+    assert g is not g2 and g.ptr(10) != g2.ptr(10)
+    assert (None, 5) not in Fh._ws_cache
+    Fh.release_workspace()
+    assert not Fh._ws_cache

@@ -509,18 +509,27 @@ def layernorm_cf(x, weight, bias, eps):
     """LayerNorm(data_format='channels_first') (util_converse.py:63-68)."""
     lib = _lib.load()
     _need_hip(x, weight, bias)
-    x = x.contiguous()
+    x, weight, bias = x.contiguous(), weight.contiguous(), bias.contiguous()
     B, C = x.shape[:2]
     HW = x[0, 0].numel() if B > 0 else 0
     y = torch.empty_like(x)
-    _lib.check(lib.cvn_layernorm_cf_f32(x.data_ptr(), B, C, HW, weight.contiguous().data_ptr(),
-                                        bias.contiguous().data_ptr(), float(eps), y.data_ptr(),
-                                        _stream(x.device)), "layernorm_cf")
+    _lib.check(lib.cvn_layernorm_cf_f32(x.data_ptr(), B, C, HW, weight.data_ptr(), bias.data_ptr(), float(eps),
+                                        y.data_ptr(), _stream(x.device)), "layernorm_cf")
     return y
 
 
 def _wmat(weight):
     return weight.reshape(weight.shape[0], -1).contiguous()
+
+
+def _dense(*ts):
+    """Contiguous tensors (or None) for a call.  The caller keeps them until the call has enqueued its kernels: a
+    copy that is dropped before then gives its memory to the next copy or output."""
+    return [t if t is None else t.contiguous() for t in ts]
+
+
+def _ptr(t):
+    return None if t is None else t.data_ptr()
 
 
 def conv1x1(x, weight, bias=None, act=None, residual=None, res_scale=None, ln=None, out=None):
@@ -535,21 +544,17 @@ def conv1x1(x, weight, bias=None, act=None, residual=None, res_scale=None, ln=No
     if Wm.shape[1] != Cin:
         raise RuntimeError("weight does not match input channels")
     y = out if out is not None else torch.empty((B, Cout, H, W), dtype=torch.float32, device=x.device)
-    if residual is not None:
-        residual = residual.contiguous()
-    bptr = bias.contiguous().data_ptr() if bias is not None else None
-    rptr = residual.data_ptr() if residual is not None else None
-    sptr = res_scale.contiguous().data_ptr() if res_scale is not None else None
+    bias, residual, res_scale = _dense(bias, residual, res_scale)
+    bptr, rptr, sptr = _ptr(bias), _ptr(residual), _ptr(res_scale)
     a = _lib.ACT_GELU if act == "gelu" else _lib.ACT_NONE
     st = _stream(x.device)
     if ln is None:
         rc = lib.cvn_conv1x1_f32(x.data_ptr(), B, Cin, H * W, Wm.data_ptr(), bptr, Cout, a, rptr, sptr,
                                  y.data_ptr(), st)
     else:
-        lw, lb, leps = ln
-        rc = lib.cvn_ln_conv1x1_f32(x.data_ptr(), B, Cin, H * W, lw.contiguous().data_ptr(),
-                                    lb.contiguous().data_ptr(), float(leps), Wm.data_ptr(), bptr, Cout, a, rptr,
-                                    sptr, y.data_ptr(), st)
+        lw, lb = _dense(*ln[:2])
+        rc = lib.cvn_ln_conv1x1_f32(x.data_ptr(), B, Cin, H * W, lw.data_ptr(), lb.data_ptr(), float(ln[2]),
+                                    Wm.data_ptr(), bptr, Cout, a, rptr, sptr, y.data_ptr(), st)
     _lib.check(rc, "conv1x1")
     return y
 
@@ -563,12 +568,10 @@ def ln_mlp_residual(x, ln_w, ln_b, ln_eps, w1, b1, w2, b2, res_scale=None, out=N
     W1 = _wmat(w1)
     W2 = _wmat(w2)
     y = out if out is not None else torch.empty_like(x)
-    rc = lib.cvn_ln_mlp_residual_f32(x.data_ptr(), B, C, H * W, ln_w.contiguous().data_ptr(),
-                                     ln_b.contiguous().data_ptr(), float(ln_eps), W1.data_ptr(),
-                                     b1.contiguous().data_ptr(), W1.shape[0], W2.data_ptr(),
-                                     b2.contiguous().data_ptr(),
-                                     res_scale.contiguous().data_ptr() if res_scale is not None else None,
-                                     y.data_ptr(), _stream(x.device))
+    ln_w, ln_b, b1, b2, res_scale = _dense(ln_w, ln_b, b1, b2, res_scale)
+    rc = lib.cvn_ln_mlp_residual_f32(x.data_ptr(), B, C, H * W, ln_w.data_ptr(), ln_b.data_ptr(), float(ln_eps),
+                                     W1.data_ptr(), b1.data_ptr(), W1.shape[0], W2.data_ptr(), b2.data_ptr(),
+                                     _ptr(res_scale), y.data_ptr(), _stream(x.device))
     _lib.check(rc, "ln_mlp_residual")
     return y
 
@@ -590,19 +593,20 @@ def conv_ln_mlp_residual(t, x, w0, b0, ln_w, ln_b, ln_eps, w1, b1, w2, b2, res_s
     C = x.shape[1]
     W0, W1, W2 = _wmat(w0), _wmat(w1), _wmat(w2)
     y = out if out is not None else torch.empty_like(x)
-    ptr = lambda v: v.contiguous().data_ptr() if v is not None else None
     act = _lib.ACT_GELU if t_act == "gelu" else _lib.ACT_NONE
-    common = (t.data_ptr(), act, B, Ct, H * W, W0.data_ptr(), ptr(b0), ptr(res_scale1), x.data_ptr(), C, ptr(ln_w),
-              ptr(ln_b), float(ln_eps), W1.data_ptr(), ptr(b1), W1.shape[0], W2.data_ptr(), ptr(b2), ptr(res_scale2),
-              y.data_ptr())
+    vs = _dense(b0, res_scale1, ln_w, ln_b, b1, b2, res_scale2)
+    b0_, s1, lw, lb, b1_, b2_, s2 = (_ptr(v) for v in vs)
+    common = (t.data_ptr(), act, B, Ct, H * W, W0.data_ptr(), b0_, s1, x.data_ptr(), C, lw, lb, float(ln_eps),
+              W1.data_ptr(), b1_, W1.shape[0], W2.data_ptr(), b2_, s2, y.data_ptr())
     if head is None:
         _lib.check(lib.cvn_conv_ln_mlp_residual_f32(*common, _stream(x.device)), "conv_ln_mlp_residual")
         return y
     hw, hb, heps, wh, bh = head
     _need_hip(wh, bh)
     Wh = _wmat(wh)
+    hw, hb, bh = _dense(hw, hb, bh)
     tn = torch.empty((B, Wh.shape[0], H, W), device=x.device, dtype=x.dtype)
-    _lib.check(lib.cvn_conv_ln_mlp_head_f32(*common, ptr(hw), ptr(hb), float(heps), Wh.data_ptr(), ptr(bh),
+    _lib.check(lib.cvn_conv_ln_mlp_head_f32(*common, _ptr(hw), _ptr(hb), float(heps), Wh.data_ptr(), _ptr(bh),
                                             tn.data_ptr(), _stream(x.device)), "conv_ln_mlp_head")
     return y, tn
 

@@ -112,3 +112,29 @@ def test_block_and_chain_on_odd_images(mode, k, pad):
         for b in blks:
             y = b(y)
     _close(y, ref, "blocks")
+
+
+def _every_other(t):
+    """The same values with gaps between them: a wrapper copies it to pass it on."""
+    return torch.stack([t, torch.full_like(t, 9.0)], -1)[..., 0] if t is not None else None
+
+
+def test_strided_parameters():
+    """Parameters that a wrapper has to copy: every copy keeps its memory until the kernels are enqueued."""
+    from conversenet_amd import functional as Fh
+
+    p = {k: torch.from_numpy(v).to(DEV) for k, v in _params(64, 128, 5).items()}
+    r = np.random.default_rng(6)
+    x, t = (torch.from_numpy(r.standard_normal((1, c, 9, 13)).astype(np.float32)).to(DEV) for c in (64, 128))
+
+    def calls(d):
+        ln = (d["lw"], d["lb"], 1e-5)
+        yield Fh.layernorm_cf(x, *ln)
+        yield Fh.conv1x1(t, d["w0"], d["b0"], residual=x, res_scale=d["a1"])
+        yield Fh.conv1x1(x, d["w1"], d["b1"], ln=ln)
+        yield Fh.ln_mlp_residual(x, *ln, d["w1"], d["b1"], d["w2"], d["b2"], d["a2"])
+        yield from Fh.conv_ln_mlp_residual(t, x, d["w0"], d["b0"], *ln, d["w1"], d["b1"], d["w2"], d["b2"], d["a1"],
+                                           d["a2"], head=(*ln, d["w1"], d["b1"]))
+
+    for n, (a, b) in enumerate(zip(calls(p), calls({k: _every_other(v) for k, v in p.items()}))):
+        assert torch.equal(a, b), n

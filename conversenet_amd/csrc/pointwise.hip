@@ -285,16 +285,20 @@ __device__ __forceinline__ int64_t tile_px(int64_t t, int64_t tpb, int Q, int NW
 // ------------------------------------------------------------------------------------------------
 // fp32 products on the fp16 matrix cores ("split fp16").  Every operand x is split as x = x_h + x_l,
 // x_h = fp16(x) and x_l = fp16(x - x_h), both rounded to nearest (x - x_h is exact in fp32), so
-// |x - x_h - x_l| <= 2^-22 |x|; a product is formed as a_l b_h + a_h b_l + a_h b_h (three
-// v_mfma_f32_16x16x32_f16, each product exact in the fp32 accumulator), dropping a_l b_l (<= 2^-22
-// |a b|).  The errors have random signs (rounded toward zero, as these splits were at first, they are
+// |x - x_h - x_l| <= 2^-22 |x| while x_l is a normal fp16 number; a product is formed as a_l b_h + a_h b_l +
+// a_h b_h (three v_mfma_f32_16x16x32_f16, each product exact in the fp32 accumulator), dropping a_l b_l
+// (<= 2^-22 |a b|).  The errors have random signs (rounded toward zero, as these splits were at first, they are
 // 2^-20 and one-sided: a ConverseBlock's relative error against fp64 was 1.1e-6, now 2.9e-7; with torch's
-// fp32 1x1 convolutions it is 3.1e-7).  fp16 inputs below the normal range are kept by the matrix cores (gradual underflow), so
-// small values lose no relative accuracy beyond 2^-24 absolute.  A 16 x 16 x 32 block update then
-// takes three of these MFMAs (8192 multiply-adds each, half the issue time of one 16x16x4 fp32 MFMA)
-// instead of eight fp32 MFMAs.  fp16's range ends at 65504: a k-chunk whose activations exceed it in
-// any lane of the wave is multiplied on the fp32 matrix cores instead (weights rebuilt as x_h + x_l),
-// so no input range is lost.
+// fp32 1x1 convolutions it is 3.1e-7).  A 16 x 16 x 32 block update takes three of these MFMAs (8192
+// multiply-adds each, half the issue time of one 16x16x4 fp32 MFMA) instead of eight fp32 MFMAs.
+// fp16's range is short at both ends: above 65504 there is no x_h, and below the normal numbers (2^-14) x_l keeps
+// to a spacing of 2^-24 (the matrix cores do not flush it).  So a weight matrix is scaled to a largest entry of
+// 2^14 (StageF16), and the pixels of a wave are, one by one, where one of them is too large or too small as it
+// is (gemm_f16s).  The operands' error is then the larger of 2^-22 of the value itself and, for activations, 2^-25 of
+// the pixel's largest, for weights 2^-39 of the matrix' largest.  (Activations as they are, whatever their size:
+// a relative error of 1.7e-6 for values of 1e-2 and 1.7e-2 for 1e-6, now 1.1e-7 for all.  With none scaled the
+// 8 x 64 x 256 x 256 tail with a head takes 234 us, 230 before the check; with all scaled 233; 128 -> 64 alone 78,
+// 75 before, when a chunk of channels did not wait for the others' loads.)
 // Operand layout of the 16x16x32 MFMA: lane l = 16 g + j holds A[row j][k = 8 g + e] and
 // B[k = 8 g + e][col j], e < 8; D as for the fp32 MFMAs (lane 16 g + j: rows 4 g + r, col j).  The k
 // slot 8 g + e (e = 4 hf + r) of input chunk c is channel 16 (2 c + hf) + 4 g + r: the channels lane
@@ -324,11 +328,20 @@ __device__ __forceinline__ void split_f16(const float (&x)[8], f16x8& h, f16x8& 
 // Weights (N outputs x K inputs, row-major fp32) in LDS for gemm_f16s: for input chunk c, output
 // block ob and lane 16 g + j, 16 bytes of high parts (W[16 ob + j][channel of k slot 8 g + e], e < 8),
 // and 1 KB further on the 16 bytes of low parts: consecutive lanes read consecutive 16-byte words.
-// The matrix is scaled by a power of two that brings its largest entry to [64, 128): a weight of 0.1 has
-// its low part below fp16's normal range (2^-14), where the spacing of 2^-24 is 3e-7 of it, several times
-// the split's own error.  The caller multiplies the sums by the returned reciprocal, in the fma that
-// adds the bias.  load() reads the block's share into registers and joins the matrix' maximum, put()
+// The matrix is scaled by a power of two that brings its largest entry to [2^14, 2^15), unless it is larger and
+// still in range: a weight of 0.1 has its low part below fp16's normal range (2^-14), where the spacing of 2^-24
+// is 6e-7 of it, several times the split's own error.  The caller multiplies the sums by the returned reciprocal, in the fma that
+// adds the bias.  load() reads the block's share into registers and notes each wave's maximum, put()
 // writes it; between the two the block synchronises (after put() too, before the first use).
+// The largest of 16 lanes (a row of the wave), in all of them.
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float m) {
+  return fmaxf(m, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(m), CTRL, 0xf, 0xf, true)));
+}
+__device__ __forceinline__ float row_max(float m) {  // rotations by 8, 4, 2 and 1 lanes
+  return max_dpp<0x121>(max_dpp<0x122>(max_dpp<0x124>(max_dpp<0x128>(m))));
+}
+
 template <int N, int K, int T>
 struct StageF16 {
   static constexpr int PER = (N * K + T - 1) / T;
@@ -339,7 +352,7 @@ struct StageF16 {
     const int ob = cob % (N / 16), c = cob / (N / 16);
     return (16 * ob + j) * K + 16 * (2 * c + hf) + 4 * g + r;
   }
-  __device__ __forceinline__ void load(const float* __restrict__ W, unsigned* top) {
+  __device__ __forceinline__ void load(const float* __restrict__ W, float* top) {  // top: T / 64 values
     float m = 0.f;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -347,14 +360,17 @@ struct StageF16 {
       w[i] = (N * K % T == 0 || e < N * K) ? W[src(e)] : 0.f;
       m = fmaxf(m, fabsf(w[i]));
     }
-#pragma unroll
-    for (int d = 1; d < 64; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
-    if ((threadIdx.x & 63) == 0) atomicMax(top, __float_as_uint(m));  // m >= 0: ordered as its bits
+    m = row_max(m);
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = m;
   }
-  __device__ __forceinline__ float put(const unsigned* top, _Float16* Wl) const {
-    // exponent of the largest entry, kept inside +-100; zero or infinite entries alone scale by 1
-    const int e2 = (int)(*top >> 23) - 127;
-    const int s = *top == 0 || e2 == 128 ? 0 : 6 - max(-100, min(e2, 100));
+  __device__ __forceinline__ float put(const float* top, _Float16* Wl) const {
+    static_assert(T == 1024, "one wave's maximum per lane of a row");
+    const float m = row_max(top[threadIdx.x & 15]);
+    // exponent of the largest entry (from -100 on); zero or infinite entries alone scale by 1
+    const int e2 = max((int)(__float_as_uint(m) >> 23) - 127, -100);
+    const int s = m == 0.f || e2 == 128 || (m <= kF16Max && e2 > 14) ? 0 : 14 - e2;
     const float sc = ldexpf(1.f, s);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -371,23 +387,61 @@ struct StageF16 {
   }
 };
 
-// acc[ob][q] += W[16 ob + j][k] v[k] over all K input channels; v in the accumulator layout.
+// A lane's flag from any of the 4 lane groups that share its pixel.
+__device__ __forceinline__ uint32_t any_group(uint64_t ballot) {
+  ballot |= ballot >> 32;
+  return (uint32_t)(ballot | ballot >> 16) & 0xffff;
+}
+
+// acc[ob][q] = W[16 ob + j][k] v[k] over all K input channels, times the scale of W unless that is undone here; v in
+// the accumulator layout (changed), acc zero on entry.  Returns the factor that undoes what is left: inv (StageF16),
+// or 1.  Pixels whose largest activation is inside [1, 65504] enter as they are: the low parts are off by at worst
+// 2^-25.  If a pixel of the wave is outside, each one is scaled by the power of two that brings
+// its largest activation to [2^14, 2^15), and the sums are scaled back by both factors at once.
 template <int K, int N, int Q>
-__device__ __forceinline__ void gemm_f16s(const v4f (&v)[K / 16][Q], const _Float16* Wl, int lane,
-                                          v4f (&acc)[N / 16][Q]) {
+__device__ __forceinline__ float gemm_f16s(v4f (&v)[K / 16][Q], const _Float16* Wl, int lane, float inv,
+                                           v4f (&acc)[N / 16][Q]) {
+  bool plain = true, inf = false;
+  int back[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    float m = 0.f;
+#pragma unroll
+    for (int rb = 0; rb < K / 16; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[rb][q][r]));  // (a NaN is left out and stays one)
+    const uint32_t any = any_group(__builtin_amdgcn_ballot_w64(m > 0.f));
+    const uint32_t fit = any_group(__builtin_amdgcn_ballot_w64(m >= 1.f));
+    plain = plain && (any & ~fit) == 0 && __builtin_amdgcn_ballot_w64(m > kF16Max) == 0;
+  }
+  if (!plain) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      float m = 0.f;
+#pragma unroll
+      for (int rb = 0; rb < K / 16; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[rb][q][r]));
+      m = fmaxf(m, __shfl_xor(m, 16));
+      m = fmaxf(m, __shfl_xor(m, 32));
+      const int e2 = (int)(__float_as_uint(m) >> 23) - 127, s = m > 0.f ? min(14 - e2, 126) : 0;
+      inf = inf || __builtin_amdgcn_ballot_w64(e2 == 128) != 0;
+      back[q] = (int)(__float_as_uint(inv) >> 23) - 127 - s;
+      const float sc = ldexpf(1.f, s);
+#pragma unroll
+      for (int rb = 0; rb < K / 16; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[rb][q][r] *= sc;
+    }
+  }
 #pragma unroll
   for (int c = 0; c < K / 32; ++c) {
     float xb[Q][8];
-    float mx = 0.f;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        xb[q][e] = v[2 * c + (e >> 2)][q][e & 3];
-        mx = fmaxf(mx, fabsf(xb[q][e]));
-      }
-    // NaN compares false here and passes through the fp16 products as NaN
-    if (__builtin_amdgcn_ballot_w64(mx > kF16Max) == 0) {
+      for (int e = 0; e < 8; ++e) xb[q][e] = v[2 * c + (e >> 2)][q][e & 3];
+    if (!inf) {
       f16x8 bh[Q], bl[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) split_f16(xb[q], bh[q], bl[q]);
@@ -403,7 +457,7 @@ __device__ __forceinline__ void gemm_f16s(const v4f (&v)[K / 16][Q], const _Floa
         }
         mem_fence_sched();
       }
-    } else {
+    } else {  // an infinity has no low part: the wave's products on the fp32 matrix cores
 #pragma unroll
       for (int ob = 0; ob < N / 16; ++ob) {
         const u32x4_t* wp = (const u32x4_t*)(Wl + (c * (N / 16) + ob) * 1024) + lane;
@@ -418,6 +472,14 @@ __device__ __forceinline__ void gemm_f16s(const v4f (&v)[K / 16][Q], const _Floa
       }
     }
   }
+  if (plain) return inv;
+#pragma unroll
+  for (int ob = 0; ob < N / 16; ++ob)
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[ob][q][r] = ldexpf(acc[ob][q][r], back[q]);
+  return 1.f;
 }
 
 // Loads a (channels x pixels) tile in the accumulator layout: channel 16 rb + 4 g + r in register r of
@@ -493,13 +555,11 @@ __global__ void __launch_bounds__(64 * NW) k_conv1x1_mfma(const float* __restric
   __shared__ float prm[2 * COUT + 2 * CIN];  // bias, residual scale, LN weight, LN bias
   float inv = 1.f;
   if constexpr (F16S) {
-    __shared__ unsigned top;
-    if (threadIdx.x == 0) top = 0;
-    __syncthreads();
+    __shared__ float top[NW];
     StageF16<COUT, CIN, 64 * NW> sw;
-    sw.load(W, &top);
+    sw.load(W, top);
     __syncthreads();
-    inv = sw.put(&top, (_Float16*)Wt);
+    inv = sw.put(top, (_Float16*)Wt);
   } else {
     stage_wt<COUT, CIN, LD>(W, Wt);
   }
@@ -523,6 +583,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv1x1_mfma(const float* __restric
     const bool inb = pw + Q * j < hw;
     v4f acc[COUT / 16][Q];
     zero_acc<COUT, Q>(acc);
+    float inv_t = 1.f;
     if constexpr (F16S) {
       v4f xv[CIN / 16][Q];
       // lanes past the image end load the wave's first pixel (valid, pw < hw), so the loads issue
@@ -530,7 +591,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv1x1_mfma(const float* __restric
       // which measured 2 % faster there); those lanes' values never reach an output
       load_acc<CIN, Q>(x + b * CIN * hw + pw, hw, true, inb ? yoff : yoff0, xv);
       if (LN) ln_acc<CIN, Q>(xv, prm + 2 * COUT, prm + 2 * COUT + CIN, eps, g, xv);
-      gemm_f16s<CIN, COUT, Q>(xv, (const _Float16*)Wt, lane, acc);
+      inv_t = gemm_f16s<CIN, COUT, Q>(xv, (const _Float16*)Wt, lane, inv, acc);
     } else {
       float xv[CIN / 4][Q];
       load_tile<CIN, Q>(x + b * CIN * hw + pw, hw, inb, xoff, xv);
@@ -538,7 +599,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv1x1_mfma(const float* __restric
       gemm_tile<CIN, COUT, Q>(xv, Wt, LD, g, j, acc);
     }
     store_tile<COUT, Q>(acc, y + b * COUT * hw + pw, residual ? residual + b * COUT * hw + pw : nullptr, hw, inb,
-                        yoff, g, inv, prm, act, prm + COUT);
+                        yoff, g, inv_t, prm, act, prm + COUT);
   }
 }
 
@@ -554,15 +615,13 @@ __global__ void __launch_bounds__(64 * NW) k_ln_mlp_mfma(const float* x, int64_t
   __shared__ __align__(16) _Float16 W1l[2 * CM * C];  // StageF16 layouts
   __shared__ __align__(16) _Float16 W2l[2 * C * CM];
   __shared__ float prm[CM + 4 * C];  // b1, b2, residual scale, LN weight, LN bias
-  __shared__ unsigned top[2];
-  if (threadIdx.x < 2) top[threadIdx.x] = 0;
-  __syncthreads();
+  __shared__ float top[2 * NW];
   StageF16<CM, C, 64 * NW> s1;
   StageF16<C, CM, 64 * NW> s2;
   s1.load(W1, top);
-  s2.load(W2, top + 1);
+  s2.load(W2, top + NW);
   __syncthreads();
-  const float inv1 = s1.put(top, W1l), inv2 = s2.put(top + 1, W2l);
+  const float inv1 = s1.put(top, W1l), inv2 = s2.put(top + NW, W2l);
   stage_vec<CM>(b1, 0.f, prm);
   stage_vec<C>(b2, 0.f, prm + CM);
   stage_vec<C>(res_scale, 1.f, prm + CM + C);
@@ -580,12 +639,13 @@ __global__ void __launch_bounds__(64 * NW) k_ln_mlp_mfma(const float* x, int64_t
     const bool inb = pw + Q * j < hw;
     const float* xw = x + b * C * hw + pw;
     v4f h[CM / 16][Q];
+    float u1;
     {
       v4f xv[C / 16][Q];
       load_acc<C, Q>(xw, hw, inb, yoff, xv);
       ln_acc<C, Q>(xv, prm + CM + 2 * C, prm + CM + 3 * C, eps, g, xv);
       zero_acc<CM, Q>(h);
-      gemm_f16s<C, CM, Q>(xv, W1l, lane, h);
+      u1 = gemm_f16s<C, CM, Q>(xv, W1l, lane, inv1, h);
     }
     // bias + GELU on the hidden activations (channel 16 rb + 4 g + r)
 #pragma unroll
@@ -594,12 +654,12 @@ __global__ void __launch_bounds__(64 * NW) k_ln_mlp_mfma(const float* x, int64_t
       for (int r = 0; r < 4; ++r) {
         const float bo = prm[16 * rb + 4 * g + r];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(fmaf(h[rb][q][r], inv1, bo));
+        for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(fmaf(h[rb][q][r], u1, bo));
       }
     v4f acc[C / 16][Q];
     zero_acc<C, Q>(acc);
-    gemm_f16s<CM, C, Q>(h, W2l, lane, acc);
-    store_tile<C, Q>(acc, y + b * C * hw + pw, xw, hw, inb, yoff, g, inv2, prm + CM, CVN_ACT_NONE, prm + CM + C);
+    const float u2 = gemm_f16s<CM, C, Q>(h, W2l, lane, inv2, acc);
+    store_tile<C, Q>(acc, y + b * C * hw + pw, xw, hw, inb, yoff, g, u2, prm + CM, CVN_ACT_NONE, prm + CM + C);
   }
 }
 
@@ -646,21 +706,20 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
   __shared__ __align__(16) _Float16 W2l[2 * C * CM];
   __shared__ __align__(16) _Float16 Whl[HEAD ? 2 * CIN * C : 8];
   __shared__ float prm[NP];  // b0, s1, LN weight, LN bias, b2, s2, b1 [, head LN weight, bias, head bias]
-  __shared__ unsigned top[4];
-  if (threadIdx.x < 4) top[threadIdx.x] = 0;
-  __syncthreads();
+  __shared__ float top[4 * NW];
   StageF16<C, CIN, 64 * NW> sw0;
   StageF16<CM, C, 64 * NW> sw1;
   StageF16<C, CM, 64 * NW> sw2;
   StageF16<CIN, HEAD ? C : 16, 64 * NW> swh;
   sw0.load(a.W0, top);
-  sw1.load(a.W1, top + 1);
-  sw2.load(a.W2, top + 2);
-  if constexpr (HEAD) swh.load(a.Wh, top + 3);
+  sw1.load(a.W1, top + NW);
+  sw2.load(a.W2, top + 2 * NW);
+  if constexpr (HEAD) swh.load(a.Wh, top + 3 * NW);
   __syncthreads();
-  const float inv0 = sw0.put(top, W0l), inv1 = sw1.put(top + 1, W1l), inv2 = sw2.put(top + 2, W2l);
+  const float inv0 = sw0.put(top, W0l), inv1 = sw1.put(top + NW, W1l),
+              inv2 = sw2.put(top + 2 * NW, W2l);
   float invh = 1.f;
-  if constexpr (HEAD) invh = swh.put(top + 3, Whl);
+  if constexpr (HEAD) invh = swh.put(top + 3 * NW, Whl);
   stage_vec<C>(a.b0, 0.f, prm);
   stage_vec<C>(a.s1, 1.f, prm + C);
   stage_vec<C>(a.lw, 1.f, prm + 2 * C);
@@ -685,6 +744,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
     const bool inb = pw + Q * j < hw;
     // first branch's last layer: acc = W0 t (t read in the accumulator layout)
     v4f acc[C / 16][Q];
+    float u0;
     {
       v4f tv[CIN / 16][Q];
       load_acc<CIN, Q>(a.t + b * CIN * hw + pw, hw, inb, yoff, tv);
@@ -697,7 +757,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
             for (int r = 0; r < 4; ++r) tv[rb][q][r] = gelu_f(tv[rb][q][r]);
       }
       zero_acc<C, Q>(acc);
-      gemm_f16s<CIN, C, Q>(tv, W0l, lane, acc);
+      u0 = gemm_f16s<CIN, C, Q>(tv, W0l, lane, inv0, acc);
     }
     // y' = x + s1 (acc + b0), channel 16 rb + 4 g + r; x read in the same layout
     const float* xw = a.x + b * C * hw + pw;
@@ -715,17 +775,19 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         }
         const float bo = prm[o], sc = prm[C + o];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) acc[rb][q][r] = fmaf(sc, fmaf(acc[rb][q][r], inv0, bo), rr[q]);
+        for (int q = 0; q < Q; ++q) acc[rb][q][r] = fmaf(sc, fmaf(acc[rb][q][r], u0, bo), rr[q]);
       }
     // out = y' + s2 (W2 GELU(W1 LN(y') + b1) + b2)
     v4f acc2[C / 16][Q];
+    float u2;
     {
       v4f h[CM / 16][Q];
+      float u1;
       {
         v4f xn[C / 16][Q];
         ln_acc<C, Q>(acc, prm + 2 * C, prm + 3 * C, a.eps, g, xn);
         zero_acc<CM, Q>(h);
-        gemm_f16s<C, CM, Q>(xn, W1l, lane, h);
+        u1 = gemm_f16s<C, CM, Q>(xn, W1l, lane, inv1, h);
       }
 #pragma unroll
       for (int rb = 0; rb < CM / 16; ++rb)
@@ -733,10 +795,10 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         for (int r = 0; r < 4; ++r) {
           const float bo = prm[6 * C + 16 * rb + 4 * g + r];
 #pragma unroll
-          for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(fmaf(h[rb][q][r], inv1, bo));
+          for (int q = 0; q < Q; ++q) h[rb][q][r] = gelu_f(fmaf(h[rb][q][r], u1, bo));
         }
       zero_acc<C, Q>(acc2);
-      gemm_f16s<CM, C, Q>(h, W2l, lane, acc2);
+      u2 = gemm_f16s<CM, C, Q>(h, W2l, lane, inv2, acc2);
     }
 #pragma unroll
     for (int rb = 0; rb < C / 16; ++rb)
@@ -745,17 +807,18 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         const int o = 16 * rb + 4 * g + r;
         const float bo = prm[4 * C + o], sc = prm[5 * C + o];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) acc2[rb][q][r] = fmaf(sc, fmaf(acc2[rb][q][r], inv2, bo), acc[rb][q][r]);
+        for (int q = 0; q < Q; ++q) acc2[rb][q][r] = fmaf(sc, fmaf(acc2[rb][q][r], u2, bo), acc[rb][q][r]);
       }
     if (inb) store_acc<C, Q>(acc2, a.y + b * C * hw + pw, hw, yoff);
     if (HEAD) {
       // next block: th = GELU(Wh LNh(out) + bh)
       v4f hh[CIN / 16][Q];
+      float uh;
       {
         v4f xn[C / 16][Q];
         ln_acc<C, Q>(acc2, prm + 6 * C + CM, prm + 7 * C + CM, a.heps, g, xn);
         zero_acc<CIN, Q>(hh);
-        gemm_f16s<C, CIN, Q>(xn, Whl, lane, hh);
+        uh = gemm_f16s<C, CIN, Q>(xn, Whl, lane, invh, hh);
       }
 #pragma unroll
       for (int rb = 0; rb < CIN / 16; ++rb)
@@ -763,7 +826,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv_ln_mlp_mfma(TailArgs a) {
         for (int r = 0; r < 4; ++r) {
           const float bo = prm[8 * C + CM + 16 * rb + 4 * g + r];
 #pragma unroll
-          for (int q = 0; q < Q; ++q) hh[rb][q][r] = gelu_f(fmaf(hh[rb][q][r], invh, bo));
+          for (int q = 0; q < Q; ++q) hh[rb][q][r] = gelu_f(fmaf(hh[rb][q][r], uh, bo));
         }
       if (inb) store_acc<CIN, Q>(hh, a.th + b * CIN * hw + pw, hw, yoff);
     }

@@ -193,10 +193,12 @@ int cvn_layernorm_cf_f32(const float* x, int64_t B, int64_t C, int64_t HW, const
  * bias: (Cout) or NULL, residual: (B,Cout,HW) or NULL, res_scale: (Cout) or NULL.
  * y may alias residual.  Channel counts with a matrix-core tile run on the MFMA units: in whole
  * 32-channel chunks as split-fp16 products (each fp32 operand x = x_h + x_l, two fp16 parts rounded to
- * nearest, the weights scaled by a power of two; three fp16 MFMAs accumulating in fp32; relative error per
- * product at most 2^-20.4, 2^-23 rms; a chunk whose activations leave fp16's range falls back to fp32
- * MFMAs), otherwise as fp32 MFMAs; 1 or 3 channels run on a VALU kernel in fp32, as do pixel counts not a
- * multiple of 4 and misaligned buffers except for 64 <-> 128 channels. */
+ * nearest; three fp16 MFMAs accumulating in fp32), weights and, where needed, pixels scaled by powers of two into
+ * fp16's range: an operand is off by at most 2^-22 of itself, or 2^-25 of the pixel's largest activation or 2^-39 of the
+ * matrix' largest weight where that is more (1.1e-7 of the result for 64 channels of any one size; weights
+ * smaller than 2^-17 of the largest one lose accuracy against their own size).  Otherwise as fp32 MFMAs;
+ * 1 or 3 channels run on a VALU kernel in fp32, as do pixel counts not a multiple of 4 and misaligned buffers
+ * except for 64 <-> 128 channels. */
 int cvn_conv1x1_f32(const float* x, int64_t B, int64_t Cin, int64_t HW, const float* weight,
                     const float* bias, int64_t Cout, int act, const float* residual,
                     const float* res_scale, float* y, cvn_stream_t stream);

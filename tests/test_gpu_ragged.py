@@ -1,9 +1,10 @@
 """The channel-mixing kernels on pixel counts that are no multiple of 4, on buffers at any 4-byte alignment, and
 on weights far from 1 (their split-fp16 parts are scaled per matrix), against the fp64 oracle.
 
-Tolerance (relative 2-norm): a split-fp16 product is off by at most 3 * 2^-22 = 7e-7 of itself, with random signs;
-GELU by 3.3e-7 absolute.  Through the three layers of a tail: 3 (7e-7 + 3.3e-7) = 3e-6 at most; fp32 rounding of the
-sums adds 1e-7 each."""
+Tolerance (relative 2-norm): the two operands and the dropped term of a split-fp16 product are off by 2^-22 each,
+3 * 2^-22 = 7e-7 of it, with random signs (2^-25 of the pixel's largest activation for the smaller ones); GELU by
+3.3e-7 absolute.  Through the three layers of a tail: 3 (7e-7 + 3.3e-7) = 3e-6 at most; fp32 rounding of the sums
+adds 1e-7 each."""
 import numpy as np
 import pytest
 import torch
@@ -92,6 +93,59 @@ def test_weight_scale(ws):
     _close(Fh.conv1x1(_t(x), _t(w)), O.conv1x1(x, w, np.zeros(128, np.float32)), ws)
     z = Fh.conv1x1(_t(x), _t(0 * w))
     assert not z.cpu().numpy().any()
+
+
+SPLIT = [(64, 128, 9, 11), (128, 64, 5, 13), (64, 64, 8, 10), (32, 32, 6, 6)]  # ragged, and 16-byte vectors of pixels
+
+
+def _conv_case(ci, co, H, W, seed):
+    r = np.random.default_rng(seed)
+    return r.standard_normal((2, ci, H, W)), (r.standard_normal((co, ci, 1, 1)) / np.sqrt(ci)).astype(np.float32)
+
+
+def _conv(x, w):
+    """On 16-byte aligned buffers (the vector forms)."""
+    from conversenet_amd import functional as Fh
+
+    return Fh.conv1x1(torch.from_numpy(x).to(DEV), torch.from_numpy(w).to(DEV)).cpu().numpy()
+
+
+@pytest.mark.parametrize("ci,co,H,W", SPLIT)
+@pytest.mark.parametrize("sx,sw", [(1e-30, 1), (1e-6, 1), (1e-4, 1), (1e-2, 1), (0.3, 1), (1e5, 1), (1e20, 1e3),
+                                   (1e36, 1e-3), (1e-3, 1e-30)])
+def test_activation_scale(ci, co, H, W, sx, sw):
+    """Activations (and weights with them) whose fp16 parts would vanish or overflow as they are."""
+    x, w = _conv_case(ci, co, H, W, 7)
+    x, w = (sx * x).astype(np.float32), np.float32(sw) * w
+    ref = np.einsum("oc,bchw->bohw", w[:, :, 0, 0].astype(np.float64), x.astype(np.float64))
+    got = _conv(x, w)
+    assert np.isfinite(got).all()
+    assert np.linalg.norm((got - ref) / sx / sw) <= TOL * np.linalg.norm(ref / sx / sw)
+
+
+@pytest.mark.parametrize("ci,co,H,W", SPLIT)
+def test_pixels_and_rows_of_different_size(ci, co, H, W):
+    """Pixels 1e-8 to 1e8, each against its own size (they are scaled one by one); an infinity stays in its pixel, and
+    is one there; output rows 1e-2.5 to 1e2.5 (a matrix has one scale: a row is exact to 2^-22 from 2^-17 of the largest
+    entry on)."""
+    r = np.random.default_rng(8)
+    x, w = _conv_case(ci, co, H, W, 9)
+    x = (x * 10.0 ** r.uniform(-8, 8, (2, 1, H, W))).astype(np.float32)
+    x[0, :, 0, 0] = 0
+    ref = np.einsum("oc,bchw->bohw", w[:, :, 0, 0].astype(np.float64), x.astype(np.float64))
+    got = _conv(x, w)
+    assert not got[0, :, 0, 0].any()
+    assert (np.linalg.norm(got - ref, axis=1) <= TOL * np.linalg.norm(ref, axis=1)).all()
+    x[1, 3, 2, 1] = np.inf
+    got2 = _conv(x, w)
+    assert (got2[1, :, 2, 1] == np.sign(w[:, 3, 0, 0]) * np.inf).all()
+    got2[1, :, 2, 1], ref[1, :, 2, 1] = 0, 0
+    assert (np.linalg.norm(got2 - ref, axis=1) <= TOL * np.linalg.norm(ref, axis=1)).all()
+    x = r.standard_normal((2, ci, H, W)).astype(np.float32)
+    w = (w * 10.0 ** r.uniform(-2.5, 2.5, (co, 1, 1, 1))).astype(np.float32)
+    ref = np.einsum("oc,bchw->bohw", w[:, :, 0, 0].astype(np.float64), x.astype(np.float64))
+    size = lambda a: np.sqrt((a ** 2).sum((0, 2, 3)))  # noqa: E731
+    assert (size(_conv(x, w) - ref) <= TOL * size(ref)).all()
 
 
 @pytest.mark.parametrize("mode,k,pad", [("circular", 7, 6), ("replicate", 5, 4)])

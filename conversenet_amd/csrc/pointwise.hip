@@ -984,9 +984,9 @@ int launch_tail(TailArgs a, int64_t B, hipStream_t st) {
   return check_launch("fused block tail");
 }
 
-// vec: pixel count a multiple of 4 and 16-byte aligned buffers.  Otherwise the shapes whose tile is one
-// pixel per lane anyway, and every LayerNorm shape (there is no other kernel for those), run with ONE; the
-// remaining shapes run on the VALU kernel (*done = false).
+// vec: pixel count a multiple of 4 and 16-byte aligned buffers.  Otherwise the split-fp16 shapes with a LayerNorm
+// (there is no other kernel for those) and those whose tile is one pixel per lane anyway run with ONE; the
+// remaining shapes run on the VALU kernel (*done = false), which has no LayerNorm (16 -> 64 and 128 -> 128: refused).
 template <bool LN>
 int dispatch_mfma(int64_t Cin, int64_t Cout, const float* x, int64_t B, int64_t HW, const float* W,
                   const float* bias, const float* lw, const float* lb, float eps, int act, const float* residual,

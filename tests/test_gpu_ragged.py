@@ -68,6 +68,31 @@ def test_tail(H, W, head):
         _close(out[1], O.gelu(O.conv1x1(O.layernorm_cf(ref, p["lw"], p["lb"], 1e-5), p["w1"], p["b1"])), "head")
 
 
+@pytest.mark.parametrize("H,W", [(1, 1), (15, 17), (7, 37)])
+@pytest.mark.parametrize("C,Cout", [(64, 64), (64, 16), (32, 32), (64, 32), (128, 64)])
+def test_ln_conv_shapes(H, W, C, Cout):
+    """The remaining LayerNorm shapes with split products, one pixel per lane."""
+    from conversenet_amd import functional as Fh
+
+    p = _params(C, Cout, 10 + C + Cout)
+    x = np.random.default_rng(H + C).standard_normal((2, C, H, W)).astype(np.float32)
+    d = {k: _t(v) for k, v in p.items()}
+    got = Fh.conv1x1(_t(x), d["w1"], d["b1"], ln=(d["lw"], d["lb"], 1e-5))
+    _close(got, O.conv1x1(O.layernorm_cf(x, p["lw"], p["lb"], 1e-5), p["w1"], p["b1"]), "ln conv")
+
+
+@pytest.mark.parametrize("H,W", [(1, 1), (8, 9)])
+@pytest.mark.parametrize("C,Cout", [(16, 64), (128, 128)])
+def test_ln_conv_shapes_without_a_ragged_kernel(H, W, C, Cout):
+    """fp32-product LayerNorm shapes: refused on ragged or misaligned input, as before."""
+    from conversenet_amd import functional as Fh
+
+    x, w, v = torch.zeros(1, C, H, W, device=DEV), torch.zeros(Cout, C, 1, 1, device=DEV), torch.ones(C, device=DEV)
+    x = x if H * W % 4 else _t(x.cpu().numpy())
+    with pytest.raises(RuntimeError, match="MFMA tile shape"):
+        Fh.conv1x1(x, w, ln=(v, v, 1e-5))
+
+
 @pytest.mark.parametrize("H,W", SIZES)
 @pytest.mark.parametrize("C,mid", [(64, 128), (32, 64)])
 def test_ln_conv_and_mlp(H, W, C, mid):

@@ -2336,6 +2336,35 @@ extern "C" size_t cvn_converse2d_bwd_workspace(int64_t B, int64_t C, int64_t H, 
   return w.total + kBwdWsAlign;  // slack to align the caller's pointer (cvn_converse2d_bwd_f32)
 }
 
+namespace {
+// 132, 256 and 260 points at scale 1 keep the compile-time kernel, whose dPhi sums stay in registers through its
+// smaller transforms: 340 us against 690 at 260 points and 1024 planes.
+bool bwd_lines(const Geo& g) {
+  if (g.s == 1 && (g.h == 132 || g.h == 256 || g.h == 260)) return false;
+  return lines_cols_bwd_ok(g.P, g.Cp == g.C ? g.B : 1, g.h, g.Hs, g.s, g.NC);
+}
+}  // namespace
+
+extern "C" int cvn_converse2d_column_pass(int call, int64_t B, int64_t C, int64_t H, int64_t W, int64_t psf_batch,
+                                          int scale, int pad) {
+  Geo g;
+  int rc = module_geo(B, C, H, W, psf_batch, 1, 1, scale, pad, &g);
+  if (rc != CVN_OK) return rc;
+  bool lines = false;
+  if (call == CVN_CALL_MODULE) {
+    if (module_ct_supported(g.h, g.w, g.s, g.pad)) return CVN_COLS_PLANNED;
+    lines = lines_cols_ok(g.P, g.h, g.Hs, g.NCs);
+  } else if (call == CVN_CALL_OP) {
+    if (op_ct_supported(g.h, g.w, g.s)) return CVN_COLS_PLANNED;
+    lines = lines_cols_op_ok(g.P, g.h, g.Hs, g.s, g.w);
+  } else if (call == CVN_CALL_BWD) {
+    lines = bwd_lines(g);
+  } else {
+    return fail(CVN_ERR_ARG, "bad call %d", call);
+  }
+  return lines ? CVN_COLS_LINES : CVN_COLS_SINGLE;
+}
+
 extern "C" int cvn_converse2d_bwd_f32(const float* grad_out, const float* x, int64_t B, int64_t C, int64_t H,
                                       int64_t W, const float* psf, int64_t psf_batch, int kh, int kw,
                                       const float* bias, float eps, int scale, int pad, int pad_mode, float* grad_x,
@@ -2376,10 +2405,7 @@ extern "C" int cvn_converse2d_bwd_f32(const float* grad_out, const float* x, int
                 CVN_OK)
     return rc;
   // column pass: dS (in place over Sx) and dPhi
-  // (132, 256 and 260 points at scale 1 keep the compile-time kernel, whose dPhi sums stay in registers
-  // through its smaller transforms: 340 us against 690 at cfg3)
-  const bool ct = g.s == 1 && (g.h == 132 || g.h == 256 || g.h == 260);
-  if (!ct && lines_cols_bwd_ok(g.P, g.Cp == g.C ? g.B : 1, g.h, g.Hs, g.s, g.NC)) {
+  if (bwd_lines(g)) {
     rc = launch_lines_cols_bwd(Sg, Sx, phi, wg ? (float2*)(base + ws.dphi) : nullptr, g.B, g.C, g.Cp / g.C, g.h, g.w,
                                g.s, (const float2*)(tabs + t.off[kTabH]), (const float2*)(tabs + t.off[kTabHs]), st);
     if (rc != CVN_OK) return rc;

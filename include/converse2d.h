@@ -162,6 +162,14 @@ int cvn_converse2d_op_f32(const float* x, const float* x0, int64_t B, int64_t C,
  * code path. */
 enum { CVN_ROUTE_OP_PLANNED = 4 };
 int cvn_converse2d_op_route(int64_t h, int64_t w, int scale);
+/* Which column pass a call on CVN_ROUTE_GENERIC runs, with 16-byte aligned buffers: the forward of a module call, the
+ * operator (H, W: its input plane, pad 0) or the backward, on a psf batch of 1 or B.  CVN_COLS_SINGLE: a
+ * block per few columns or per alias class; CVN_COLS_LINES: blocks of 16 columns of any planes; CVN_COLS_PLANNED:
+ * compile-time plans.  Negative: CVN_ERR_*.  All compute the same solve: for tests and reports. */
+enum { CVN_CALL_MODULE = 0, CVN_CALL_OP = 1, CVN_CALL_BWD = 2 };
+enum { CVN_COLS_SINGLE = 0, CVN_COLS_LINES = 1, CVN_COLS_PLANNED = 2 };
+int cvn_converse2d_column_pass(int call, int64_t B, int64_t C, int64_t H, int64_t W, int64_t psf_batch, int scale,
+                               int pad);
 size_t cvn_converse2d_op_table_bytes(int64_t C, int64_t h, int64_t w, int kh, int kw, int scale);
 size_t cvn_converse2d_op_scratch_bytes(int64_t B, int64_t C, int64_t h, int64_t w, int scale);
 int cvn_converse2d_op_table_f32(const float* psf, int kh, int kw, const float* bias, float eps, int64_t C,

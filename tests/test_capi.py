@@ -179,3 +179,15 @@ def test_noalloc_limit_and_rejection_without_device():
     # invalid geometry: the forward's own argument error
     rc = lib.cvn_converse2d_fwd_noalloc_f32(None, 1, 2, 8, 8, None, 3, 3, 3, None, 1e-5, 1, 1, 3, 0, None, None)
     assert rc == _lib.CVN_ERR_ARG
+
+
+def test_column_pass_query():
+    """Host-side: few alias classes keep the class-per-block pass, a geometry outside the limits its error."""
+    lib = _lib.load()
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_OP, 2, 54, 49, 17, 1, 3, 0) == _lib.COLS_LINES
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_OP, 1, 2, 49, 17, 1, 3, 0) == _lib.COLS_SINGLE
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_OP, 8, 8, 256, 256, 1, 3, 0) == _lib.COLS_PLANNED
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_BWD, 16, 64, 256, 256, 1, 1, 2) == _lib.COLS_SINGLE  # 260 rows
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_BWD, 8, 128, 96, 96, 1, 1, 6) == _lib.COLS_LINES
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_MODULE, 1, 1, 5000, 8, 1, 1, 0) == _lib.CVN_ERR_UNSUPPORTED
+    assert lib.cvn_converse2d_column_pass(3, 1, 1, 8, 8, 1, 1, 0) == _lib.CVN_ERR_ARG

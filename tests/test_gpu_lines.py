@@ -72,22 +72,29 @@ def test_shapes_modes_scales(B, C, H, W, k, s, p, mode, pb):
     _check(x, w, b, s, p, mode, (H, W, s, p))
 
 
-# (B, C, h, w, k, s): enough classes for the lines pass; even and odd w (self-mirrored classes 0 and w / 2),
-# dense and staged lengths, a length (500 rows at s = 2) whose members exceed LDS and stay on the class-per-block pass
+# (B, C, h, w, k, s, lines): even and odd w (self-mirrored classes 0 and w / 2, the middle member of an odd scale),
+# dense and staged lengths, each with classes enough for the lines pass; too few of them, and a length (500 rows at
+# s = 2) whose members exceed LDS, which stay on the class-per-block pass
 OP_CASES = [
-    (2, 40, 21, 37, 3, 1),
-    (3, 33, 15, 26, 3, 2),
-    (2, 30, 49, 17, 5, 3),
-    (2, 80, 10, 12, 7, 4),
-    (1, 97, 37, 31, 2, 2),
-    (2, 4, 250, 44, 3, 2),
+    (2, 40, 21, 37, 3, 1, True),
+    (3, 33, 15, 26, 3, 2, True),
+    (2, 54, 49, 17, 5, 3, True),
+    (2, 40, 9, 24, 3, 3, True),
+    (2, 92, 10, 12, 7, 4, True),
+    (1, 120, 7, 21, 3, 4, True),
+    (1, 97, 37, 31, 2, 2, True),
+    (2, 30, 49, 17, 5, 3, False),
+    (2, 80, 10, 12, 7, 4, False),
+    (2, 14, 250, 44, 3, 2, False),
 ]
 
 
-@pytest.mark.parametrize("B,C,h,w,k,s", OP_CASES)
-def test_operator_arbitrary_x0(B, C, h, w, k, s):
+@pytest.mark.parametrize("B,C,h,w,k,s,lines", OP_CASES)
+def test_operator_arbitrary_x0(B, C, h, w, k, s, lines):
+    from conversenet_amd import _lib
     from conversenet_amd import functional as Fh
 
+    assert _lib.load().cvn_converse2d_column_pass(_lib.CALL_OP, B, C, h, w, 1, s, 0) == int(lines)
     x, psf, b = _inputs(B, C, h, w, k, h * w)
     x0 = np.random.default_rng(w).standard_normal((B, C, h * s, w * s)).astype(np.float32)
     ref = O.converse2d_op_stable(x, x0, psf, b, s, 1e-5)
@@ -96,27 +103,29 @@ def test_operator_arbitrary_x0(B, C, h, w, k, s):
     assert err <= TOL, err
 
 
-# (B, C, H, W, k, s, p, mode, psf batch): several planes per psf and blocks that straddle psf groups
+# (B, C, H, W, k, s, p, mode, psf batch, lines): several planes per psf and blocks that straddle psf groups
 BWD_CASES = [
-    (3, 5, 31, 29, 3, 1, 4, "circular", 1),     # 39 x 37
-    (2, 3, 33, 57, 5, 1, 2, "reflect", 2),      # 37 x 61
-    (4, 3, 94, 43, 3, 1, 3, "replicate", 1),    # 100 x 49
-    (3, 4, 15, 26, 3, 2, 1, "constant", 1),     # 34 x 56
-    (2, 3, 17, 13, 5, 3, 2, "circular", 2),     # 63 x 51
-    (3, 2, 10, 21, 2, 4, 1, "reflect", 1),      # 48 x 92
-    (1, 5, 16, 20, 3, 2, 0, "circular", 1),     # 32 x 40: one plane per psf, the lines pass
-    (2, 60, 14, 110, 3, 2, 0, "circular", 1),   # 28 x 220: blocks for most of the chip, the lines pass
-    (8, 3, 24, 10, 3, 1, 0, "circular", 1),     # 24 x 10: few blocks, a column class or more per block
-    (4, 2, 100, 9, 3, 3, 1, "replicate", 1),    # 306 x 33 (17 a factor): the lines pass at few blocks
-    (3, 3, 70, 9, 3, 3, 0, "constant", 1),      # 210 x 27: few blocks of long columns
+    (3, 5, 31, 29, 3, 1, 4, "circular", 1, True),     # 39 x 37
+    (2, 3, 33, 57, 5, 1, 2, "reflect", 2, True),      # 37 x 61
+    (4, 3, 94, 43, 3, 1, 3, "replicate", 1, True),    # 100 x 49
+    (3, 4, 15, 26, 3, 2, 1, "constant", 1, True),     # 34 x 56
+    (2, 3, 17, 13, 5, 3, 2, "circular", 2, True),     # 63 x 51
+    (3, 2, 10, 21, 2, 4, 1, "reflect", 1, False),      # 48 x 92
+    (1, 5, 16, 20, 3, 2, 0, "circular", 1, True),     # 32 x 40: one plane per psf, the lines pass
+    (2, 60, 14, 110, 3, 2, 0, "circular", 1, True),   # 28 x 220: blocks for most of the chip, the lines pass
+    (8, 3, 24, 10, 3, 1, 0, "circular", 1, False),     # 24 x 10: few blocks, a column class or more per block
+    (4, 2, 100, 9, 3, 3, 1, "replicate", 1, True),    # 306 x 33 (17 a factor): the lines pass at few blocks
+    (3, 3, 70, 9, 3, 3, 0, "constant", 1, False),      # 210 x 27: few blocks of long columns
 ]
 
 
-@pytest.mark.parametrize("B,C,H,W,k,s,p,mode,pb", BWD_CASES)
+@pytest.mark.parametrize("B,C,H,W,k,s,p,mode,pb,lines", BWD_CASES)
 @pytest.mark.parametrize("weights", [True, False])
-def test_backward(B, C, H, W, k, s, p, mode, pb, weights):
+def test_backward(B, C, H, W, k, s, p, mode, pb, lines, weights):
+    from conversenet_amd import _lib
     from conversenet_amd import functional as Fh
 
+    assert _lib.load().cvn_converse2d_column_pass(_lib.CALL_BWD, B, C, H, W, pb, s, p) == int(lines)
     x, w, b = _inputs(B, C, H, W, k, H + W, pb)
     go = np.random.default_rng(W).standard_normal((B, C, H * s, W * s)).astype(np.float32)
     ref = O.converse2d_module_backward(x, w, b, go, s, p, mode, 1e-5)

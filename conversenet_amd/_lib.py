@@ -55,6 +55,7 @@ SIGNATURES = {
     "cvn_converse2d_op_f32": (_int, [_ptr, _ptr, _i64, _i64, _i64, _i64, _ptr, _int, _int, _ptr, _f32, _int, _ptr,
                                      _ptr, _size, _ptr]),
     "cvn_converse2d_op_route": (_int, [_i64, _i64, _int]),
+    "cvn_converse2d_row_pass": (_int, [_i64, _i64, _i64]),
     "cvn_converse2d_column_pass": (_int, [_int, _i64, _i64, _i64, _i64, _i64, _int, _int]),
     "cvn_converse2d_op_table_bytes": (_size, [_i64, _i64, _i64, _int, _int, _int]),
     "cvn_converse2d_op_scratch_bytes": (_size, [_i64, _i64, _i64, _i64, _int]),

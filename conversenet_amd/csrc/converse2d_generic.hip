@@ -12,7 +12,8 @@
 //       X = X0 + conj(K) (tile_s(F(y)) - M(K X0)) / (M(|K|^2) + lambda),   out = Re F^-1(X).
 //
 // Kernels:
-//   (row and module column passes of lengths up to 1024: converse2d_lines.hip, on the same scratch and tables)
+//   (row and module column passes of lengths up to 1024 run in converse2d_lines.hip, on the same scratch and tables,
+//   except where its blocks are too few: lines_rows_ok, lines_cols_ok)
 //   k_phi_module / k_phi_op : transfer tables in fp64 (one block per channel column class)
 //   k_rows_fwd               : padding on load, R2C along rows (two real rows per complex FFT),
 //                              writes the half spectrum column-major  S[plane][col][row]
@@ -799,9 +800,11 @@ struct RowFwdArgs {
   float2* S;       // (P, NC, h)
 };
 
+// LC > 0: the row length a.w, fixed at compile time (fft_fixed_ct; constant index arithmetic).
+template <int LC>
 __global__ void __launch_bounds__(256) k_rows_fwd(RowFwdArgs a) {
   extern __shared__ float2 sm[];
-  const int L = a.w, ntr = a.rpb / 2, ld = L + 2;
+  const int L = LC > 0 ? LC : a.w, ntr = a.rpb / 2, ld = L + 2;
   float2* tw = sm;
   float2* A = tw + L;
   float2* Bf = A + ntr * ld;
@@ -809,10 +812,63 @@ __global__ void __launch_bounds__(256) k_rows_fwd(RowFwdArgs a) {
   const int r0 = blockIdx.x * a.rpb;
   const int tid = threadIdx.x, nth = blockDim.x;
   char* rad = (char*)sm + a.rad_off;
-  load_plan_tabs(a.plan, a.tabs, tw, rad, tid, nth);
+  if constexpr (LC > 0) {  // the twiddles only (no Rader stage at these lengths)
+    const float2* gt = (const float2*)a.tabs;
+    for (int m = tid; m < LC; m += nth) tw[m] = gt[m];
+  } else {
+    load_plan_tabs(a.plan, a.tabs, tw, rad, tid, nth);
+  }
   const float* xp = a.x + plane * (int64_t)a.Hin * a.Win;
   const FastDiv fL = fast_div(L), frpb = fast_div(a.rpb);
-  for (int i0 = tid; i0 < ntr * L; i0 += kBatch * nth) {
+  // Compile-time length with 16-byte aligned rows of a multiple of 4 samples: the interior of each
+  // row as float4 loads (one row index map per item instead of three per sample), then the 2 pad
+  // border columns per row from their padding sources
+  const bool vec4 = LC > 0 && a.Win % 4 == 0 && ((uintptr_t)a.x & 15) == 0 && a.Win + 2 * a.pad == L;
+  if (vec4) {
+    const int W4 = a.Win >> 2, nI = ntr * W4, nb = 2 * a.pad;
+    const FastDiv fW4 = fast_div(W4);
+    for (int i0 = tid; i0 < nI; i0 += kBatch * nth) {
+      float4 va[kBatch], vb[kBatch];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        const int idx = i0 + k * nth;
+        va[k] = vb[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (idx < nI) {
+          const int t = idx / fW4, q = idx - t * W4;
+          const int ra = r0 + 2 * t, rb = ra + 1;
+          const int sa = ra < a.h ? pad_src(ra, a.Hin, a.pad, a.mode) : -1;
+          const int sb = rb < a.h ? pad_src(rb, a.Hin, a.pad, a.mode) : -1;
+          if (sa >= 0) va[k] = *(const float4*)(xp + (int64_t)sa * a.Win + 4 * q);
+          if (sb >= 0) vb[k] = *(const float4*)(xp + (int64_t)sb * a.Win + 4 * q);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        const int idx = i0 + k * nth;
+        if (idx < nI) {
+          const int t = idx / fW4, q = idx - t * W4;
+          float2* d = A + t * L + a.pad + 4 * q;
+          d[0] = make_float2(va[k].x, vb[k].x);
+          d[1] = make_float2(va[k].y, vb[k].y);
+          d[2] = make_float2(va[k].z, vb[k].z);
+          d[3] = make_float2(va[k].w, vb[k].w);
+        }
+      }
+    }
+    for (int idx = tid; idx < ntr * nb; idx += nth) {
+      const int t = idx / nb, e = idx - t * nb;
+      const int c = e < a.pad ? e : a.Win + e;  // border column of the padded row
+      const int ra = r0 + 2 * t, rb = ra + 1;
+      const int sc = pad_src(c, a.Win, a.pad, a.mode);
+      const int sa = ra < a.h ? pad_src(ra, a.Hin, a.pad, a.mode) : -1;
+      const int sb = rb < a.h ? pad_src(rb, a.Hin, a.pad, a.mode) : -1;
+      float2 v = make_float2(0.f, 0.f);
+      if (sc >= 0 && sa >= 0) v.x = xp[(int64_t)sa * a.Win + sc];
+      if (sc >= 0 && sb >= 0) v.y = xp[(int64_t)sb * a.Win + sc];
+      A[t * L + c] = v;
+    }
+  }
+  for (int i0 = vec4 ? ntr * L : tid; i0 < ntr * L; i0 += kBatch * nth) {
     float2 v[kBatch];
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) {
@@ -841,7 +897,9 @@ __global__ void __launch_bounds__(256) k_rows_fwd(RowFwdArgs a) {
     }
   }
   __syncthreads();
-  const float2* Z = fft_lds<false>(a.plan, A, Bf, ntr, tw, tid, nth, rad);
+  const float2* Z;
+  if constexpr (LC > 0) Z = fft_fixed_ct<LC, 0, false>(A, Bf, ntr, tw, tid, nth);
+  else Z = fft_lds<false>(a.plan, A, Bf, ntr, tw, tid, nth, rad);
   // unpack two real rows: Ya = (Z[c] + conj Z[-c]) / 2, Yb = (Z[c] - conj Z[-c]) / (2i)
   float2* Sp = a.S + plane * (int64_t)a.NC * a.h;
   for (int idx = tid; idx < a.NC * a.rpb; idx += nth) {
@@ -1050,17 +1108,23 @@ struct RowInvArgs {
   int rad_off;       // byte offset of the plan's Rader tables in LDS
 };
 
+template <int LC>  // LC > 0: the row length a.Ws, fixed at compile time
 __global__ void __launch_bounds__(256) k_rows_inv(RowInvArgs a) {
   extern __shared__ float2 sm[];
   const int tid = threadIdx.x, nth = blockDim.x;
-  const int L = a.Ws, ntr = a.rpb / 2, ld = L + 2;
+  const int L = LC > 0 ? LC : a.Ws, ntr = a.rpb / 2, ld = L + 2;
   float2* tw = sm;
   float2* A = tw + L;
   float2* Bf = A + ntr * ld;
   const int64_t plane = blockIdx.y;
   const int r0 = blockIdx.x * a.rpb;  // local output row
   char* rad = (char*)sm + a.rad_off;
-  load_plan_tabs(a.plan, a.tabs, tw, rad, tid, nth);
+  if constexpr (LC > 0) {  // the twiddles only (no Rader stage at these lengths)
+    const float2* gt = (const float2*)a.tabs;
+    for (int m = tid; m < LC; m += nth) tw[m] = gt[m];
+  } else {
+    load_plan_tabs(a.plan, a.tabs, tw, rad, tid, nth);
+  }
   int* csrc = (int*)((char*)sm + a.csrc_off);
   if (a.pad >= 0 && a.pmode != CVN_PAD_ZEROS)
     for (int q = tid; q < 2 * a.pad; q += nth)
@@ -1099,7 +1163,9 @@ __global__ void __launch_bounds__(256) k_rows_inv(RowInvArgs a) {
     A[t * L + v] = make_float2(ha.x - hb.y, ha.y + hb.x);
   }
   __syncthreads();
-  const float2* Z = fft_lds<true>(a.plan, A, Bf, ntr, tw, tid, nth, rad);
+  const float2* Z;
+  if constexpr (LC > 0) Z = fft_fixed_ct<LC, 0, true>(A, Bf, ntr, tw, tid, nth);
+  else Z = fft_lds<true>(a.plan, A, Bf, ntr, tw, tid, nth, rad);
   if (a.pad >= 0) {
     const int pad = a.pad, Hd = a.nrows - 2 * pad, Wd = a.ncols - 2 * pad;
     const int nb = (a.pmode == CVN_PAD_ZEROS) ? 0 : 2 * pad;
@@ -1114,13 +1180,42 @@ __global__ void __launch_bounds__(256) k_rows_inv(RowInvArgs a) {
         a.side[(plane * nb + (r < pad ? r : r - Hd)) * (int64_t)Wd + j] = v;
     };
     if (!all_edge) {
-      const int j0 = nb > 0 ? pad + 1 : 0, nrest = (nb > 0 ? Wd - 1 - pad : Wd) - j0;  // non-edge columns
-      const FastDiv fr = fast_div(nrest);
-      for (int idx = tid; idx < a.rpb * nrest; idx += nth) {
-        const int rl = idx / fr, j = j0 + idx - rl * nrest;
-        if (r0 + rl >= a.nrows) continue;
-        const float2 z = Z[(rl >> 1) * L + j + pad];
-        put(rl, j, (rl & 1) ? z.y : z.x);
+      // non-edge columns [j0, j1): with a compile-time length and 16-byte aligned rows, the aligned
+      // middle [jb0, jb1) as float4 stores and the rest one sample at a time
+      const int j0 = nb > 0 ? pad + 1 : 0, j1 = nb > 0 ? Wd - 1 - pad : Wd;
+      int jb0 = j0, jb1 = j0;
+      if (LC > 0 && Wd % 4 == 0 && ((uintptr_t)a.out & 15) == 0 && ((uintptr_t)a.side & 15) == 0) {
+        jb0 = (j0 + 3) & ~3;
+        jb1 = j1 & ~3;
+        if (jb1 < jb0) jb1 = jb0;
+      }
+      const int nq = (jb1 - jb0) >> 2;
+      if (nq > 0) {
+        const FastDiv fq = fast_div(nq);
+        for (int idx = tid; idx < a.rpb * nq; idx += nth) {
+          const int rl = idx / fq, q = idx - rl * nq;
+          const int r = r0 + rl;
+          if (r >= a.nrows) continue;
+          const int j = jb0 + 4 * q;
+          const float2* zr = Z + (rl >> 1) * L + j + pad;
+          const float4 v = (rl & 1) ? make_float4(zr[0].y, zr[1].y, zr[2].y, zr[3].y)
+                                    : make_float4(zr[0].x, zr[1].x, zr[2].x, zr[3].x);
+          float* dst = (r >= pad && r < pad + Hd) ? a.out + (plane * Hd + (r - pad)) * (int64_t)Wd + j
+                       : (nb > 0 ? a.side + (plane * nb + (r < pad ? r : r - Hd)) * (int64_t)Wd + j : nullptr);
+          if (dst) *(float4*)dst = v;
+        }
+      }
+      const int nrest = (j1 - j0) - 4 * nq;  // columns [j0, jb0) and [jb1, j1)
+      if (nrest > 0) {
+        const FastDiv fr = fast_div(nrest);
+        const int nh = jb0 - j0;
+        for (int idx = tid; idx < a.rpb * nrest; idx += nth) {
+          const int rl = idx / fr, e = idx - rl * nrest;
+          if (r0 + rl >= a.nrows) continue;
+          const int j = e < nh ? j0 + e : jb1 + (e - nh);
+          const float2 z = Z[(rl >> 1) * L + j + pad];
+          put(rl, j, (rl & 1) ? z.y : z.x);
+        }
       }
     }
     for (int idx = tid; idx < a.rpb * ne; idx += nth) {
@@ -1706,7 +1801,9 @@ constexpr size_t kLdsLimit = 160 * 1024;
 std::atomic<uint64_t> g_attr_done{0};
 void set_lds_attrs() {
   once_per_device(g_attr_done, [] {
-    for (const void* k : {(const void*)k_rows_fwd, (const void*)k_rows_inv, (const void*)k_cols_bwd<0>,
+    for (const void* k : {(const void*)k_rows_fwd<0>, (const void*)k_rows_fwd<132>, (const void*)k_rows_fwd<256>,
+                          (const void*)k_rows_fwd<260>, (const void*)k_rows_inv<0>, (const void*)k_rows_inv<132>,
+                          (const void*)k_rows_inv<256>, (const void*)k_rows_inv<260>, (const void*)k_cols_bwd<0>,
                           (const void*)k_cols_bwd<132>, (const void*)k_cols_bwd<256>, (const void*)k_cols_bwd<260>})
       (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
     (void)hipFuncSetAttribute((const void*)k_cols_module, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
@@ -1878,7 +1975,7 @@ int launch_phi(const float* psf, const float* bias, float eps, const Geo& g, boo
 
 int launch_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, int mode, int h, int w,
                     const char* tabs, float2* S, hipStream_t st) {
-  if (lines_rows_ok(P, h, w))  // lengths up to 1024: this kernel took 214 us where that one takes 58 (128 planes 333 x 493)
+  if (lines_rows_ok(P, h, w))  // (128 planes 333 x 493: this kernel 214 us, that one 58)
     return launch_lines_rows_fwd(x, P, Hin, Win, pad, mode, h, w, (const float2*)tabs, S, st);
   RowFwdArgs a;
   a.x = x; a.Hin = Hin; a.Win = Win; a.h = h; a.w = w; a.pad = pad; a.mode = mode;
@@ -1890,7 +1987,12 @@ int launch_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, int mo
   a.S = S;
   dim3 grid((h + a.rpb - 1) / a.rpb, (unsigned)P);
   const size_t lds = a.rad_off + rader_lds_bytes(a.plan);
-  hipLaunchKernelGGL(k_rows_fwd, grid, dim3(kThreads), lds, st, a);
+  switch (w) {  // lengths with a compile-time plan
+    case 132: hipLaunchKernelGGL(k_rows_fwd<132>, grid, dim3(kThreads), lds, st, a); break;
+    case 256: hipLaunchKernelGGL(k_rows_fwd<256>, grid, dim3(kThreads), lds, st, a); break;
+    case 260: hipLaunchKernelGGL(k_rows_fwd<260>, grid, dim3(kThreads), lds, st, a); break;
+    default: hipLaunchKernelGGL(k_rows_fwd<0>, grid, dim3(kThreads), lds, st, a); break;
+  }
   return check_launch("row forward pass");
 }
 
@@ -1911,7 +2013,12 @@ int launch_rows_inv(const float2* SH, const Geo& g, int row0, int nrows, int col
   a.tabs = tabs;
   dim3 grid((nrows + a.rpb - 1) / a.rpb, (unsigned)g.P);
   const size_t lds = a.csrc_off + sizeof(int) * 2 * std::max(pad, 0);
-  hipLaunchKernelGGL(k_rows_inv, grid, dim3(kThreads), lds, st, a);
+  switch (g.Ws) {  // lengths with a compile-time plan
+    case 132: hipLaunchKernelGGL(k_rows_inv<132>, grid, dim3(kThreads), lds, st, a); break;
+    case 256: hipLaunchKernelGGL(k_rows_inv<256>, grid, dim3(kThreads), lds, st, a); break;
+    case 260: hipLaunchKernelGGL(k_rows_inv<260>, grid, dim3(kThreads), lds, st, a); break;
+    default: hipLaunchKernelGGL(k_rows_inv<0>, grid, dim3(kThreads), lds, st, a); break;
+  }
   return check_launch("row inverse pass");
 }
 
@@ -2344,6 +2451,12 @@ bool bwd_lines(const Geo& g) {
   return lines_cols_bwd_ok(g.P, g.Cp == g.C ? g.B : 1, g.h, g.Hs, g.s, g.NC);
 }
 }  // namespace
+
+extern "C" int cvn_converse2d_row_pass(int64_t planes, int64_t h, int64_t w) {
+  if (planes < 1 || h < 1 || w < 1 || h > kMaxFftLen || w > kMaxFftLen)
+    return fail(CVN_ERR_ARG, "bad shape");
+  return lines_rows_ok(planes, (int)h, (int)w) ? CVN_COLS_LINES : CVN_COLS_SINGLE;
+}
 
 extern "C" int cvn_converse2d_column_pass(int call, int64_t B, int64_t C, int64_t H, int64_t W, int64_t psf_batch,
                                           int scale, int pad) {

@@ -671,11 +671,15 @@ void line_attrs() {
   });
 }
 
+constexpr int kCus = 256;  // compute units of the device
+
 // Threads per block.  The kernels take up to 128 VGPRs, so a CU holds 16 waves.  Measured over 27 lengths
 // from 24 to 560 (1 to 16 waves per block): a power of two near one wave per 64 elements of length (16
 // elements per thread) is the fastest or within 6 % of it, and an uneven share of the 16 waves (3, 5) up to
 // 30 % slower.  Where the blocks are too few to fill the chip, waves are doubled while all blocks stay
-// resident and the widest pass still gives every wave a butterfly per lane (64 planes of 136 x 136: 37 -> 28 us).
+// resident and the widest pass still gives every wave a butterfly per lane (64 planes of 136 x 136: 37 -> 28 us), or,
+// for the loads and stores, a thread has 4 elements or more (a call on 2 to 64 planes of 16 to 264 rows or columns of
+// 64: 1 to 3 us of 20 to 27 us less; 2 elements: 0.5 us more than 4).
 // lds: the block's LDS, where it holds more than one line buffer (fewer blocks per CU, more waves each).
 int line_threads(const LinePlan& p, int nblk, size_t lds = 0) {
   int w = 1, most = 1;
@@ -683,13 +687,47 @@ int line_threads(const LinePlan& p, int nblk, size_t lds = 0) {
   for (int t = 0; t < p.np; ++t) most = std::max(most, p.ps[t].nl * kLines);
   if (lds) most = std::max(most, p.L * 8);  // the product's items
   while (lds && 2 * w * (int)(kLineLds / lds) <= 16 && 64 * w < most) w *= 2;
-  while (2 * w <= 16 && (int64_t)nblk * 2 * w <= 256 * 16 && 64 * w < most) w *= 2;
+  most = std::max(most, p.L * kLines / 4);
+  while (2 * w <= 16 && (int64_t)nblk * 2 * w <= kCus * 16 && 64 * w < most) w *= 2;
   return std::max(64 * w, line_min_threads(p));
+}
+
+// Whether the runtime-plan passes' transform of length L has no prime above 13: with one, they are never the faster
+// (136 = 8 17: 1.8 times this engine's time at any number of blocks).
+bool plain_plan(int L) {
+  const FftPlan* p = fft_plan(L);
+  if (!p) return false;
+  for (int i = 0; i < p->nst; ++i)
+    if (p->radix[i] > 13) return false;
+  return true;
+}
+
+// Butterflies of the widest radix.
+int narrowest(const LinePlan& p) {
+  int n = p.L;
+  for (int t = 0; t < p.np; ++t) n = std::min(n, p.ps[t].nl);
+  return n;
 }
 
 }  // namespace
 
-bool lines_rows_ok(int64_t P, int h, int w) { return line_plan(w) && P * ((h + 1) / 2) < (1 << 30); }
+// Rows of lengths up to 1024, except where the blocks leave much of the chip idle and the runtime-plan pass, with 2 to 8
+// rows to a block instead of 32, is the faster one (two row passes and a column pass of 64 rows, us, that / this):
+//   one or two butterflies per line, so that most of a block idles: rows of 24: 18.7 / 19.3, 32: 19.2 / 21.2, 50:
+//     21.2 / 22.3 (of 16: 18.4 / 18.4; three of 48: 20.7 / 19.9); at 128 blocks 19.5 / 19.9, 20.0 / 21.2, 22.3 / 22.3, at 256
+//     20.8 / 19.6, 21.5 / 20.9, 24.6 / 22.6;
+//   the lengths with a compile-time form of that pass: 132: 19.5 / 22.4, 256: 22.8 / 24.6, 260: 22.4 / 24.9; at 128
+//     blocks 21.9 / 23.4, 27.5 / 26.7, 30.0 / 27.1; at 192 23.8 / 23.9, 32.7 / 27.8, 34.7 / 28.3;
+//   long rows in few blocks, one per CU: 640: 31.2 / 33.2, 768: 29.0 / 35.2, 1024: 31.6 / 37.5 (600: 31.7 / 32.0); at 48
+//     blocks 40.3 / 35.2, 42.2 / 37.8, 49.3 / 40.8.
+bool lines_rows_ok(int64_t P, int h, int w) {
+  const LinePlan* p = line_plan(w);
+  const int64_t lines = P * ((h + 1) / 2), nblk = (lines + kLines - 1) / kLines;
+  if (!p || lines >= (1 << 30)) return false;
+  const bool few = narrowest(*p) <= 2 ? 4 * nblk < 3 * kCus
+                   : w == 132 || w == 256 || w == 260 ? nblk * w < 100 * kCus : w >= 640 && 8 * nblk < kCus;
+  return !few || !plain_plan(w);
+}
 
 int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, int mode, int h, int w,
                           const float2* tw, float2* S, hipStream_t st) {
@@ -709,8 +747,15 @@ int launch_lines_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, 
   return check_launch("row forward pass");
 }
 
+// Columns that fit the LDS, except long ones in few blocks, where k_cols_module has more and smaller ones (a call of
+// 64 columns of the length at scale 1, us, that / this): 512: 27.8 / 33.5, 768: 28.9 / 40.4, 1024: 30.6 / 45.3, at 50 blocks
+// 31.3 / 34.9, 35.5 / 43.1, 39.8 / 48.8, at 132 blocks 43.7 / 40.2, 57.4 / 52.3, 64.4 / 60.0; with other factors only from 900
+// on: 800 30.9 / 30.6, 1000 32.1 / 38.2, at 50 blocks 37.5 / 32.3, 40.4 / 40.8.
 bool lines_cols_ok(int64_t P, int h, int Hs, int NCs) {
   if (!line_plan(h) || !line_plan(Hs) || P * NCs >= (1 << 30)) return false;
+  const int64_t nblk = (P * NCs + kLines - 1) / kLines;
+  if ((Hs % 128 == 0 ? Hs >= 512 && 8 * nblk < 3 * kCus : Hs >= 900 && 8 * nblk < kCus) && plain_plan(h) && plain_plan(Hs))
+    return false;
   return line_buf_bytes(Hs) + line_tab_bytes(*line_plan(h)) + line_tab_bytes(*line_plan(Hs)) +
                  3 * kLines * sizeof(int64_t) <= kLineLds;
 }
@@ -759,15 +804,10 @@ namespace {
 //     B 16 200 / 210), or at few blocks of long columns (320 rows, 42 blocks, B 4 125 / 134); otherwise 36 rows, 38
 //     blocks, B 16 180 / 160; 120 rows, 62 blocks, B 16 235 / 217; 200 rows 282 / 288.
 bool few_bwd_blocks(int64_t nblk, int64_t nplanes, int h, int s) {
-  const FftPlan *p = fft_plan(h), *pH = fft_plan(h * s);
-  if (!p || !pH) return false;
-  for (const FftPlan* q : {p, pH})
-    for (int i = 0; i < q->nst; ++i)
-      if (q->radix[i] > 13) return false;
+  const FftPlan* p = fft_plan(h);
+  if (!plain_plan(h) || !plain_plan(h * s)) return false;
   if (s > 1) return nblk < (h * s <= 192 ? 200 : 100) && nplanes > 1;
-  int narrow = h;  // butterflies of the widest radix
-  const LinePlan* lp = line_plan(h);
-  for (int t = 0; t < lp->np; ++t) narrow = std::min(narrow, lp->ps[t].nl);
+  const int narrow = narrowest(*line_plan(h));
   return (nblk < 100 && nplanes >= 8 && (narrow < 4 || p->nst <= 2)) ||
          (nblk < 50 && nplanes >= 4 && (narrow < 4 || h >= 256));
 }

@@ -170,6 +170,9 @@ enum { CVN_CALL_MODULE = 0, CVN_CALL_OP = 1, CVN_CALL_BWD = 2 };
 enum { CVN_COLS_SINGLE = 0, CVN_COLS_LINES = 1, CVN_COLS_PLANNED = 2 };
 int cvn_converse2d_column_pass(int call, int64_t B, int64_t C, int64_t H, int64_t W, int64_t psf_batch, int scale,
                                int pad);
+/* The same for a row pass over planes of h rows of w samples (padded, at the pass's scale): CVN_COLS_LINES (blocks of 16
+ * row pairs of any planes) or CVN_COLS_SINGLE (blocks of a few rows of one plane). */
+int cvn_converse2d_row_pass(int64_t planes, int64_t h, int64_t w);
 size_t cvn_converse2d_op_table_bytes(int64_t C, int64_t h, int64_t w, int kh, int kw, int scale);
 size_t cvn_converse2d_op_scratch_bytes(int64_t B, int64_t C, int64_t h, int64_t w, int scale);
 int cvn_converse2d_op_table_f32(const float* psf, int kh, int kw, const float* bias, float eps, int64_t C,

@@ -191,3 +191,11 @@ def test_column_pass_query():
     assert lib.cvn_converse2d_column_pass(_lib.CALL_BWD, 8, 128, 96, 96, 1, 1, 6) == _lib.COLS_LINES
     assert lib.cvn_converse2d_column_pass(_lib.CALL_MODULE, 1, 1, 5000, 8, 1, 1, 0) == _lib.CVN_ERR_UNSUPPORTED
     assert lib.cvn_converse2d_column_pass(3, 1, 1, 8, 8, 1, 1, 0) == _lib.CVN_ERR_ARG
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_MODULE, 1, 3, 1024, 64, 1, 1, 0) == _lib.COLS_SINGLE  # 7 blocks
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_MODULE, 1, 64, 1024, 64, 1, 1, 0) == _lib.COLS_LINES
+    assert lib.cvn_converse2d_column_pass(_lib.CALL_MODULE, 1, 3, 1003, 64, 1, 1, 0) == _lib.COLS_LINES  # 17 59
+    for w, few, many in ((32, 95, 96), (260, 49, 50), (768, 15, 16), (100, 0, 1), (34, 0, 1)):
+        # (64 rows: two blocks a plane)
+        assert few == 0 or lib.cvn_converse2d_row_pass(few, 64, w) == _lib.COLS_SINGLE, w
+        assert lib.cvn_converse2d_row_pass(many, 64, w) == _lib.COLS_LINES, w
+    assert lib.cvn_converse2d_row_pass(1, 0, 8) == _lib.CVN_ERR_ARG

@@ -47,6 +47,37 @@ def test_every_length(first):
             _check(x, w, b, 1, 0, "circular", (H, W))
 
 
+@pytest.mark.parametrize("part", range(4))
+def test_lengths_with_a_kernel_for_few_blocks(part):
+    """Lengths whose rows or columns run on another kernel at two planes, on enough planes for this one, and on the
+    largest number that keeps the other."""
+    from conversenet_amd import _lib
+
+    lib = _lib.load()
+
+    def cols(P, L):
+        return lib.cvn_converse2d_column_pass(_lib.CALL_MODULE, 1, P, L, 3, 1, 1, 0)
+
+    def rows(P, L):
+        return lib.cvn_converse2d_row_pass(P, 1, L)
+
+    seen = [0, 0]
+    for L in range(1 + part, 1025, 4):
+        for n, (kernel, H, W) in enumerate(((rows, 1, L), (cols, L, 3))):
+            if kernel(2, L) == _lib.COLS_LINES:
+                continue
+            lo, hi = 2, 4096  # the last count on the other kernel, the first on this one
+            while hi - lo > 1:
+                mid = (lo + hi) // 2
+                lo, hi = (mid, hi) if kernel(mid, L) == _lib.COLS_SINGLE else (lo, mid)
+            assert kernel(hi, L) == _lib.COLS_LINES
+            seen[n] += 1
+            for P in (lo, hi):
+                x, w, b = _inputs(1, P, H, W, 1, L)
+                _check(x, w, b, 1, 0, "circular", (P, H, W))
+    assert min(seen) >= 1
+
+
 # (B, C, H, W, k, s, p, mode, psf batch): blocks that straddle planes and channels, odd rows and crops, a
 # mirrored LR column at s > 1, dense primes (37, 61, 127) and staged parts (49, 64, 81, 343) in both directions
 CASES = [

@@ -297,8 +297,7 @@ __device__ __forceinline__ int64_t tile_px(int64_t t, int64_t tpb, int Q, int NW
 // is (gemm_f16s).  The operands' error is then the larger of 2^-22 of the value itself and, for activations, 2^-25 of
 // the pixel's largest, for weights 2^-39 of the matrix' largest.  (Activations as they are, whatever their size:
 // a relative error of 1.7e-6 for values of 1e-2 and 1.7e-2 for 1e-6, now 1.1e-7 for all.  With none scaled the
-// 8 x 64 x 256 x 256 tail with a head takes 234 us, 230 before the check; with all scaled 233; 128 -> 64 alone 78,
-// 75 before, when a chunk of channels did not wait for the others' loads.)
+// 8 x 64 x 256 x 256 tail with a head takes 234 us, 230 before the check; with all scaled 233.)
 // Operand layout of the 16x16x32 MFMA: lane l = 16 g + j holds A[row j][k = 8 g + e] and
 // B[k = 8 g + e][col j], e < 8; D as for the fp32 MFMAs (lane 16 g + j: rows 4 g + r, col j).  The k
 // slot 8 g + e (e = 4 hf + r) of input chunk c is channel 16 (2 c + hf) + 4 g + r: the channels lane
@@ -398,79 +397,106 @@ __device__ __forceinline__ uint32_t any_group(uint64_t ballot) {
 // or 1.  Pixels whose largest activation is inside [1, 65504] enter as they are: the low parts are off by at worst
 // 2^-25.  If a pixel of the wave is outside, each one is scaled by the power of two that brings
 // its largest activation to [2^14, 2^15), and the sums are scaled back by both factors at once.
-template <int K, int N, int Q>
+// STREAM: v is on its way from memory.  If the first 32 channels already hold an activation of 1 or more for every pixel,
+// the products start with them, before the other channels have arrived; a later one above 65504 starts them over.
+// (128 -> 64 channels at 4 x 256 x 256: 42.5 us without, 38 with; the tail's first layer, beside three more, and 64
+// channels gain nothing.)
+template <int K, int N, int Q, bool STREAM = false>
 __device__ __forceinline__ float gemm_f16s(v4f (&v)[K / 16][Q], const _Float16* Wl, int lane, float inv,
                                            v4f (&acc)[N / 16][Q]) {
-  bool plain = true, inf = false;
+  bool whole = true, plain = true, inf = false;  // whole: all channels are looked at first
   int back[Q];
-#pragma unroll
-  for (int q = 0; q < Q; ++q) {
-    float m = 0.f;
-#pragma unroll
-    for (int rb = 0; rb < K / 16; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[rb][q][r]));  // (a NaN is left out and stays one)
-    const uint32_t any = any_group(__builtin_amdgcn_ballot_w64(m > 0.f));
-    const uint32_t fit = any_group(__builtin_amdgcn_ballot_w64(m >= 1.f));
-    plain = plain && (any & ~fit) == 0 && __builtin_amdgcn_ballot_w64(m > kF16Max) == 0;
-  }
-  if (!plain) {
+  if constexpr (STREAM) {
+    whole = false;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       float m = 0.f;
 #pragma unroll
-      for (int rb = 0; rb < K / 16; ++rb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[rb][q][r]));
-      m = fmaxf(m, __shfl_xor(m, 16));
-      m = fmaxf(m, __shfl_xor(m, 32));
-      const int e2 = (int)(__float_as_uint(m) >> 23) - 127, s = m > 0.f ? min(14 - e2, 126) : 0;
-      inf = inf || __builtin_amdgcn_ballot_w64(e2 == 128) != 0;
-      back[q] = (int)(__float_as_uint(inv) >> 23) - 127 - s;
-      const float sc = ldexpf(1.f, s);
-#pragma unroll
-      for (int rb = 0; rb < K / 16; ++rb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[rb][q][r] *= sc;
+      for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(v[e >> 2][q][e & 3]));
+      whole = whole || any_group(__builtin_amdgcn_ballot_w64(m >= 1.f)) != 0xffff;
     }
   }
+  for (;;) {
+    if (whole) {
 #pragma unroll
-  for (int c = 0; c < K / 32; ++c) {
-    float xb[Q][8];
+      for (int q = 0; q < Q; ++q) {
+        float m = 0.f;
 #pragma unroll
-    for (int q = 0; q < Q; ++q)
+        for (int rb = 0; rb < K / 16; ++rb)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) xb[q][e] = v[2 * c + (e >> 2)][q][e & 3];
-    if (!inf) {
-      f16x8 bh[Q], bl[Q];
-#pragma unroll
-      for (int q = 0; q < Q; ++q) split_f16(xb[q], bh[q], bl[q]);
-#pragma unroll
-      for (int ob = 0; ob < N / 16; ++ob) {
-        const u32x4_t* wp = (const u32x4_t*)(Wl + (c * (N / 16) + ob) * 1024) + lane;
-        const f16x8 ah = __builtin_bit_cast(f16x8, wp[0]), al = __builtin_bit_cast(f16x8, wp[64]);
+          for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[rb][q][r]));  // (a NaN is left out and stays one)
+        const uint32_t any = any_group(__builtin_amdgcn_ballot_w64(m > 0.f));
+        const uint32_t fit = any_group(__builtin_amdgcn_ballot_w64(m >= 1.f));
+        plain = plain && (any & ~fit) == 0 && __builtin_amdgcn_ballot_w64(m > kF16Max) == 0;
+      }
+      if (!plain) {
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-          v4f t = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[q], acc[ob][q], 0, 0, 0);
-          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[q], t, 0, 0, 0);
-          acc[ob][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[q], t, 0, 0, 0);
+          float m = 0.f;
+#pragma unroll
+          for (int rb = 0; rb < K / 16; ++rb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[rb][q][r]));
+          m = fmaxf(m, __shfl_xor(m, 16));
+          m = fmaxf(m, __shfl_xor(m, 32));
+          const int e2 = (int)(__float_as_uint(m) >> 23) - 127, s = m > 0.f ? min(14 - e2, 126) : 0;
+          inf = inf || __builtin_amdgcn_ballot_w64(e2 == 128) != 0;
+          back[q] = (int)(__float_as_uint(inv) >> 23) - 127 - s;
+          const float sc = ldexpf(1.f, s);
+#pragma unroll
+          for (int rb = 0; rb < K / 16; ++rb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[rb][q][r] *= sc;
         }
-        mem_fence_sched();
-      }
-    } else {  // an infinity has no low part: the wave's products on the fp32 matrix cores
-#pragma unroll
-      for (int ob = 0; ob < N / 16; ++ob) {
-        const u32x4_t* wp = (const u32x4_t*)(Wl + (c * (N / 16) + ob) * 1024) + lane;
-        const f16x8 ah = __builtin_bit_cast(f16x8, wp[0]), al = __builtin_bit_cast(f16x8, wp[64]);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float w = (float)ah[e] + (float)al[e];  // (scaled like the fp16 products)
-#pragma unroll
-          for (int q = 0; q < Q; ++q) acc[ob][q] = mfma4(w, xb[q][e], acc[ob][q]);
-        }
-        mem_fence_sched();
       }
     }
+    bool over = false;
+#pragma unroll
+    for (int c = 0; c < K / 32; ++c) {
+      float xb[Q][8];
+      float mx = 0.f;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          xb[q][e] = v[2 * c + (e >> 2)][q][e & 3];
+          if (STREAM) mx = fmaxf(mx, fabsf(xb[q][e]));
+        }
+      if (STREAM) over = over || __builtin_amdgcn_ballot_w64(mx > kF16Max) != 0;
+      if (!inf) {
+        f16x8 bh[Q], bl[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) split_f16(xb[q], bh[q], bl[q]);
+#pragma unroll
+        for (int ob = 0; ob < N / 16; ++ob) {
+          const u32x4_t* wp = (const u32x4_t*)(Wl + (c * (N / 16) + ob) * 1024) + lane;
+          const f16x8 ah = __builtin_bit_cast(f16x8, wp[0]), al = __builtin_bit_cast(f16x8, wp[64]);
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            v4f t = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[q], acc[ob][q], 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[q], t, 0, 0, 0);
+            acc[ob][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[q], t, 0, 0, 0);
+          }
+          mem_fence_sched();
+        }
+      } else {  // an infinity has no low part: the wave's products on the fp32 matrix cores
+#pragma unroll
+        for (int ob = 0; ob < N / 16; ++ob) {
+          const u32x4_t* wp = (const u32x4_t*)(Wl + (c * (N / 16) + ob) * 1024) + lane;
+          const f16x8 ah = __builtin_bit_cast(f16x8, wp[0]), al = __builtin_bit_cast(f16x8, wp[64]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float w = (float)ah[e] + (float)al[e];  // (scaled like the fp16 products)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) acc[ob][q] = mfma4(w, xb[q][e], acc[ob][q]);
+          }
+          mem_fence_sched();
+        }
+      }
+    }
+    if (whole || !over) break;
+    whole = true;
+    zero_acc<N, Q>(acc);
   }
   if (plain) return inv;
 #pragma unroll
@@ -591,7 +617,7 @@ __global__ void __launch_bounds__(64 * NW) k_conv1x1_mfma(const float* __restric
       // which measured 2 % faster there); those lanes' values never reach an output
       load_acc<CIN, Q>(x + b * CIN * hw + pw, hw, true, inb ? yoff : yoff0, xv);
       if (LN) ln_acc<CIN, Q>(xv, prm + 2 * COUT, prm + 2 * COUT + CIN, eps, g, xv);
-      inv_t = gemm_f16s<CIN, COUT, Q>(xv, (const _Float16*)Wt, lane, inv, acc);
+      inv_t = gemm_f16s<CIN, COUT, Q, !LN && CIN >= 128>(xv, (const _Float16*)Wt, lane, inv, acc);
     } else {
       float xv[CIN / 4][Q];
       load_tile<CIN, Q>(x + b * CIN * hw + pw, hw, inb, xoff, xv);

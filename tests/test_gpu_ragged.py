@@ -149,6 +149,16 @@ def test_activation_scale(ci, co, H, W, sx, sw):
 
 
 @pytest.mark.parametrize("ci,co,H,W", SPLIT)
+def test_large_activation_in_a_late_channel(ci, co, H, W):
+    """Pixels that fit by their first 32 channels, with one above fp16's end in the last: the products start over."""
+    x, w = _conv_case(ci, co, H, W, 11)
+    x = x.astype(np.float32)
+    x[0, -1, 1, 2], x[1, -1, 0, 0] = 3e5, -1e30
+    ref = np.einsum("oc,bchw->bohw", w[:, :, 0, 0].astype(np.float64), x.astype(np.float64))
+    assert (np.linalg.norm(_conv(x, w) - ref, axis=1) <= TOL * np.linalg.norm(ref, axis=1)).all()
+
+
+@pytest.mark.parametrize("ci,co,H,W", SPLIT)
 def test_pixels_and_rows_of_different_size(ci, co, H, W):
     """Pixels 1e-8 to 1e8, each against its own size (they are scaled one by one); an infinity stays in its pixel, and
     is one there; output rows 1e-2.5 to 1e2.5 (a matrix has one scale: a row is exact to 2^-22 from 2^-17 of the largest

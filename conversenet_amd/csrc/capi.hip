@@ -31,6 +31,12 @@ extern "C" const char* cvn_last_error(void) { return last_error_slot().c_str(); 
 
 extern "C" int cvn_clear_cache(void) { return CVN_OK; }
 
+extern "C" int cvn_event_record(void* event, cvn_stream_t stream) {
+  if (!event) return fail(CVN_ERR_ARG, "null event");
+  const hipError_t e = hipEventRecord((hipEvent_t)event, (hipStream_t)stream);
+  return e == hipSuccess ? CVN_OK : fail(CVN_ERR_HIP, "event record: %s", hipGetErrorString(e));
+}
+
 extern "C" int cvn_event_wait(void* event, cvn_stream_t stream) {
   if (!event) return fail(CVN_ERR_ARG, "null event");
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;

@@ -80,6 +80,9 @@ def _capturing(stream) -> bool:
     return stream != 0 and torch._C._cuda_isCurrentStreamCapturing()
 
 
+_marks: dict = {}  # (device, stream) -> event behind the latest table made there
+
+
 class _Made:
     """Where the kernels that made a table were enqueued, and what other streams need before they read it."""
 
@@ -88,8 +91,15 @@ class _Made:
     def __init__(self, dev, stream):
         self.dev, self.stream = dev, stream
         self.streams = {stream}  # streams that may use the table and its memory in their own order
-        self.event = torch.cuda.Event()  # None once it is known to have passed
-        self.event.record(torch.cuda.current_stream(dev))
+        # one event per stream, recorded again by each table (a new one costs 5 us more): waiting for a later
+        # table too is no harm
+        self.event = _marks.get((dev.index, stream))  # None once it is known to have passed
+        if self.event is None:
+            self.event = torch.cuda.Event()
+            self.event.record(torch.cuda.current_stream(dev))
+            _marks[dev.index, stream] = self.event
+        else:
+            _lib.check(_lib.load().cvn_event_record(self.event.cuda_event, stream), "transfer table")
 
     def join(self, table, stream):
         """Orders the current stream (its handle) after the making of the table, and the release of the table's

@@ -188,6 +188,8 @@ int cvn_converse2d_op_apply_f32(const float* x, const float* x0, int64_t B, int6
  * it is kept so that a binding of the reference's clear_cache has a symbol to call. */
 int cvn_clear_cache(void);
 
+/* Records a HIP event (hipEvent_t) on a stream. */
+int cvn_event_record(void* event, cvn_stream_t stream);
 /* Waits on the host until a HIP event (hipEvent_t, recorded on `stream` outside any graph) has passed.  Unlike a
  * plain hipEventSynchronize it may be called by a thread whose stream records a graph, so that a table built
  * before the recording is complete before the graph reads it.  Returns at once where `stream` itself records now:

@@ -678,8 +678,9 @@ constexpr int kCus = 256;  // compute units of the device
 // elements per thread) is the fastest or within 6 % of it, and an uneven share of the 16 waves (3, 5) up to
 // 30 % slower.  Where the blocks are too few to fill the chip, waves are doubled while all blocks stay
 // resident and the widest pass still gives every wave a butterfly per lane (64 planes of 136 x 136: 37 -> 28 us), or,
-// for the loads and stores, a thread has 4 elements or more (a call on 2 to 64 planes of 16 to 264 rows or columns of
-// 64: 1 to 3 us of 20 to 27 us less; 2 elements: 0.5 us more than 4).
+// for the loads and stores, a thread has 4 elements or more and the chip is half empty (a call on 2 to 64 planes of 16 to
+// 264 rows or columns of 64: 1 to 3 us of 20 to 27 us less; 2 elements: 0.5 us more than 4; beyond half full 1 to 4 %
+// slower).
 // lds: the block's LDS, where it holds more than one line buffer (fewer blocks per CU, more waves each).
 int line_threads(const LinePlan& p, int nblk, size_t lds = 0) {
   int w = 1, most = 1;
@@ -687,8 +688,8 @@ int line_threads(const LinePlan& p, int nblk, size_t lds = 0) {
   for (int t = 0; t < p.np; ++t) most = std::max(most, p.ps[t].nl * kLines);
   if (lds) most = std::max(most, p.L * 8);  // the product's items
   while (lds && 2 * w * (int)(kLineLds / lds) <= 16 && 64 * w < most) w *= 2;
-  most = std::max(most, p.L * kLines / 4);
   while (2 * w <= 16 && (int64_t)nblk * 2 * w <= kCus * 16 && 64 * w < most) w *= 2;
+  while (2 * w <= 16 && (int64_t)nblk * 2 * w <= kCus * 8 && 4 * 64 * w < p.L * kLines) w *= 2;
   return std::max(64 * w, line_min_threads(p));
 }
 
@@ -794,22 +795,20 @@ size_t cols_bwd_lines_lds(int h, int Hs, int s) {
 
 namespace {
 // Whether k_cols_bwd (1 to 8 columns per block) is the faster one: with less than about a block per CU, the lines
-// pass is a serial chain over the planes of a psf beside idle CUs.  k_cols_bwd's plan must hold no prime above
-// 13 (34 rows, scale 1: 412 us against 205).  Whole backward, us, that / this, B planes per psf:
-//   scale > 1: 32 rows, 18 blocks, B 2 74 / 82, B 16 175 / 269; 128 rows, 98 blocks, B 16 313 / 363, 392 blocks, B 4
-//     265 / 213; 192 rows, 132 blocks, B 16 523 / 643; 400 rows, 42 blocks, B 4 163 / 185; 200 rows, 102 blocks, B 4
-//     184 / 177, 204 blocks, B 16 747 / 537; B 1 within 5 %.
-//   scale 1, where a block holds one column buffer less: only if the lines pass has a radix that leaves most of a
-//     block idle (24 rows in one radix, 34 blocks, B 4 77 / 81, B 16 150 / 180) or that one has two stages (64 rows, 98 blocks,
-//     B 16 200 / 210), or at few blocks of long columns (320 rows, 42 blocks, B 4 125 / 134); otherwise 36 rows, 38
-//     blocks, B 16 180 / 160; 120 rows, 62 blocks, B 16 235 / 217; 200 rows 282 / 288.
+// pass is a serial chain over the planes of a psf beside idle CUs.  Time of the whole backward with that one over the
+// time with this one, columns of h, B planes per psf, 4 to 84 blocks (it hardly depends on their number there):
+//   scale > 1: B 2 0.97 to 0.87, B 4 0.96 to 0.78, B 16 0.89 to 0.64 at h s = 32 to 400; B 1 1.04 to 0.97 at scale 2, 0.99 to
+//     0.93 at scale 3.  Columns up to 192: still at 132 blocks (192 rows, B 16 523 / 643 us); longer ones: 98 blocks
+//     313 / 363, 102 blocks of 400 rows 184 / 177, 392 blocks of 256 265 / 213.
+//   scale 1, where a block holds one column buffer less: h 24 1.00 at B 2, 0.96 at B 4, 0.85 at B 16, and 32 0.95, 0.88, 0.74, one
+//     butterfly per line; 64 (k_cols_bwd in two stages) 1.00 at B 4, 0.96 at B 8, 0.93 at B 16; 320 and 400 0.93 at B 4, 0.85 at B 16,
+//     but 1.02 at 84 blocks; otherwise 36 1.12, 48 1.08, 120 1.10 at any B, 100 and 128 1.00 at B 4, 0.95 at B 16, 200 1.00.
 bool few_bwd_blocks(int64_t nblk, int64_t nplanes, int h, int s) {
-  const FftPlan* p = fft_plan(h);
   if (!plain_plan(h) || !plain_plan(h * s)) return false;
-  if (s > 1) return nblk < (h * s <= 192 ? 200 : 100) && nplanes > 1;
-  const int narrow = narrowest(*line_plan(h));
-  return (nblk < 100 && nplanes >= 8 && (narrow < 4 || p->nst <= 2)) ||
-         (nblk < 50 && nplanes >= 4 && (narrow < 4 || h >= 256));
+  const int64_t part = h * s <= 192 ? 4 * nblk : 8 * nblk;  // of 3 blocks per CU
+  if (s > 1) return part < 3 * kCus && (nplanes > 1 || s > 2);
+  if (narrowest(*line_plan(h)) <= 2) return 8 * nblk < 3 * kCus && nplanes > 1;
+  return h >= 256 ? 5 * nblk < kCus && nplanes >= 4 : 8 * nblk < 3 * kCus && nplanes >= 8 && fft_plan(h)->nst <= 2;
 }
 }  // namespace
 

@@ -136,17 +136,18 @@ def test_operator_arbitrary_x0(B, C, h, w, k, s, lines):
 
 # (B, C, H, W, k, s, p, mode, psf batch, lines): several planes per psf and blocks that straddle psf groups
 BWD_CASES = [
-    (3, 5, 31, 29, 3, 1, 4, "circular", 1, True),     # 39 x 37
-    (2, 3, 33, 57, 5, 1, 2, "reflect", 2, True),      # 37 x 61
-    (4, 3, 94, 43, 3, 1, 3, "replicate", 1, True),    # 100 x 49
-    (3, 4, 15, 26, 3, 2, 1, "constant", 1, True),     # 34 x 56
-    (2, 3, 17, 13, 5, 3, 2, "circular", 2, True),     # 63 x 51
-    (3, 2, 10, 21, 2, 4, 1, "reflect", 1, False),      # 48 x 92
-    (1, 5, 16, 20, 3, 2, 0, "circular", 1, True),     # 32 x 40: one plane per psf, the lines pass
-    (2, 60, 14, 110, 3, 2, 0, "circular", 1, True),   # 28 x 220: blocks for most of the chip, the lines pass
-    (8, 3, 24, 10, 3, 1, 0, "circular", 1, False),     # 24 x 10: few blocks, a column class or more per block
-    (4, 2, 100, 9, 3, 3, 1, "replicate", 1, True),    # 306 x 33 (17 a factor): the lines pass at few blocks
-    (3, 3, 70, 9, 3, 3, 0, "constant", 1, False),      # 210 x 27: few blocks of long columns
+    (3, 5, 31, 29, 3, 1, 4, "circular", 1, True),  # 39 x 37
+    (2, 3, 33, 57, 5, 1, 2, "reflect", 2, True),  # 37 x 61
+    (4, 3, 94, 43, 3, 1, 3, "replicate", 1, True),  # 100 x 49
+    (3, 4, 15, 26, 3, 2, 1, "constant", 1, True),  # 34 x 56
+    (2, 3, 17, 13, 5, 3, 2, "circular", 2, False),  # 63 x 51: few blocks, one plane per psf
+    (2, 135, 5, 20, 5, 3, 2, "circular", 2, True),  # 27 x 72
+    (3, 2, 10, 21, 2, 4, 1, "reflect", 1, False),  # 48 x 92
+    (1, 5, 16, 20, 3, 2, 0, "circular", 1, True),  # 32 x 40: one plane per psf, the lines pass
+    (2, 60, 14, 110, 3, 2, 0, "circular", 1, True),  # 28 x 220: blocks for most of the chip, the lines pass
+    (8, 3, 24, 10, 3, 1, 0, "circular", 1, False),  # 24 x 10: few blocks, a column class or more per block
+    (4, 2, 100, 9, 3, 3, 1, "replicate", 1, True),  # 306 x 33 (17 a factor): the lines pass at few blocks
+    (3, 3, 70, 9, 3, 3, 0, "constant", 1, False),  # 210 x 27: few blocks of long columns
 ]
 
 

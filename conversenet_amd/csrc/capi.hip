@@ -31,10 +31,26 @@ extern "C" const char* cvn_last_error(void) { return last_error_slot().c_str(); 
 
 extern "C" int cvn_clear_cache(void) { return CVN_OK; }
 
+namespace {
+int event_rc(hipError_t e, const char* what) {
+  return e == hipSuccess ? CVN_OK : fail(CVN_ERR_HIP, "event %s: %s", what, hipGetErrorString(e));
+}
+}  // namespace
+
+extern "C" int cvn_event_create(void** event) {
+  if (!event) return fail(CVN_ERR_ARG, "null event");
+  return event_rc(hipEventCreateWithFlags((hipEvent_t*)event, hipEventDisableTiming | hipEventDisableSystemFence),
+                  "create");
+}
+
 extern "C" int cvn_event_record(void* event, cvn_stream_t stream) {
   if (!event) return fail(CVN_ERR_ARG, "null event");
-  const hipError_t e = hipEventRecord((hipEvent_t)event, (hipStream_t)stream);
-  return e == hipSuccess ? CVN_OK : fail(CVN_ERR_HIP, "event record: %s", hipGetErrorString(e));
+  return event_rc(hipEventRecord((hipEvent_t)event, (hipStream_t)stream), "record");
+}
+
+extern "C" int cvn_event_join(void* event, cvn_stream_t stream) {
+  if (!event) return fail(CVN_ERR_ARG, "null event");
+  return event_rc(hipStreamWaitEvent((hipStream_t)stream, (hipEvent_t)event, 0), "join");
 }
 
 extern "C" int cvn_event_wait(void* event, cvn_stream_t stream) {
@@ -48,7 +64,7 @@ extern "C" int cvn_event_wait(void* event, cvn_stream_t stream) {
     const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
     if (e == hipSuccess) e = back;
   }
-  return e == hipSuccess ? CVN_OK : fail(CVN_ERR_HIP, "event wait: %s", hipGetErrorString(e));
+  return event_rc(e, "wait");
 }
 
 extern "C" int cvn_copy_f32(const float* src, float* dst, int64_t n, cvn_stream_t stream) {

@@ -7,6 +7,7 @@ kernels on torch's current stream.  No CPU fallback exists here: a missing libra
 """
 from __future__ import annotations
 
+import ctypes
 import os
 import threading
 
@@ -91,29 +92,29 @@ class _Made:
     def __init__(self, dev, stream):
         self.dev, self.stream = dev, stream
         self.streams = {stream}  # streams that may use the table and its memory in their own order
-        # one event per stream, recorded again by each table (a new one costs 5 us more): waiting for a later
-        # table too is no harm
+        # one event per stream, recorded again by each table (waiting for a later table too is no harm), without a
+        # system-wide fence: writing the caches back would cost the first call on new weights 30 us
+        lib = _lib.load()
         self.event = _marks.get((dev.index, stream))  # None once it is known to have passed
         if self.event is None:
-            self.event = torch.cuda.Event()
-            self.event.record(torch.cuda.current_stream(dev))
-            _marks[dev.index, stream] = self.event
-        else:
-            _lib.check(_lib.load().cvn_event_record(self.event.cuda_event, stream), "transfer table")
+            e = ctypes.c_void_p()
+            with torch.cuda.device(dev):
+                _lib.check(lib.cvn_event_create(ctypes.byref(e)), "transfer table")
+            self.event = _marks.setdefault((dev.index, stream), e)
+        _lib.check(lib.cvn_event_record(self.event, stream), "transfer table")
 
     def join(self, table, stream):
         """Orders the current stream (its handle) after the making of the table, and the release of the table's
         memory after what that stream has enqueued by then."""
-        cur = torch.cuda.current_stream(self.dev)
         if self.event is not None:
-            cur.wait_event(self.event)
-        table.record_stream(cur)
+            _lib.check(_lib.load().cvn_event_join(self.event, stream), "transfer table")
+        table.record_stream(torch.cuda.current_stream(self.dev))
         self.streams.add(stream)
 
     def finish(self):
         """Waits on the host: a stream that records a graph cannot wait for an event from outside it."""
         if self.event is not None:
-            _lib.check(_lib.load().cvn_event_wait(self.event.cuda_event, self.stream), "transfer table")
+            _lib.check(_lib.load().cvn_event_wait(self.event, self.stream), "transfer table")
             self.event = None
 
 
@@ -528,18 +529,17 @@ def layernorm_cf(x, weight, bias, eps):
     return y
 
 
-def _wmat(weight):
-    return weight.reshape(weight.shape[0], -1).contiguous()
-
-
-def _dense(*ts):
-    """Contiguous tensors (or None) for a call.  The caller keeps them until the call has enqueued its kernels: a
-    copy that is dropped before then gives its memory to the next copy or output."""
-    return [t if t is None else t.contiguous() for t in ts]
-
-
-def _ptr(t):
-    return None if t is None else t.data_ptr()
+def _ptrs(keep, *ts):
+    """Addresses of contiguous tensors (None for None).  Copies of others go to `keep`, which the caller holds until
+    the call has enqueued its kernels: a copy that is dropped before then gives its memory to the next copy or
+    output."""
+    out = []
+    for t in ts:
+        if t is not None and not t.is_contiguous():
+            t = t.contiguous()
+            keep.append(t)
+        out.append(None if t is None else t.data_ptr())
+    return out
 
 
 def conv1x1(x, weight, bias=None, act=None, residual=None, res_scale=None, ln=None, out=None):
@@ -549,22 +549,19 @@ def conv1x1(x, weight, bias=None, act=None, residual=None, res_scale=None, ln=No
     _need_hip(x, weight, bias, residual, res_scale)
     x = x.contiguous()
     B, Cin, H, W = x.shape
-    Wm = _wmat(weight)
-    Cout = Wm.shape[0]
-    if Wm.shape[1] != Cin:
+    Cout = weight.shape[0]
+    if weight.numel() != Cout * Cin:
         raise RuntimeError("weight does not match input channels")
     y = out if out is not None else torch.empty((B, Cout, H, W), dtype=torch.float32, device=x.device)
-    bias, residual, res_scale = _dense(bias, residual, res_scale)
-    bptr, rptr, sptr = _ptr(bias), _ptr(residual), _ptr(res_scale)
+    keep = []
+    wptr, bptr, rptr, sptr = _ptrs(keep, weight, bias, residual, res_scale)
     a = _lib.ACT_GELU if act == "gelu" else _lib.ACT_NONE
     st = _stream(x.device)
     if ln is None:
-        rc = lib.cvn_conv1x1_f32(x.data_ptr(), B, Cin, H * W, Wm.data_ptr(), bptr, Cout, a, rptr, sptr,
-                                 y.data_ptr(), st)
+        rc = lib.cvn_conv1x1_f32(x.data_ptr(), B, Cin, H * W, wptr, bptr, Cout, a, rptr, sptr, y.data_ptr(), st)
     else:
-        lw, lb = _dense(*ln[:2])
-        rc = lib.cvn_ln_conv1x1_f32(x.data_ptr(), B, Cin, H * W, lw.data_ptr(), lb.data_ptr(), float(ln[2]),
-                                    Wm.data_ptr(), bptr, Cout, a, rptr, sptr, y.data_ptr(), st)
+        rc = lib.cvn_ln_conv1x1_f32(x.data_ptr(), B, Cin, H * W, *_ptrs(keep, *ln[:2]), float(ln[2]), wptr, bptr, Cout,
+                                    a, rptr, sptr, y.data_ptr(), st)
     _lib.check(rc, "conv1x1")
     return y
 
@@ -575,13 +572,11 @@ def ln_mlp_residual(x, ln_w, ln_b, ln_eps, w1, b1, w2, b2, res_scale=None, out=N
     _need_hip(x, w1, b1, w2, b2, res_scale)
     x = x.contiguous()
     B, C, H, W = x.shape
-    W1 = _wmat(w1)
-    W2 = _wmat(w2)
+    keep = []
     y = out if out is not None else torch.empty_like(x)
-    ln_w, ln_b, b1, b2, res_scale = _dense(ln_w, ln_b, b1, b2, res_scale)
-    rc = lib.cvn_ln_mlp_residual_f32(x.data_ptr(), B, C, H * W, ln_w.data_ptr(), ln_b.data_ptr(), float(ln_eps),
-                                     W1.data_ptr(), b1.data_ptr(), W1.shape[0], W2.data_ptr(), b2.data_ptr(),
-                                     _ptr(res_scale), y.data_ptr(), _stream(x.device))
+    lw, lb, w1_, b1_, w2_, b2_, sp = _ptrs(keep, ln_w, ln_b, w1, b1, w2, b2, res_scale)
+    rc = lib.cvn_ln_mlp_residual_f32(x.data_ptr(), B, C, H * W, lw, lb, float(ln_eps), w1_, b1_, w1.shape[0], w2_, b2_,
+                                     sp, y.data_ptr(), _stream(x.device))
     _lib.check(rc, "ln_mlp_residual")
     return y
 
@@ -601,23 +596,21 @@ def conv_ln_mlp_residual(t, x, w0, b0, ln_w, ln_b, ln_eps, w1, b1, w2, b2, res_s
     x = x.contiguous()
     B, Ct, H, W = t.shape
     C = x.shape[1]
-    W0, W1, W2 = _wmat(w0), _wmat(w1), _wmat(w2)
     y = out if out is not None else torch.empty_like(x)
     act = _lib.ACT_GELU if t_act == "gelu" else _lib.ACT_NONE
-    vs = _dense(b0, res_scale1, ln_w, ln_b, b1, b2, res_scale2)
-    b0_, s1, lw, lb, b1_, b2_, s2 = (_ptr(v) for v in vs)
-    common = (t.data_ptr(), act, B, Ct, H * W, W0.data_ptr(), b0_, s1, x.data_ptr(), C, lw, lb, float(ln_eps),
-              W1.data_ptr(), b1_, W1.shape[0], W2.data_ptr(), b2_, s2, y.data_ptr())
+    keep = []
+    w0_, b0_, s1, lw, lb, w1_, b1_, w2_, b2_, s2 = _ptrs(keep, w0, b0, res_scale1, ln_w, ln_b, w1, b1, w2, b2, res_scale2)
+    common = (t.data_ptr(), act, B, Ct, H * W, w0_, b0_, s1, x.data_ptr(), C, lw, lb, float(ln_eps), w1_, b1_,
+              w1.shape[0], w2_, b2_, s2, y.data_ptr())
     if head is None:
         _lib.check(lib.cvn_conv_ln_mlp_residual_f32(*common, _stream(x.device)), "conv_ln_mlp_residual")
         return y
     hw, hb, heps, wh, bh = head
     _need_hip(wh, bh)
-    Wh = _wmat(wh)
-    hw, hb, bh = _dense(hw, hb, bh)
-    tn = torch.empty((B, Wh.shape[0], H, W), device=x.device, dtype=x.dtype)
-    _lib.check(lib.cvn_conv_ln_mlp_head_f32(*common, _ptr(hw), _ptr(hb), float(heps), Wh.data_ptr(), _ptr(bh),
-                                            tn.data_ptr(), _stream(x.device)), "conv_ln_mlp_head")
+    hw_, hb_, wh_, bh_ = _ptrs(keep, hw, hb, wh, bh)
+    tn = torch.empty((B, wh.shape[0], H, W), device=x.device, dtype=x.dtype)
+    _lib.check(lib.cvn_conv_ln_mlp_head_f32(*common, hw_, hb_, float(heps), wh_, bh_, tn.data_ptr(), _stream(x.device)),
+               "conv_ln_mlp_head")
     return y, tn
 
 

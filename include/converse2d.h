@@ -188,8 +188,12 @@ int cvn_converse2d_op_apply_f32(const float* x, const float* x0, int64_t B, int6
  * it is kept so that a binding of the reference's clear_cache has a symbol to call. */
 int cvn_clear_cache(void);
 
-/* Records a HIP event (hipEvent_t) on a stream. */
+/* Events of one device that order streams after a table's kernels, without the system-wide fence of an ordinary one
+ * (which writes the caches back): create on the current device, record on a stream, let a stream wait.  The
+ * event is a hipEvent_t; the caller destroys it. */
+int cvn_event_create(void** event);
 int cvn_event_record(void* event, cvn_stream_t stream);
+int cvn_event_join(void* event, cvn_stream_t stream);
 /* Waits on the host until a HIP event (hipEvent_t, recorded on `stream` outside any graph) has passed.  Unlike a
  * plain hipEventSynchronize it may be called by a thread whose stream records a graph, so that a table built
  * before the recording is complete before the graph reads it.  Returns at once where `stream` itself records now:

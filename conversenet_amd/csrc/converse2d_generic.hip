@@ -1987,7 +1987,7 @@ int launch_rows_fwd(const float* x, int64_t P, int Hin, int Win, int pad, int mo
   a.S = S;
   dim3 grid((h + a.rpb - 1) / a.rpb, (unsigned)P);
   const size_t lds = a.rad_off + rader_lds_bytes(a.plan);
-  switch (w) {  // lengths with a compile-time plan
+  switch (w) {  // fixed_len
     case 132: hipLaunchKernelGGL(k_rows_fwd<132>, grid, dim3(kThreads), lds, st, a); break;
     case 256: hipLaunchKernelGGL(k_rows_fwd<256>, grid, dim3(kThreads), lds, st, a); break;
     case 260: hipLaunchKernelGGL(k_rows_fwd<260>, grid, dim3(kThreads), lds, st, a); break;
@@ -2013,7 +2013,7 @@ int launch_rows_inv(const float2* SH, const Geo& g, int row0, int nrows, int col
   a.tabs = tabs;
   dim3 grid((nrows + a.rpb - 1) / a.rpb, (unsigned)g.P);
   const size_t lds = a.csrc_off + sizeof(int) * 2 * std::max(pad, 0);
-  switch (g.Ws) {  // lengths with a compile-time plan
+  switch (g.Ws) {  // fixed_len
     case 132: hipLaunchKernelGGL(k_rows_inv<132>, grid, dim3(kThreads), lds, st, a); break;
     case 256: hipLaunchKernelGGL(k_rows_inv<256>, grid, dim3(kThreads), lds, st, a); break;
     case 260: hipLaunchKernelGGL(k_rows_inv<260>, grid, dim3(kThreads), lds, st, a); break;
@@ -2444,10 +2444,11 @@ extern "C" size_t cvn_converse2d_bwd_workspace(int64_t B, int64_t C, int64_t H, 
 }
 
 namespace {
-// 132, 256 and 260 points at scale 1 keep the compile-time kernel, whose dPhi sums stay in registers through its
-// smaller transforms: 340 us against 690 at 260 points and 1024 planes.
+// Columns with a compile-time pass keep it: its dPhi sums stay in registers through its smaller transforms.  Whole backward
+// with the lines pass over the one with this, 1 to 16 planes per psf and 3 to 64 channels: 132 points 0.98 (64 planes of
+// 260 columns) to 1.67, 256 points 1.05 to 2.16, 260 points 1.05 to 1.87 (1024 planes of 260 columns 845 / 1144 us).
 bool bwd_lines(const Geo& g) {
-  if (g.s == 1 && (g.h == 132 || g.h == 256 || g.h == 260)) return false;
+  if (g.s == 1 && fixed_len(g.h)) return false;
   return lines_cols_bwd_ok(g.P, g.Cp == g.C ? g.B : 1, g.h, g.Hs, g.s, g.NC);
 }
 }  // namespace
@@ -2533,7 +2534,7 @@ extern "C" int cvn_converse2d_bwd_f32(const float* grad_out, const float* x, int
     a.rad_off = (int)align_up(cols_bwd_lds(g.h, g.Hs, g.s, a.cpb, wg), 16);
     const size_t lds = col_lds;
     const dim3 grid((unsigned)((g.NC + a.cpb - 1) / a.cpb), (unsigned)(a.psf_batch == 1 ? g.C : g.P));
-    const int hc = g.s == 1 ? g.h : 0;  // column lengths with a compile-time plan (scale 1)
+    const int hc = g.s == 1 && fixed_len(g.h) ? g.h : 0;
     switch (hc) {
       case 132: hipLaunchKernelGGL(k_cols_bwd<132>, grid, dim3(kColsBwdThreads), lds, st, a); break;
       case 256: hipLaunchKernelGGL(k_cols_bwd<256>, grid, dim3(kColsBwdThreads), lds, st, a); break;

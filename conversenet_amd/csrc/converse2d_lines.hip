@@ -726,7 +726,8 @@ bool lines_rows_ok(int64_t P, int h, int w) {
   const int64_t lines = P * ((h + 1) / 2), nblk = (lines + kLines - 1) / kLines;
   if (!p || lines >= (1 << 30)) return false;
   const bool few = narrowest(*p) <= 2 ? 4 * nblk < 3 * kCus
-                   : w == 132 || w == 256 || w == 260 ? nblk * w < 100 * kCus : w >= 640 && 8 * nblk < kCus;
+                   : fixed_len(w)        ? nblk * w < 100 * kCus
+                                         : w >= 640 && 8 * nblk < kCus;
   return !few || !plain_plan(w);
 }
 

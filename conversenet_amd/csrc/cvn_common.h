@@ -224,6 +224,9 @@ int launch_module_ct(const float* x, int64_t P, int64_t C, int64_t psf_batch, in
                      const float2* tw_w, const float2* tw_h, const float2* tw_Hs, const float2* tw_Ws,
                      const float2* phi, float2* S, float2* SH, float* out, hipStream_t st);
 
+// Lengths for which the row passes and the backward column pass of converse2d_generic.hip have a compile-time form.
+inline bool fixed_len(int L) { return L == 132 || L == 256 || L == 260; }
+
 // Row and column passes on the in-place prime-factor engine (converse2d_lines.hip), lengths up to 1024.
 // Same scratch, table and twiddle layouts as the runtime-plan passes; tw_*: exp(-2 pi i m / L), m < L.
 bool lines_rows_ok(int64_t P, int h, int w);

@@ -68,7 +68,7 @@ SIGNATURES = {
     "cvn_clear_cache": (_int, []),
     "cvn_event_create": (_int, [ctypes.POINTER(_ptr)]),
     "cvn_event_record": (_int, [_ptr, _ptr]),
-    "cvn_event_join": (_int, [_ptr, _ptr]),
+    "cvn_event_join": (_int, [_ptr, _ptr, _ptr]),
     "cvn_event_wait": (_int, [_ptr, _ptr]),
     "cvn_layernorm_cf_f32": (_int, [_ptr, _i64, _i64, _i64, _ptr, _ptr, _f32, _ptr, _ptr]),
     "cvn_conv1x1_f32": (_int, [_ptr, _i64, _i64, _i64, _ptr, _ptr, _i64, _int, _ptr, _ptr, _ptr, _ptr]),

@@ -20,7 +20,7 @@ ARCH = os.environ.get("CVN_OFFLOAD_ARCH", "gfx950")
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
-    # packed fp32 VALU ops stay disabled on this target (correctness trap on these boxes)
+    # packed fp32 VALU ops stay disabled on this target: some of their forms have given wrong results
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]

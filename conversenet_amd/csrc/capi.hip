@@ -35,6 +35,14 @@ namespace {
 int event_rc(hipError_t e, const char* what) {
   return e == hipSuccess ? CVN_OK : fail(CVN_ERR_HIP, "event %s: %s", what, hipGetErrorString(e));
 }
+// Whether a stream records a graph (the null stream cannot).  HIP refuses waits for events of such a stream, and
+// the attempt spoils the recording.
+hipError_t recording(hipStream_t stream, bool* yes) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  const hipError_t e = stream ? hipStreamIsCapturing(stream, &status) : hipSuccess;
+  *yes = status != hipStreamCaptureStatusNone;
+  return e;
+}
 }  // namespace
 
 extern "C" int cvn_event_create(void** event) {
@@ -48,8 +56,12 @@ extern "C" int cvn_event_record(void* event, cvn_stream_t stream) {
   return event_rc(hipEventRecord((hipEvent_t)event, (hipStream_t)stream), "record");
 }
 
-extern "C" int cvn_event_join(void* event, cvn_stream_t stream) {
+extern "C" int cvn_event_join(void* event, cvn_stream_t recorded_on, cvn_stream_t stream) {
   if (!event) return fail(CVN_ERR_ARG, "null event");
+  bool busy = false;
+  const hipError_t e = recording((hipStream_t)recorded_on, &busy);
+  if (e != hipSuccess) return event_rc(e, "join");
+  if (busy) return fail(CVN_ERR_UNSUPPORTED, "event join: the event's stream records a graph");
   return event_rc(hipStreamWaitEvent((hipStream_t)stream, (hipEvent_t)event, 0), "join");
 }
 
@@ -58,9 +70,9 @@ extern "C" int cvn_event_wait(void* event, cvn_stream_t stream) {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
   if (e == hipSuccess) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (stream) e = hipStreamIsCapturing((hipStream_t)stream, &status);
-    if (e == hipSuccess && status == hipStreamCaptureStatusNone) e = hipEventSynchronize((hipEvent_t)event);
+    bool busy = false;
+    e = recording((hipStream_t)stream, &busy);
+    if (e == hipSuccess && !busy) e = hipEventSynchronize((hipEvent_t)event);
     const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
     if (e == hipSuccess) e = back;
   }

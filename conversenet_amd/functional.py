@@ -105,11 +105,15 @@ class _Made:
 
     def join(self, table, stream):
         """Orders the current stream (its handle) after the making of the table, and the release of the table's
-        memory after what that stream has enqueued by then."""
+        memory after what that stream has enqueued by then.  False while the making stream records a graph."""
         if self.event is not None:
-            _lib.check(_lib.load().cvn_event_join(self.event, stream), "transfer table")
+            rc = _lib.load().cvn_event_join(self.event, self.stream, stream)
+            if rc == _lib.CVN_ERR_UNSUPPORTED:
+                return False
+            _lib.check(rc, "transfer table")
         table.record_stream(torch.cuda.current_stream(self.dev))
         self.streams.add(stream)
+        return True
 
     def finish(self):
         """Waits on the host: a stream that records a graph cannot wait for an event from outside it."""
@@ -173,9 +177,7 @@ class TableCache:
         if _capturing(stream):
             e.made.finish()
             return self._keep_recorded(e)
-        if stream not in e.made.streams:
-            e.made.join(e[0], stream)
-        return True
+        return stream in e.made.streams or e.made.join(e[0], stream)
 
     def get(self, key, stream=None):
         """The table of `key` or None.  stream: the current stream's handle, where the table is to be read."""

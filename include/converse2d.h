@@ -190,10 +190,11 @@ int cvn_clear_cache(void);
 
 /* Events of one device that order streams after a table's kernels, without the system-wide fence of an ordinary one
  * (which writes the caches back): create on the current device, record on a stream, let a stream wait.  The
- * event is a hipEvent_t; the caller destroys it. */
+ * event is a hipEvent_t; the caller destroys it.  The join returns CVN_ERR_UNSUPPORTED, with nothing enqueued, while
+ * the stream that the event was recorded on records a graph. */
 int cvn_event_create(void** event);
 int cvn_event_record(void* event, cvn_stream_t stream);
-int cvn_event_join(void* event, cvn_stream_t stream);
+int cvn_event_join(void* event, cvn_stream_t recorded_on, cvn_stream_t stream);
 /* Waits on the host until a HIP event (hipEvent_t, recorded on `stream` outside any graph) has passed.  Unlike a
  * plain hipEventSynchronize it may be called by a thread whose stream records a graph, so that a table built
  * before the recording is complete before the graph reads it.  Returns at once where `stream` itself records now:

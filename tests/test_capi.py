@@ -60,7 +60,7 @@ def test_argument_errors_without_device():
     assert lib.cvn_conv1x1_f32(None, 1, 2, 4, None, None, 2, 0, None, None, None, None) == _lib.CVN_ERR_ARG
     assert lib.cvn_copy_f32(None, None, 4, None) == _lib.CVN_ERR_ARG
     assert lib.cvn_event_wait(None, None) == _lib.CVN_ERR_ARG
-    assert lib.cvn_event_record(None, None) == lib.cvn_event_join(None, None) == _lib.CVN_ERR_ARG
+    assert lib.cvn_event_record(None, None) == lib.cvn_event_join(None, None, None) == _lib.CVN_ERR_ARG
     assert lib.cvn_event_create(None) == _lib.CVN_ERR_ARG
 
 

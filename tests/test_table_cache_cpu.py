@@ -120,12 +120,15 @@ def _fake_streams(monkeypatch):
 
     class Made:
         def __init__(self, dev, stream):
-            self.streams = {stream}
+            self.made_on, self.streams = stream, {stream}
             log.append(("made", stream))
 
         def join(self, table, stream):
+            if self.made_on in state["capturing"]:
+                return False
             self.streams.add(stream)
             log.append(("wait and hold", stream))
+            return True
 
         def finish(self):
             log.append(("host wait",))
@@ -142,6 +145,10 @@ def test_hits_wait_for_the_stream_that_made_the_table(monkeypatch):
     c.put(_key(w, b), torch.empty(8, dtype=torch.uint8), (w, b), 7)
     assert c.get(_key(w, b), 7) is not None and log == [("made", 7)]
     assert c.get(_key(w, b), 9) is not None and log[1:] == [("wait and hold", 9)]
+    state["capturing"] = {7}  # no wait for a stream that records a graph: the call makes its own table
+    assert c.get(_key(w, b), 8) is None
+    state["capturing"] = set()
+    assert c.get(_key(w, b), 8) is not None
 
 
 def test_tables_and_recorded_graphs(monkeypatch):
